@@ -157,3 +157,41 @@ def test_segment_sum_table(W):
     torch.cuda.synchronize()
     assert ((out.cpu().double() - ref).abs() / (mag + 1e-12)).max() < 2e-6
     assert (out[N - 10:] == 0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,W,n_in,n_out", [(1, 4, 1, 1), (65, 4, 9, 9), (129, 12, 9, 5),
+                                            (9, 128, 9, 9), (10, 100, 3, 7), (3, 512, 31, 9),
+                                            (2, 512, 40, 4)])
+def test_rotation_tiles_match_general(E, W, n_in, n_out):
+    """The LDS-tiled forms (16-byte aligned rows of float4s) against the general ones, which
+    take the same call on a view off 16-byte alignment: one edge, a partial last workgroup, more
+    edges than a workgroup holds, rows too long for the tile (general form on both sides), an
+    empty output row and a repeated term.  The rotation and the segment sum add in one order, so
+    they are bit-equal; the coefficient adjoint adds W products in another, so each side is within
+    (W + 1) 2^-24 of the sum of the magnitudes."""
+    from tt_atom import rotation, scatter
+    g = torch.Generator().manual_seed(E * 1000 + W)
+    ij = [(i, j) for i in range(n_out) for j in range(n_in) if (i * 5 + j) % 3 != 1 and i != 2]
+    ij.append(ij[0])
+
+    def pair(*shape):
+        """The same values at a 16-byte aligned address and 4 bytes past one."""
+        a = torch.randn(*shape, generator=g).to(DEV)
+        b = torch.empty(a.numel() + 4, device=DEV)[1:1 + a.numel()].view(*shape)
+        b.copy_(a)
+        return a, b
+
+    x, go = pair(E, n_in * W), pair(E, n_out * W)
+    coef = torch.randn(E, len(ij), generator=g).to(DEV)
+    out = [rotation.rotate(None, v, ij, coef, n_in, W, None, n_out=n_out) for v in x]
+    vjp = [rotation.rotate_bw(None, a, b, ij, coef, n_in, W, None, n_out=n_out)
+           for a, b in zip(x, go)]
+    table, D = scatter.build_gather(torch.randint(3, (E,), generator=g), 4, E, min_width=9)
+    seg = [scatter.segment_sum(None, v, torch.from_numpy(table), D, 4, n_in * W) for v in x]
+    torch.cuda.synchronize()
+    assert torch.equal(*out) and torch.equal(vjp[0][0], vjp[1][0]) and torch.equal(*seg)
+    ii, jj = [i for i, _ in ij], [j for _, j in ij]
+    prod = go[0].double().view(E, n_out, W)[:, ii] * x[0].double().view(E, n_in, W)[:, jj]
+    for _, gc in vjp:
+        assert ((gc.double() - prod.sum(2)).abs() <= (W + 1) * 2.0 ** -24 * prod.abs().sum(2)).all()
