@@ -216,6 +216,46 @@ def test_split_gemm_small_splitk_group(nat):
         assert ((o.cpu().double() - ref).abs() / mag).max().item() < 2e-6
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 36, 128), (31, 130, 132), (33, 64, 1024), (256, 1000, 160),
+                                   (257, 640, 768), (65, 2052, 256), (700, 1021, 260),
+                                   (2000, 1024, 128), (4095, 260, 388)])
+@pytest.mark.parametrize("mode", [1, 3, 6, 16])
+def test_small_launch_gemm(nat, mode, M, N, K):
+    """The small-launch kernel over its tiles (32 x 32, 32 x 64, 64 x 64; eight wavefronts up to 256
+    rows, four above) and the first shapes past them: ragged rows, columns and k slabs, fewer slabs
+    than wavefronts, an unaligned output (N = 1021), the row-gather term, and in mode 16 rows that
+    are scaled and rows that start late or grow along K.  An operand plane pair keeps 22 bits, a
+    bf16 pair 16, one bf16 8, and the fp32 sums add (K + 16) roundings at random: the bounds, of
+    |A| |B| + |bias| + |gathered rows|, are 4 x 2^-22 (modes 6, 16), 4 x 2^-16 and 4 x 2^-8."""
+    g = torch.Generator().manual_seed(M * 31 + K + mode)
+    A = torch.randn(M, K, generator=g)
+    if mode == 16 and M > 4:
+        A[1] *= 2.0 ** 20
+        A[2] *= 2.0 ** -30
+        A[3, :K // 2] = 0.0
+        A[4, K // 2:] *= 2.0 ** 17
+    B = torch.randn(K, N, generator=g) / math.sqrt(K)
+    bias, P = torch.randn(N, generator=g), torch.randn(7, 2 * N, generator=g)
+    i0, i1 = (torch.randint(7, (M,), generator=g) for _ in range(2))
+    packed = nat.PackedWeight(B.to(DEV), mode).packed
+    Ad, bd, Pd = A.to(DEV), bias.to(DEV), P.to(DEV)
+    j0, j1 = i0.to(DEV, torch.int32), i1.to(DEV, torch.int32)
+    out = torch.full((M + 1, N), 7.5, device=DEV)
+    outs = []
+    for _ in range(2):
+        nat._call("tta_gemm_bf16x", Ad.data_ptr(), packed.data_ptr(), out.data_ptr(),
+                  bd.data_ptr(), None, None, M, N, K, K, N, mode, Pd.data_ptr(), 2 * N,
+                  j0.data_ptr(), j1.data_ptr(), N, 7, nat.EPI_STORE, nat._stream())
+        torch.cuda.synchronize()
+        outs.append(out[:M].cpu())
+    assert torch.equal(*outs) and (out[M] == 7.5).all()
+    extra = P.double()[i0, :N] + P.double()[i1, N:]
+    ref = A.double() @ B.double() + bias.double() + extra
+    mag = A.double().abs() @ B.double().abs() + bias.double().abs() + extra.abs()
+    bits = {1: 8, 3: 16, 6: 22, 16: 22}[mode]
+    assert ((outs[0].double() - ref).abs() / mag).max().item() < 4 * 2.0 ** -bits
+
+
 def test_gemm_batched_strided(nat):
     g = torch.Generator().manual_seed(5)
     N_, C, H = 50, 32, 24

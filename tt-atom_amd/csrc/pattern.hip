@@ -50,8 +50,8 @@ __global__ __launch_bounds__(256) void k_rotate_pattern(const float* __restrict_
 // coefficients of EB consecutive edges to LDS, each once and coalesced, and a thread forms all
 // output blocks of one float4 column of one edge.  Bound by HBM (each input and output byte
 // crosses it once); the element-per-thread form read every input block once per term through the
-// cache (about four times over for an lmax = 2 rotation) with a 64-bit division per element.  E = 20,011, nine blocks of 128 channels, 35
-// terms (187 MB): 153-168 -> 37 us (5.0 TB/s).
+// cache (about four times over for an lmax = 2 rotation) with a 64-bit division per element.
+// E = 20,011, nine blocks of 128 channels, 35 terms (187 MB): 153-168 -> 37 us (5.0 TB/s).
 __global__ __launch_bounds__(256) void k_rotate_pattern_tiled(const float* __restrict__ x,
                                                               const float* __restrict__ coef,
                                                               float* __restrict__ out, int64_t E,

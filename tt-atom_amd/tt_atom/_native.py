@@ -288,33 +288,47 @@ SPLIT_F32, SPLIT_F16X3, SPLIT_3, SPLIT_BF16 = 6, 16, 3, 1
 MODE_KIND = {6: "bf16x6", 16: "f16x3", 3: "bf16x3", 1: "bf16x1"}
 # mode-16 products that tta_gemm_bf16x(_group) runs on its short-K panel kernel (K <= 128, one
 # 32-wide k-slab count for the whole group, plain or SiLU epilogue, no row gathers, at least 128
-# columns, 16-byte aligned rows and operands, ldc < 2^22) are reported as their own family
+# columns, 16-byte aligned rows and operands, ldc < 2^22; launches of fewer than 4096 rows are
+# filed with the rest) are reported as their own family
 PANEL_KIND = "f16x3-panel"
 
 
 def _panel_item(M, N, K, ldc, epilogue, ptrs, gather=False):
     al = all(q is None or q % 16 == 0 for q in ptrs)
-    return (K <= 128 and epilogue in (EPI_STORE, EPI_SILU) and not gather and N >= 128
+    return (M >= 4096 and K <= 128 and epilogue in (EPI_STORE, EPI_SILU) and not gather and N >= 128
             and N % 4 == 0 and ldc % 4 == 0 and ldc < (1 << 22) and al)
 
 
 class PackedWeight:
     """A constant GEMM operand w_t [K, N] (fp32, row-major) plus its bf16-plane packing for the
     split kernel (``mode`` 6, 16, 3 or 1; None keeps only the fp32 matrix for the fp32-MFMA
-    kernel).  ``shape`` / ``T``-free: it stands wherever a [K, N] weight is passed to linear()."""
+    kernel).  ``shape`` / ``T``-free: it stands wherever a [K, N] weight is passed to linear().
+    The reduced modes (1, 3) apply to products of at least 4096 rows; below that a product is
+    fp32-accurate, so those weights are packed for mode 16 as well."""
 
     def __init__(self, w_t, mode=SPLIT_F32):
         if w_t.dim() != 2 or w_t.dtype != torch.float32 or not w_t.is_cuda:
             raise RuntimeError("PackedWeight: w_t must be a 2-D fp32 device tensor")
         self.w_t = w_t
         self.mode = mode
-        self.packed = None
-        K, N = w_t.shape
-        if mode is not None and K % 4 == 0:
-            n = load().tta_pack_b_elems(K, N, mode)
-            self.packed = torch.empty(n, dtype=torch.int16, device=w_t.device)
-            _call("tta_pack_b", _ptr(w_t, name="w_t", contiguous=False), K, N, _ld(w_t, "w_t"),
-                  mode, self.packed.data_ptr(), n, _stream())
+        self.packed = self._pack(mode)
+        self._packed_few = self._pack(SPLIT_F16X3) if mode in (SPLIT_3, SPLIT_BF16) else None
+
+    def _pack(self, mode):
+        K, N = self.w_t.shape
+        if mode is None or K % 4:
+            return None
+        n = load().tta_pack_b_elems(K, N, mode)
+        packed = torch.empty(n, dtype=torch.int16, device=self.w_t.device)
+        _call("tta_pack_b", _ptr(self.w_t, name="w_t", contiguous=False), K, N,
+              _ld(self.w_t, "w_t"), mode, packed.data_ptr(), n, _stream())
+        return packed
+
+    def planes(self, M):
+        """(packed planes, mode) of a product of M rows."""
+        if self._packed_few is not None and M < 4096:
+            return self._packed_few, SPLIT_F16X3
+        return self.packed, self.mode
 
     @property
     def shape(self):
@@ -332,6 +346,7 @@ def _same_rows(out, out2, aux, where):
 def _gemm_bf16x(x, pw, out, bias, epilogue, out2, aux, P=None, idx0=None, idx1=None, off1=0):
     M, K = x.shape
     N = pw.w_t.shape[1]
+    packed, mode = pw.planes(M)
     _same_rows(out, out2, aux, "linear")
     _span(x, "x", M, _ld(x, "x"), K)
     for t, nm in ((out, "out"), (out2, "out2"), (aux, "aux")):
@@ -339,15 +354,15 @@ def _gemm_bf16x(x, pw, out, bias, epilogue, out2, aux, P=None, idx0=None, idx1=N
     probe = _gemm_probe
     if probe is not None:
         c_passes = 1 + (epilogue in (EPI_ACCUM, EPI_PRE_SILU, EPI_SILU_GRAD)) + (2 if P is not None else 0)
-        panel = pw.mode == 16 and _panel_item(
+        panel = mode == 16 and _panel_item(
             M, N, K, _ld(out, "out"), epilogue,
             [out.data_ptr(), None if bias is None else bias.data_ptr()], gather=P is not None)
         probe.before(2.0 * M * N * K, 4.0 * (M * K + K * N + c_passes * M * N),
-                     PANEL_KIND if panel else MODE_KIND[pw.mode])
-    _call("tta_gemm_bf16x", x.data_ptr(), pw.packed.data_ptr(), out.data_ptr(),
+                     PANEL_KIND if panel else MODE_KIND[mode])
+    _call("tta_gemm_bf16x", x.data_ptr(), packed.data_ptr(), out.data_ptr(),
           None if bias is None else _ptr(bias, numel=N, name="bias"),
           None if out2 is None else out2.data_ptr(), None if aux is None else aux.data_ptr(),
-          M, N, K, _ld(x, "x"), _ld(out, "out"), pw.mode,
+          M, N, K, _ld(x, "x"), _ld(out, "out"), mode,
           None if P is None else _ptr(P, name="P"), 0 if P is None else _ld(P, "P"),
           None if idx0 is None else _i32(idx0, M), None if idx1 is None else _i32(idx1, M),
           off1, 0 if P is None else P.shape[0], epilogue, _stream())
@@ -355,62 +370,14 @@ def _gemm_bf16x(x, pw, out, bias, epilogue, out2, aux, P=None, idx0=None, idx1=N
         probe.after()
 
 
-def _split_ok(x, pw, min_rows=4096):
-    """The split kernel (128 x 128 x 32 tiles) runs edge-level GEMMs; short-K or small-M
-    products stay on the fp32 MFMA kernel, whose smaller tiles fill the chip better there
-    (small-M products of packed weights may take the split kernel's split-K form instead:
-    ``_small_split``)."""
+def _split_ok(x, pw):
+    """Whether a product runs on the split kernels (packed weight, 16-byte aligned rows); short-K
+    products and the unpacked weights of the heads stay on the fp32 MFMA kernel.  The library
+    chooses the tile by the launch's size (128 x 128, or the small-launch kernel's)."""
     M, K = x.shape
-    return (isinstance(pw, PackedWeight) and pw.packed is not None and M >= min_rows
+    return (isinstance(pw, PackedWeight) and pw.packed is not None and M > 0
             and K >= 128 and K % 4 == 0 and x.data_ptr() % 16 == 0 and _ld(x, "x") % 4 == 0
             and _ld(x, "x") < (1 << 21))
-
-
-def _fp32_tiles(shapes):
-    return sum(-(-M // 32) * -(-N // 64) for M, N in shapes)
-
-
-def _small_split(items):
-    """items = [(x, PackedWeight, bias, out, epilogue, out2, aux)] of products with M < 4096:
-    the split kernel's split-K launch (tta_gemm_bf16x_group_splitk) when the fp32 kernel would run
-    them unsplit at its matrix rate (160 or more of its 32 x 64 tiles in all: its split-K form
-    takes smaller launches) and the split kernel's rule splits them.  Returns False, having
-    launched nothing, otherwise."""
-    if not all(isinstance(w, PackedWeight) and w.packed is not None and w.mode == items[0][1].mode
-               and x.shape[0] < 4096 and x.shape[1] >= 256 and _split_ok(x, w, min_rows=1)
-               for x, w, *_ in items):
-        return False
-    if _fp32_tiles([(x.shape[0], w.shape[1]) for x, w, *_ in items]) < 160:
-        return False
-    probs = (GemmProblem * len(items))()
-    flops = nbytes = 0.0
-    for i, (x, w, bias, out, epi, out2, aux) in enumerate(items):
-        M, K = x.shape
-        N = w.shape[1]
-        ldc = _ld(out, "out")
-        probs[i] = GemmProblem(
-            _rows(x, M, _ld(x, "x"), K, "x"), w.packed.data_ptr(), _rows(out, M, ldc, N, "out"),
-            None if bias is None else _ptr(bias, numel=N, name="bias"),
-            None if out2 is None else _rows(out2, M, _ld(out2, "out2"), N, "out2"),
-            None if aux is None else _rows(aux, M, _ld(aux, "aux"), N, "aux"),
-            M, N, K, _ld(x, "x"), 0, ldc, epi)
-        flops += 2.0 * M * N * K
-        nbytes += 4.0 * (M * K + K * N + (1 + (epi in (EPI_ACCUM, EPI_PRE_SILU, EPI_SILU_GRAD)))
-                         * M * N)
-    need = load().tta_gemm_bf16x_splitk_work(probs, len(items))
-    if need < 0:
-        raise RuntimeError("tta_gemm_bf16x_splitk_work: bad product list")
-    if need == 0:
-        return False
-    work = torch.empty(need, device=items[0][0].device, dtype=torch.float32)
-    probe = _gemm_probe
-    if probe is not None:
-        probe.before(flops, nbytes, MODE_KIND[items[0][1].mode])
-    _call("tta_gemm_bf16x_group_splitk", probs, len(items), items[0][1].mode, work.data_ptr(),
-          work.numel(), _stream())
-    if probe is not None:
-        probe.after()
-    return True
 
 
 def linear_group_gate(items, c0, sig, x0, idx8, H, backward=False):
@@ -420,17 +387,18 @@ def linear_group_gate(items, c0, sig, x0, idx8, H, backward=False):
     the sigmoid of the convolution's gating columns (any row stride; linear() with
     EPI_SIGMOID), ``x0`` [M, H] receives coefficient 0's pre-activation.  ``backward``: the
     adjoint products with the gate's input adjoint applied instead
-    (tta_gemm_bf16x_group_gate_bwd; x0 is read).  Launches with fewer than 4096 rows take the
-    split-K form when the library's rule splits them."""
+    (tta_gemm_bf16x_group_gate_bwd; x0 is read)."""
     if not items or len(items) > MAX_GROUP or len(c0) != len(items):
         raise RuntimeError("linear_group_gate: 1..8 products, one first coefficient each")
-    mode = items[0][1].mode
+    M = items[0][0].shape[0]
+    if not isinstance(items[0][1], PackedWeight):
+        raise RuntimeError("linear_group_gate: every product needs a packed weight")
+    mode = items[0][1].planes(M)[1]
     probs = (GemmProblem * len(items))()
     flops = nbytes = 0.0
     L = max(_host_idx8(idx8)) + 1
-    M = items[0][0].shape[0]
     for i, (x, w, bias, out) in enumerate(items):
-        if not (isinstance(w, PackedWeight) and w.packed is not None and w.mode == mode
+        if not (isinstance(w, PackedWeight) and w.packed is not None and w.planes(M)[1] == mode
                 and x.shape[1] % 4 == 0 and x.data_ptr() % 16 == 0 and _ld(x, "x") % 4 == 0
                 and _ld(x, "x") < (1 << 21)):
             raise RuntimeError("linear_group_gate: every product needs a packed weight of one "
@@ -440,7 +408,7 @@ def linear_group_gate(items, c0, sig, x0, idx8, H, backward=False):
         if Mi != M or K != w.shape[0] or out.shape != (M, N) or N % H:
             raise RuntimeError("linear_group_gate: shape mismatch")
         ldc = _ld(out, "out")
-        probs[i] = GemmProblem(_rows(x, M, _ld(x, "x"), K, "x"), w.packed.data_ptr(),
+        probs[i] = GemmProblem(_rows(x, M, _ld(x, "x"), K, "x"), w.planes(M)[0].data_ptr(),
                                _rows(out, M, ldc, N, "out"),
                                None if bias is None else _ptr(bias, numel=N, name="bias"),
                                None, None, M, N, K, _ld(x, "x"), 0, ldc,
@@ -450,21 +418,13 @@ def linear_group_gate(items, c0, sig, x0, idx8, H, backward=False):
         nbytes += 4.0 * (M * K + K * N + 2 * M * N)
     gp = _rows(sig, M, _ld(sig, "sig"), L * H, "sig")
     xp = _rows(x0, M, _ld(x0, "x0"), H, "x0")
-    work = None
-    if M < 4096:
-        need = load().tta_gemm_bf16x_splitk_work(probs, len(items))
-        if need < 0:
-            raise RuntimeError("tta_gemm_bf16x_splitk_work: bad product list")
-        if need > 0:
-            work = torch.empty(need, device=items[0][0].device, dtype=torch.float32)
     probe = _gemm_probe
     if probe is not None:
         probe.before(flops, nbytes, MODE_KIND[mode], part="gate")
     _call("tta_gemm_bf16x_group_gate_bwd" if backward else "tta_gemm_bf16x_group_gate", probs,
           len(items), mode,
           (ctypes.c_int64 * len(items))(*c0), gp, _ld(sig, "sig"), xp, _ld(x0, "x0"), H,
-          _host_idx8(idx8), None if work is None else work.data_ptr(),
-          0 if work is None else work.numel(), _stream())
+          _host_idx8(idx8), None, 0, _stream())
     if probe is not None:
         probe.after()
 
@@ -520,8 +480,6 @@ def linear(x, w_t, bias=None, out=None, epilogue=EPI_STORE, out2=None, aux=None)
         if _split_ok(x, w_t):
             _gemm_bf16x(x, w_t, out, bias, epilogue, out2, aux)
             return out
-        if _small_split([(x, w_t, bias, out, epilogue, out2, aux)]):
-            return out
         w_t = w_t.w_t
     if M < 4096 and K >= 256 and _gemm_f32_splitk([(x, w_t, bias, out, epilogue, out2, aux)]):
         return out
@@ -544,19 +502,18 @@ def linear_group(items):
             raise RuntimeError("linear_group: shape mismatch")
         _same_rows(out, out2, aux, "linear_group")
     split = [isinstance(w, PackedWeight) and _split_ok(x, w) for x, w, *_ in items]
-    modes = {w.mode for (x, w, *_), sp in zip(items, split) if sp}
+    modes = {w.planes(x.shape[0])[1] for (x, w, *_), sp in zip(items, split) if sp}
     if len(items) > MAX_GROUP or (any(split) and not all(split)) or len(modes) > 1:
         for x, w, bias, out, epi, out2, aux in items:
             linear(x, w, bias, out, epi, out2, aux)
-        return
-    if not any(split) and _small_split(items):
         return
     if not split[0] and any(x.shape[1] >= 256 for x, *_ in items) and _gemm_f32_splitk(
             [(x, w.w_t if isinstance(w, PackedWeight) else w, *rest) for x, w, *rest in items]):
         return
     probs = (GemmProblem * len(items))()
     flops = nbytes = 0.0
-    panel = split[0] and items[0][1].mode == 16 and len({(x.shape[1] + 31) // 32 for x, *_ in items}) == 1
+    mode = modes.pop() if split[0] else None
+    panel = mode == 16 and len({(x.shape[1] + 31) // 32 for x, *_ in items}) == 1
     for x, w, bias, out, epi, out2, aux in items:
         panel = panel and _panel_item(x.shape[0], w.shape[1], x.shape[1], _ld(out, "out"), epi,
                                       [out.data_ptr(), None if bias is None else bias.data_ptr()])
@@ -567,7 +524,7 @@ def linear_group(items):
         ldc = _ld(out, "out")
         probs[i] = GemmProblem(
             _rows(x, M, _ld(x, "x"), K, "x"),
-            wt.packed.data_ptr() if split[0] else _rows(wt, K, _ld(wt, "w_t"), N, "w_t"),
+            w.planes(M)[0].data_ptr() if split[0] else _rows(wt, K, _ld(wt, "w_t"), N, "w_t"),
             _rows(out, M, ldc, N, "out"),
             None if bias is None else _ptr(bias, numel=N, name="bias"),
             None if out2 is None else _rows(out2, M, _ld(out2, "out2"), N, "out2"),
@@ -579,10 +536,10 @@ def linear_group(items):
         nbytes += 4.0 * (M * K + K * N + c_passes * M * N)
     probe = _gemm_probe
     if probe is not None:
-        probe.before(flops, nbytes, (PANEL_KIND if panel else MODE_KIND[items[0][1].mode])
+        probe.before(flops, nbytes, (PANEL_KIND if panel else MODE_KIND[mode])
                      if split[0] else "f32")
     if split[0]:
-        _call("tta_gemm_bf16x_group", probs, len(items), items[0][1].mode, _stream())
+        _call("tta_gemm_bf16x_group", probs, len(items), mode, _stream())
     else:
         _call("tta_gemm_f32_group", probs, len(items), _stream())
     if probe is not None:
