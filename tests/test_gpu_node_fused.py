@@ -90,6 +90,15 @@ def test_spectral_block_fwd_bwd(nat, N, C, H, with_add0, with_res):
     assert torch.equal(x2b, x2o)
 
 
+@pytest.mark.parametrize("N,C,H", [(1, 128, 128), (511, 48, 16), (515, 32, 96), (1021, 16, 48),
+                                   (1025, 64, 128), (2045, 48, 16), (2051, 128, 128)])
+def test_spectral_block_nodes_per_workgroup(nat, N, C, H):
+    """Each number of nodes per workgroup (2, 4, 8, 16: up to 512, 1024, 2048 and more nodes on 256
+    compute units) with a partly filled last workgroup, at widths with one and two weight chunks
+    in a group, held to the same bounds."""
+    test_spectral_block_fwd_bwd(nat, N, C, H, True, True)
+
+
 @pytest.mark.parametrize("N,C,H", [(41, 128, 128), (9, 16, 32)])
 def test_energy_head_fwd_bwd(nat, N, C, H):
     g = torch.Generator().manual_seed(7 * N + C)

@@ -11,15 +11,25 @@
 //   k_energy_head_fwd      per-node energy MLP on coefficient 0 (model.py:223-235)
 //   k_energy_head_bwd      its adjoint seeded with dE/dnode_e = 1 (forces.py:438-461)
 //
-// A workgroup owns NT = 16 nodes.  Their rows live in LDS as [coefficient][node][channel] (row
-// stride C + 4 floats: the 16 rows of an MFMA A fragment then fall in distinct banks), and every
-// product is a per-coefficient matrix product on the fp32 matrix cores
-// (v_mfma_f32_16x16x4_f32): rows = the 16 nodes of one coefficient, the weight of the
-// coefficient's degree l as the B operand, read from global memory (the weights are shared by
-// every workgroup and stay in L2).  Lane l supplies A[l%16][l/16] and B[l/16][l%16]; the result
-// D[4*(l/16)+r][l%16] lands in accumulator element r.  Each wave owns whole 16-column output
-// tiles for all nine coefficients, so the gate's per-degree sums over coefficients are
-// register-local.  Per-node norms run one wavefront per node (64 lanes x 2 channels).
+// A spectral workgroup owns T = 2, 4, 8 or 16 nodes.  Their rows live in LDS grouped by degree
+// (Pack<T>: the (2 l + 1) T rows of degree l, padded to whole 16-row tiles; row stride C + 4 floats:
+// the 16 rows of an MFMA A fragment then fall in distinct banks), and every product is a matrix
+// product of one degree's rows with that degree's weight on the fp32 matrix cores
+// (v_mfma_f32_16x16x4_f32), the weight read from global memory (shared by every workgroup, it
+// stays in L2).  Lane l supplies A[l%16][l/16] and B[l/16][l%16]; the result D[4*(l/16)+r][l%16]
+// lands in accumulator element r.  Each wave owns whole 16-column output tiles for every row, so
+// the gate's per-degree sums over coefficients stay inside a wavefront.  Per-node norms run one
+// wavefront per node (64 lanes x 2 channels).  The energy head's workgroups own NT = 16 nodes (one
+// row each).
+//
+// What bounds a spectral block: up to a few thousand nodes the chain inside one workgroup (load,
+// norm, three products that each stream a weight, norm), not a rate of the chip.  Nine 16-node
+// tiles cost 9 x 128 MFMAs per product and wavefront however few nodes they hold; packed by degree,
+// two nodes take 3 tiles, four 4, eight 6.  T is the smallest with one workgroup per compute unit
+// (pick_nodes), and each product's first weights are loaded a phase ahead.  Per launch, forward /
+// backward, one coefficient per 16-row tile -> packed: 24 nodes 42.4 / 43.3 -> 22.8 / 26.3 us; 256
+// nodes 44.8 / 44.4 -> 24.0 / 27.1; 1000 nodes 45.4 / 49.1 -> 29.9 / 35.4; 2048 nodes 49.7 / 52.6 ->
+// 40.4 / 44.2.
 //
 // Requirements (checked on the host): C and H multiples of 16, at most 128; lmax = 2.
 #include "common.h"
@@ -30,13 +40,12 @@ namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-constexpr int NT = 16;        // nodes per workgroup
+constexpr int NT = 16;        // nodes per energy-head workgroup, rows of an MFMA tile
 constexpr int NW = 8;         // waves per workgroup
 constexpr int NTH = 64 * NW;
-constexpr int NS = NT / NW;   // nodes per wave in the per-node phases
 constexpr int CMAX = 128;     // largest C / H
 constexpr int LDP = CMAX + 4; // LDS row stride (floats) of the [coef][node][channel] buffer
-constexpr int MAXJ = (CMAX / 16 + NW - 1) / NW;  // output column tiles per wave
+static_assert(CMAX / 16 <= NW, "one output column tile per wave");
 
 __device__ __forceinline__ int ndeg(int j) { return j == 0 ? 0 : (j < 4 ? 1 : 2); }
 __device__ __forceinline__ float nbdw(int j) {
@@ -47,34 +56,59 @@ __device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// LDS row of (coefficient c, local node r)
-__device__ __forceinline__ float* lrow(float* buf, int c, int r) { return buf + (c * NT + r) * LDP; }
+// Rows of T nodes grouped by degree: tiles [first(l), first(l + 1)) of 16 rows hold degree l, its
+// coefficient m (c = l^2 + m) of node n in row m T + n.  T divides 16, so row 4 q + e of any tile is
+// a row of node (4 q + e) % T.
+template <int T>
+struct Pack {
+  static_assert(16 % T == 0, "");
+  static constexpr int T1 = (3 * T + 15) / 16, T2 = (5 * T + 15) / 16, TILES = 1 + T1 + T2;
+  static __device__ constexpr int first(int l) { return l == 0 ? 0 : l == 1 ? 1 : 1 + T1; }
+  static __device__ constexpr int deg(int tile) { return tile < 1 ? 0 : tile < 1 + T1 ? 1 : 2; }
+  static __device__ __forceinline__ int row(int c, int n) {
+    const int l = ndeg(c);
+    return 16 * first(l) + (c - l * l) * T + n;
+  }
+  // coefficient of row 4 q + e of a tile, and whether the row is one (not padding)
+  static __device__ __forceinline__ int coef(int tile, int qe) {
+    const int l = deg(tile);
+    return l * l + ((tile - first(l)) * 16 + qe) / T;
+  }
+  static __device__ __forceinline__ bool used(int tile, int qe) {
+    const int l = deg(tile);
+    return ((tile - first(l)) * 16 + qe) / T < 2 * l + 1;
+  }
+};
+// one row tile with the degree 0 weight (the scalar products)
+struct Scalar {
+  static constexpr int TILES = 1;
+  static __device__ constexpr int deg(int) { return 0; }
+};
 
-// acc[c][jj] (+)= X[c] (16 x K, LDS rows at stride ldx) @ W[deg(c)] (K x Nout, row-major at
-// ldw, per-degree stride dstride) for the column tiles j = wave + NW jj of the Nout / 16 tiles;
-// NC = 9 (all coefficients) or 1 (coefficient 0 only, degree 0 weight).  A wave whose j is past
-// the last tile (narrow layers only) recomputes a valid tile and its caller discards the result,
-// so the inner loop has no branches.  K runs in chunks of 16: in MFMA step s of a chunk, slot q
-// (= lane / 16) of both operands is k = k0 + 4 q + s, so a lane reads its A values of a chunk as
-// one float4 from LDS.  The B values arrive D chunks at a time, the next D chunks' loads in
-// flight while the current ones are multiplied: D = 1 suffices when nine coefficients' MFMAs
-// cover a load (NC = 9); the single-coefficient products take D = 4 (K a multiple of 64) so
-// that their short chunks do not each wait out a load.
-template <int NC, int D>
-__device__ __forceinline__ void coef_mm_d(const float* X, int ldx, int K,
-                                          const float* __restrict__ W, int64_t dstride, int ldw,
-                                          int Nout, int wave, int lane, floatx4 (&acc)[9][MAXJ]) {
-  constexpr int NL = NC == 9 ? 3 : 1;
-  const int ntile = Nout / 16;
-  const int r = lane & 15, q = lane >> 4;
-  // 32-bit element offsets from the (wave-uniform) weight base
-  unsigned off[NL][MAXJ];
-#pragma unroll
-  for (int l = 0; l < NL; ++l)
-#pragma unroll
-    for (int jj = 0; jj < MAXJ; ++jj)
-      off[l][jj] = (unsigned)(l * dstride + ((wave + NW * jj) % ntile) * 16 + r + 4 * q * ldw);
-  auto loadb = [&](float (&b)[D][4][NL][MAXJ], int k0) {
+// LDS row of (coefficient c, local node n)
+template <int T>
+__device__ __forceinline__ float* lrow(float* buf, int c, int n) {
+  return buf + Pack<T>::row(c, n) * LDP;
+}
+
+// One product acc[i][jj] += X tile i (16 x K, LDS rows at stride ldx) @ W[deg(i)] (K x ncol,
+// row-major at ldw, per-degree stride dstride) for JT 16-column tiles per wave: tile
+// (wave + NW jj) % (ncol / 16) at column offset jj cstep.  (A wave whose tile is past the last one,
+// narrow layers only, recomputes a valid tile and its caller discards the result, so the inner
+// loop has no branches.)  K runs in chunks of 16: in MFMA step s of a chunk, slot q (= lane / 16) of
+// both operands is k = k0 + 4 q + s, so a lane reads its A values of a chunk as one float4 from
+// LDS.  The B values arrive D chunks at a time (K a multiple of 16 D), two groups in flight; they do
+// not depend on the rows, so start() is called a phase ahead (before a norm, a gate or a barrier)
+// and the product finds its first groups landed.
+template <class P, int D, int JT>
+struct Product {
+  static constexpr int NC = P::TILES, NL = NC > 1 ? 3 : 1, G = 16 * D;
+  const float* W;
+  int ldw, K;
+  unsigned off[NL][JT];  // 32-bit element offsets from the (wave-uniform) weight base
+  float b0[D][4][NL][JT], b1[D][4][NL][JT];
+
+  __device__ __forceinline__ void load(float (&b)[D][4][NL][JT], int k0) const {
 #pragma unroll
     for (int d = 0; d < D; ++d)
 #pragma unroll
@@ -82,75 +116,79 @@ __device__ __forceinline__ void coef_mm_d(const float* X, int ldx, int K,
 #pragma unroll
         for (int l = 0; l < NL; ++l)
 #pragma unroll
-          for (int jj = 0; jj < MAXJ; ++jj)
+          for (int jj = 0; jj < JT; ++jj)
             b[d][s][l][jj] = W[off[l][jj] + (unsigned)((k0 + 16 * d + s) * ldw)];
-  };
-  const float* xr = X + r * ldx + 4 * q;
-  auto mul = [&](const float (&b)[D][4][NL][MAXJ], int g0) {
+  }
+  __device__ __forceinline__ void start(const float* __restrict__ W_, int64_t dstride, int ldw_,
+                                        int K_, int ncol, int cstep, int wave, int lane) {
+    W = W_;
+    ldw = ldw_;
+    K = K_;
+    const int ntile = ncol / 16;
+#pragma unroll
+    for (int l = 0; l < NL; ++l)
+#pragma unroll
+      for (int jj = 0; jj < JT; ++jj)
+        off[l][jj] = (unsigned)(l * dstride + jj * cstep + (wave % ntile) * 16 + (lane & 15) +
+                                4 * (lane >> 4) * ldw);
+    load(b0, 0);
+    if (G < K) load(b1, G);
+  }
+  __device__ __forceinline__ void mul(const float (&b)[D][4][NL][JT], const float* xr, int ldx,
+                                      int g0, floatx4 (&acc)[NC][JT]) const {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      const int k0 = g0 + 16 * d;
       floatx4 a[NC];
 #pragma unroll
       for (int c = 0; c < NC; ++c)
-        a[c] = *reinterpret_cast<const floatx4*>(xr + c * NT * ldx + k0);
+        a[c] = *reinterpret_cast<const floatx4*>(xr + c * 16 * ldx + g0 + 16 * d);
 #pragma unroll
       for (int s = 0; s < 4; ++s)
 #pragma unroll
         for (int c = 0; c < NC; ++c)
 #pragma unroll
-          for (int jj = 0; jj < MAXJ; ++jj)
-            acc[c][jj] = mfma4(a[c][s], b[d][s][NC == 9 ? ndeg(c) : 0][jj], acc[c][jj]);
+          for (int jj = 0; jj < JT; ++jj)
+            acc[c][jj] = mfma4(a[c][s], b[d][s][P::deg(c)][jj], acc[c][jj]);
     }
-  };
-  // two register buffers in turn: the next group's loads are in flight during this one's MFMAs
-  constexpr int G = 16 * D;
-  float b0[D][4][NL][MAXJ], b1[D][4][NL][MAXJ];
-  loadb(b0, 0);
-  for (int g0 = 0; g0 < K; g0 += 2 * G) {
-    if (g0 + G < K) loadb(b1, g0 + G);
-    mul(b0, g0);
-    if (g0 + G >= K) break;
-    if (g0 + 2 * G < K) loadb(b0, g0 + 2 * G);
-    mul(b1, g0 + G);
   }
-}
+  __device__ __forceinline__ void run(const float* X, int ldx, int lane, floatx4 (&acc)[NC][JT]) {
+    const float* xr = X + (lane & 15) * ldx + 4 * (lane >> 4);
+    for (int g0 = 0; g0 < K; g0 += 2 * G) {
+      mul(b0, xr, ldx, g0, acc);
+      if (g0 + 2 * G < K) load(b0, g0 + 2 * G);
+      if (g0 + G >= K) break;
+      mul(b1, xr, ldx, g0 + G, acc);
+      if (g0 + 3 * G < K) load(b1, g0 + 3 * G);
+    }
+  }
+};
 
-template <int NC>
-__device__ __forceinline__ void coef_mm(const float* X, int ldx, int K,
-                                        const float* __restrict__ W, int64_t dstride, int ldw,
-                                        int Nout, int wave, int lane, floatx4 (&acc)[9][MAXJ]) {
-  if (NC == 1 && K % 64 == 0)
-    coef_mm_d<NC, 4>(X, ldx, K, W, dstride, ldw, Nout, wave, lane, acc);
-  else
-    coef_mm_d<NC, 1>(X, ldx, K, W, dstride, ldw, Nout, wave, lane, acc);
-}
-
-__device__ __forceinline__ void zero_acc(floatx4 (&acc)[9][MAXJ]) {
+template <int NC, int JT>
+__device__ __forceinline__ void zero_acc(floatx4 (&acc)[NC][JT]) {
 #pragma unroll
-  for (int c = 0; c < 9; ++c)
+  for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int jj = 0; jj < MAXJ; ++jj) acc[c][jj] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int jj = 0; jj < JT; ++jj) acc[c][jj] = floatx4{0.f, 0.f, 0.f, 0.f};
 }
 
 // RMSNormSH forward of one node's 9 x C rows (norm.py:93-111): centre coefficient 0 over the
 // channels, ms = mean_c sum_j bdw_j xc_j^2, inv = rsqrt(ms + eps), y = xc * inv * aw[l(j)],
-// y[0] += ab (+ add0).  xs: the node's rows (stride xstride); writes y rows (stride ystride).
-// One wavefront; lane handles channels lane, lane + 64.
-__device__ __forceinline__ float rms_fwd_node(const float* xs, int64_t xstride, float* ys,
-                                              int64_t ystride, const float* __restrict__ aw,
+// y[0] += ab (+ add0).  xr(j) / yr(j): the node's input and output rows.  One wavefront; lane
+// handles channels lane, lane + 64.
+template <class XR, class YR>
+__device__ __forceinline__ float rms_fwd_node(XR xr, YR yr, const float* __restrict__ aw,
                                               const float* __restrict__ ab,
                                               const float* __restrict__ add0row, int C,
                                               int lane, float eps) {
   float s0 = 0.f;
-  for (int c = lane; c < C; c += 64) s0 += xs[c];
+  for (int c = lane; c < C; c += 64) s0 += xr(0)[c];
   const float mu = tta_group_sum(s0, 64) / C;
   float ms = 0.f;
   for (int c = lane; c < C; c += 64) {
     float sc = 0.f;
 #pragma unroll
     for (int j = 0; j < 9; ++j) {
-      const float v = j == 0 ? xs[c] - mu : xs[j * xstride + c];
+      const float v = j == 0 ? xr(0)[c] - mu : xr(j)[c];
       sc += v * v * nbdw(j);
     }
     ms += sc;
@@ -160,7 +198,7 @@ __device__ __forceinline__ float rms_fwd_node(const float* xs, int64_t xstride, 
   for (int c = lane; c < C; c += 64) {
     float v[9];
 #pragma unroll
-    for (int j = 0; j < 9; ++j) v[j] = j == 0 ? xs[c] - mu : xs[j * xstride + c];
+    for (int j = 0; j < 9; ++j) v[j] = j == 0 ? xr(0)[c] - mu : xr(j)[c];
 #pragma unroll
     for (int j = 0; j < 9; ++j) {
       float o = v[j] * (inv * aw[ndeg(j) * C + c]);
@@ -168,7 +206,7 @@ __device__ __forceinline__ float rms_fwd_node(const float* xs, int64_t xstride, 
         o = o + ab[c];
         if (add0row) o = o + add0row[c];
       }
-      ys[j * ystride + c] = o;
+      yr(j)[c] = o;
     }
   }
   return inv;
@@ -225,32 +263,38 @@ __device__ __forceinline__ void rms_bwd_vals(GV gv, XV xv, const float* __restri
   }
 }
 
-// The 16-node tile of a [N, 9, C] tensor into the [coefficient][node][channel] LDS layout, one
-// wavefront per (node, coefficient) row (wave-uniform indices, no per-element division); rows
-// of absent nodes are zero.
-__device__ __forceinline__ void load_tile(float* buf, const float* __restrict__ x, int64_t n0,
-                                          int nv, int C, int wave, int lane) {
-  constexpr int RPW = 9 * NT / NW;   // rows per wave
-  float v[RPW][2];                   // all of a wave's loads in flight before any store
+// T nodes of a [N, 9, C] tensor into the Pack<T> LDS rows, one wavefront per (node, coefficient)
+// row (wave-uniform indices, no per-element division); rows of absent nodes are zero.  (Padding
+// rows are left as they are: a row of an MFMA operand reaches only its own output row.)
+template <int T>
+struct NodeRows {
+  static constexpr int RPW = (9 * T + NW - 1) / NW;  // rows per wave
+  float v[RPW][2];
+  __device__ __forceinline__ void load(const float* __restrict__ x, int64_t n0, int nv, int C,
+                                       int wave, int lane) {
 #pragma unroll
-  for (int i = 0; i < RPW; ++i) {
-    const int rc = wave + NW * i, rr = rc / 9, c = rc - 9 * rr;
+    for (int i = 0; i < RPW; ++i) {
+      const int rc = wave + NW * i, rr = rc / 9, c = rc - 9 * rr;
 #pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const int ch = lane + 64 * hh;
-      v[i][hh] = (rr < nv && ch < C) ? x[((n0 + rr) * 9 + c) * C + ch] : 0.f;
+      for (int hh = 0; hh < 2; ++hh) {
+        const int ch = lane + 64 * hh;
+        v[i][hh] = (rr < nv && ch < C) ? x[((n0 + rr) * 9 + c) * C + ch] : 0.f;
+      }
     }
   }
+  __device__ __forceinline__ void store(float* buf, int C, int wave, int lane) const {
 #pragma unroll
-  for (int i = 0; i < RPW; ++i) {
-    const int rc = wave + NW * i, rr = rc / 9, c = rc - 9 * rr;
+    for (int i = 0; i < RPW; ++i) {
+      const int rc = wave + NW * i, rr = rc / 9, c = rc - 9 * rr;
+      if (rr >= T) continue;
 #pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const int ch = lane + 64 * hh;
-      if (ch < C) lrow(buf, c, rr)[ch] = v[i][hh];
+      for (int hh = 0; hh < 2; ++hh) {
+        const int ch = lane + 64 * hh;
+        if (ch < C) lrow<T>(buf, c, rr)[ch] = v[i][hh];
+      }
     }
   }
-}
+};
 
 struct SpecFwdArgs {
   const float* x1;                        // [N, 9, C] block state after the edgewise residual
@@ -265,111 +309,109 @@ struct SpecFwdArgs {
   int64_t N;
   int C, H;
   float eps;
-  int npb;                                // nodes per workgroup, NT or NT / 2 (rows past it zero)
 };
 
+template <int T, int D>
 __global__ __launch_bounds__(NTH, 1) void k_spectral_block_fwd(SpecFwdArgs p) {
-  __shared__ float buf[9 * NT * LDP];
-  __shared__ float gat[NT * (2 * CMAX + 4)];
+  typedef Pack<T> P;
+  __shared__ float buf[P::TILES * 16 * LDP];
+  __shared__ float gat[T * (2 * CMAX + 4)];
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int C = p.C, H = p.H, LH = 2 * H, ldg = 2 * CMAX + 4;
-  const int64_t n0 = (int64_t)blockIdx.x * p.npb;
-  const int nv = (int)min((int64_t)p.npb, p.N - n0);
+  const int64_t n0 = (int64_t)blockIdx.x * T;
+  const int nv = (int)min((int64_t)T, p.N - n0);
+  const int r = lane & 15, q = lane >> 4;
+  const bool hok = wave < H / 16, cok = wave < C / 16;  // this wave owns a column tile
+  const int col = wave * 16 + r;
   // 1. x1 rows -> LDS (rows of absent nodes zero)
-  load_tile(buf, p.x1, n0, nv, C, wave, lane);
+  NodeRows<T> rows;
+  rows.load(p.x1, n0, nv, C, wave, lane);
+  Product<Scalar, D, 2> scal;
+  scal.start(p.ws_t, 0, LH, C, H, H, wave, lane);
+  Product<P, D, 1> lin;
+  lin.start(p.w1t, (int64_t)C * H, H, C, H, 0, wave, lane);
+  rows.store(buf, C, wave, lane);
   __syncthreads();
   // 2. norm_2 in place, one wave per node
-  for (int r = wave; r < nv; r += NW) {
-    float* xs = lrow(buf, 0, r);
-    const float inv = rms_fwd_node(xs, (int64_t)NT * LDP, xs, (int64_t)NT * LDP, p.aw2, p.ab2,
-                                   nullptr, C, lane, p.eps);
-    if (lane == 0) p.inv2[n0 + r] = inv;
+  for (int rr = wave; rr < nv; rr += NW) {
+    auto row = [&](int j) { return lrow<T>(buf, j, rr); };
+    const float inv = rms_fwd_node(row, row, p.aw2, p.ab2, nullptr, C, lane, p.eps);
+    if (lane == 0) p.inv2[n0 + rr] = inv;
   }
   __syncthreads();
-  const int r = lane & 15, q = lane >> 4;
-  floatx4 acc[9][MAXJ];
-  // 3. scalar MLP on coefficient 0: a_s = n2_0 @ ws_t + bs (saved), gating = silu(a_s) -> LDS.
-  //    2H columns = 2 x (H / 16) tiles; this wave takes tiles wave + NW jj of each H half.
+  // 3. scalar MLP on coefficient 0: a_s = n2_0 @ ws_t + bs (saved), gating = silu(a_s) -> LDS; this
+  //    wave's column tile of both H halves
+  floatx4 as[1][2];
+  zero_acc(as);
+  scal.run(buf, LDP, lane, as);
+  // 4. h = n2 @ w1t[l] (+ b1 on coefficient 0)
+  floatx4 acc[P::TILES][1];
+  zero_acc(acc);
+  lin.run(buf, LDP, lane, acc);
+  lin.start(p.w2t, (int64_t)H * C, C, H, C, 0, wave, lane);
+  if (hok) {
 #pragma unroll
-  for (int half = 0; half < 2; ++half) {
-    zero_acc(acc);
-    coef_mm<1>(buf, LDP, C, p.ws_t + half * H, 0, LH, H, wave, lane, acc);
-#pragma unroll
-    for (int jj = 0; jj < MAXJ; ++jj) {
-      const int j = wave + NW * jj;
-      if (j >= H / 16) continue;
-      const int col = half * H + j * 16 + r;
-      const float bias = p.bs[col];
+    for (int half = 0; half < 2; ++half) {
+      const float bias = p.bs[half * H + col];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int row = 4 * q + e;
-        const float a = acc[0][jj][e] + bias;
-        if (row < nv) p.a_s[(n0 + row) * LH + col] = a;
-        gat[row * ldg + col] = tta_silu(a);
+        const float a = as[0][half][e] + bias;
+        if (row < nv) p.a_s[(n0 + row) * LH + half * H + col] = a;
+        if (row < T) gat[row * ldg + half * H + col] = tta_silu(a);
       }
     }
   }
-  // 4. h = n2 @ w1t[l] (+ b1 on coefficient 0)
-  zero_acc(acc);
-  coef_mm<9>(buf, LDP, C, p.w1t, (int64_t)C * H, H, H, wave, lane, acc);
   __syncthreads();  // every wave is done reading n2; gating is complete
   // 5. h saved; gout = gate(h) -> LDS (natural order: l = 1 rows gate block 0, l = 2 block 1);
   //    the gate values sigmoid(gating) once per (node, degree, channel)
-  float sig[MAXJ][2][4];
-#pragma unroll
-  for (int jj = 0; jj < MAXJ; ++jj) {
-    const int col = ((wave + NW * jj) % (H / 16)) * 16 + r;
+  if (hok) {
+    float sig[2][4];
 #pragma unroll
     for (int l = 0; l < 2; ++l)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        sig[jj][l][e] = tta_sigmoid_acc(gat[(4 * q + e) * ldg + l * H + col]);
-  }
+        sig[l][e] = tta_sigmoid_acc(gat[(4 * q + e) % T * ldg + l * H + col]);
+    const float b1 = p.b1[col];
 #pragma unroll
-  for (int c = 0; c < 9; ++c)
-#pragma unroll
-    for (int jj = 0; jj < MAXJ; ++jj) {
-      const int j = wave + NW * jj;
-      if (j >= H / 16) continue;
-      const int col = j * 16 + r;
-      const float bias = c == 0 ? p.b1[col] : 0.f;
+    for (int i = 0; i < P::TILES; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int row = 4 * q + e;
-        const float v = acc[c][jj][e] + bias;
-        if (row < nv) p.h[((n0 + row) * 9 + c) * H + col] = v;
-        const float g = c == 0 ? tta_silu(v) : v * sig[jj][ndeg(c) - 1][e];
-        lrow(buf, c, row)[col] = g;
+        const int n = (4 * q + e) % T;
+        const float v = acc[i][0][e] + (i == 0 ? b1 : 0.f);
+        if (n < nv && P::used(i, 4 * q + e))
+          p.h[((n0 + n) * 9 + P::coef(i, 4 * q + e)) * H + col] = v;
+        const float g = i == 0 ? tta_silu(v) : v * sig[P::deg(i) == 2][e];
+        buf[(16 * i + 4 * q + e) * LDP + col] = g;
       }
+  }
+  // the residual's x1 values, for step 6: they arrive during the product
+  float xr[P::TILES][4];
+#pragma unroll
+  for (int i = 0; i < P::TILES; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int n = (4 * q + e) % T;
+      xr[i][e] = cok && n < nv && P::used(i, 4 * q + e)
+                     ? p.x1[((n0 + n) * 9 + P::coef(i, 4 * q + e)) * C + col]
+                     : 0.f;
     }
   __syncthreads();
   // 6. out = x1 + gout @ w2t[l] (+ b2 on coefficient 0)
   zero_acc(acc);
-  coef_mm<9>(buf, LDP, H, p.w2t, (int64_t)H * C, C, C, wave, lane, acc);
+  lin.run(buf, LDP, lane, acc);
   if (p.awn) __syncthreads();  // the next norm reuses the buffer for x2
-  // residual: all of this lane's x1 values are loaded before any x2 store, so the loads overlap
-#pragma unroll
-  for (int jj = 0; jj < MAXJ; ++jj) {
-    const int j = wave + NW * jj;
-    if (j >= C / 16) continue;
-    const int col = j * 16 + r;
+  if (cok) {
     const float b2 = p.b2[col];
-    float xr[9][4];
 #pragma unroll
-    for (int c = 0; c < 9; ++c)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = 4 * q + e;
-        xr[c][e] = row < nv ? p.x1[((n0 + row) * 9 + c) * C + col] : 0.f;
-      }
-#pragma unroll
-    for (int c = 0; c < 9; ++c)
+    for (int i = 0; i < P::TILES; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int row = 4 * q + e;
-        const float v = acc[c][jj][e] + (c == 0 ? b2 : 0.f) + xr[c][e];
-        if (row < nv) p.x2[((n0 + row) * 9 + c) * C + col] = v;
-        if (p.awn) lrow(buf, c, row)[col] = v;
+        const int n = (4 * q + e) % T;
+        const float v = acc[i][0][e] + (i == 0 ? b2 : 0.f) + xr[i][e];
+        if (n < nv && P::used(i, 4 * q + e))
+          p.x2[((n0 + n) * 9 + P::coef(i, 4 * q + e)) * C + col] = v;
+        if (p.awn) buf[(16 * i + 4 * q + e) * LDP + col] = v;
       }
   }
   if (!p.awn) return;
@@ -377,8 +419,9 @@ __global__ __launch_bounds__(NTH, 1) void k_spectral_block_fwd(SpecFwdArgs p) {
   // 7. the next RMSNormSH on x2 (coefficient 0 + the system embedding when given)
   for (int rr = wave; rr < nv; rr += NW) {
     const int64_t n = n0 + rr;
-    const float inv = rms_fwd_node(lrow(buf, 0, rr), (int64_t)NT * LDP, p.yn + n * 9 * C, C, p.awn,
-                                   p.abn, p.add0 ? p.add0 + n * C : nullptr, C, lane, p.eps);
+    const float inv = rms_fwd_node([&](int j) { return lrow<T>(buf, j, rr); },
+                                   [&](int j) { return p.yn + (n * 9 + j) * C; }, p.awn, p.abn,
+                                   p.add0 ? p.add0 + n * C : nullptr, C, lane, p.eps);
     if (lane == 0) p.invn[n] = inv;
   }
 }
@@ -391,36 +434,46 @@ struct SpecBwdArgs {
   float* g_x1;                            // [N, 9, C]
   int64_t N;
   int C, H;
-  int npb;                                // nodes per workgroup, NT or NT / 2 (rows past it zero)
 };
 
+template <int T, int D>
 __global__ __launch_bounds__(NTH, 1) void k_spectral_block_bwd(SpecBwdArgs p) {
-  __shared__ float buf[9 * NT * LDP];
+  typedef Pack<T> P;
+  constexpr int NS = (T + NW - 1) / NW;   // nodes per wave in the per-node phases
+  __shared__ float buf[P::TILES * 16 * LDP];
   __shared__ float gas[NT * (2 * CMAX + 4)];
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int C = p.C, H = p.H, LH = 2 * H, ldg = 2 * CMAX + 4;
-  const int64_t n0 = (int64_t)blockIdx.x * p.npb;
-  const int nv = (int)min((int64_t)p.npb, p.N - n0);
+  const int64_t n0 = (int64_t)blockIdx.x * T;
+  const int nv = (int)min((int64_t)T, p.N - n0);
+  const int r = lane & 15, q = lane >> 4;
+  const bool hok = wave < H / 16, cok = wave < C / 16;  // this wave owns a column tile
+  const int col = wave * 16 + r;
   // 1. g_x2 = next-norm backward (+ res), one wave per node; kept in registers for step 5 and
   //    written to LDS as the FF's output adjoint (absent nodes: zero rows).  The x2 tile comes
   //    into LDS by coalesced rows; each wave's g_n values (its nodes wave + NW s, channels
   //    lane + 64 hh) go straight to registers, all loads in flight together.
   float gx2[NS][9][2];
-  load_tile(buf, p.x2, n0, nv, C, wave, lane);
+  // values of a [N, 9, C] tensor at this wave's nodes and channels (0 outside)
+  auto node_vals = [&](const float* __restrict__ x, float (&v)[NS][9][2]) {
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    const int rr = wave + NW * s;
-    const int64_t n = n0 + rr;
+    for (int s = 0; s < NS; ++s)
 #pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const int c = lane + 64 * hh;
-      const bool in = rr < nv && c < C;
+      for (int hh = 0; hh < 2; ++hh) {
+        const int rr = wave + NW * s, c = lane + 64 * hh;
+        const bool in = rr < nv && c < C;
 #pragma unroll
-      for (int j = 0; j < 9; ++j) {
-        gx2[s][j][hh] = in ? p.g_n[(n * 9 + j) * C + c] : 0.f;
+        for (int j = 0; j < 9; ++j) v[s][j][hh] = in ? x[((n0 + rr) * 9 + j) * C + c] : 0.f;
       }
-    }
+  };
+  {
+    NodeRows<T> rows;
+    rows.load(p.x2, n0, nv, C, wave, lane);
+    node_vals(p.g_n, gx2);
+    rows.store(buf, C, wave, lane);
   }
+  Product<P, D, 1> lin;
+  lin.start(p.w2, (int64_t)C * H, H, C, H, 0, wave, lane);
   __syncthreads();
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
@@ -429,10 +482,9 @@ __global__ __launch_bounds__(NTH, 1) void k_spectral_block_bwd(SpecBwdArgs p) {
       // an absent node's rows stay zero (its x2 rows were zero-filled above)
       continue;
     }
-    const float* xs = lrow(buf, 0, rr);
     float o[9][2];
     rms_bwd_vals([&](int j, int hh) { return gx2[s][j][hh]; },
-                 [&](int j, int hh) { return xs[j * NT * LDP + lane + 64 * hh]; }, p.awn,
+                 [&](int j, int hh) { return lrow<T>(buf, j, rr)[lane + 64 * hh]; }, p.awn,
                  p.invn[n0 + rr], C, lane, o);
     const int64_t n = n0 + rr;
 #pragma unroll
@@ -441,100 +493,102 @@ __global__ __launch_bounds__(NTH, 1) void k_spectral_block_bwd(SpecBwdArgs p) {
 #pragma unroll
       for (int j = 0; j < 9; ++j) {
         gx2[s][j][hh] = o[j][hh] + ((p.res && c < C) ? p.res[(n * 9 + j) * C + c] : 0.f);
-        if (c < C) lrow(buf, j, rr)[c] = gx2[s][j][hh];   // this wave's own node rows
+        if (c < C) lrow<T>(buf, j, rr)[c] = gx2[s][j][hh];   // this wave's own node rows
       }
     }
   }
-  __syncthreads();
-  const int r = lane & 15, q = lane >> 4;
-  floatx4 acc[9][MAXJ];
-  // 2. g_gout = g_x2 @ w2[l]  ([C, H] per degree)
-  zero_acc(acc);
-  coef_mm<9>(buf, LDP, C, p.w2, (int64_t)C * H, H, H, wave, lane, acc);
-  // 3. gate backward: g_h0 = g_gout0 silu'(h0); g_h_c = g_gout_c sig(gating); the degree sums
-  //    sum_{c in l} g_gout_c h_c (register-local: this wave holds all nine coefficients of its
-  //    columns) give g_a_s = sum * sig'(gating) * silu'(a_s)
-  __syncthreads();  // every wave is done reading g_x2
-#pragma unroll
-  for (int jj = 0; jj < MAXJ; ++jj) {
-    const int j = wave + NW * jj;
-    if (j >= H / 16) continue;
-    const int col = j * 16 + r;
-    // this lane's saved forward values first (all loads in flight together)
-    float hs[9][4], as[2][4];
+  // this lane's saved forward values for step 3; they arrive during the product where its registers
+  // leave room for them (T < 16)
+  float hs[P::TILES][4], as[2][4];
+  auto saved_vals = [&]() {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int row = 4 * q + e;
-      const int64_t n = n0 + row;
-      const bool in = row < nv;
+      const int nd = (4 * q + e) % T;
+      const int64_t n = n0 + nd;
+      const bool in = hok && nd < nv;
 #pragma unroll
-      for (int c = 0; c < 9; ++c) hs[c][e] = in ? p.h[(n * 9 + c) * H + col] : 0.f;
+      for (int i = 0; i < P::TILES; ++i)
+        hs[i][e] = in && P::used(i, 4 * q + e)
+                       ? p.h[(n * 9 + P::coef(i, 4 * q + e)) * H + col]
+                       : 0.f;
       as[0][e] = in ? p.a_s[n * LH + col] : 0.f;
       as[1][e] = in ? p.a_s[n * LH + H + col] : 0.f;
     }
+  };
+  if (T < 16) saved_vals();
+  __syncthreads();
+  // 2. g_gout = g_x2 @ w2[l]  ([C, H] per degree)
+  floatx4 acc[P::TILES][1];
+  zero_acc(acc);
+  lin.run(buf, LDP, lane, acc);
+  if (T == 16) saved_vals();
+  lin.start(p.w1, (int64_t)H * C, C, H, C, 0, wave, lane);
+  Product<Scalar, D, 1> scal;
+  if (T < 16) scal.start(p.ws, 0, C, LH, C, 0, wave, lane);
+  // 3. gate backward: g_h0 = g_gout0 silu'(h0); g_h_c = g_gout_c sig(gating); the degree sums
+  //    sum_{c in l} g_gout_c h_c (this wave holds every row of its columns: the lane's rows of a
+  //    node, then the lanes 16 and 32 apart that hold the others) give
+  //    g_a_s = sum * sig'(gating) * silu'(a_s)
+  __syncthreads();  // every wave is done reading g_x2
+  if (hok) {
+    float sum[2][4], sg[2][4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int row = 4 * q + e;
-      float s1 = 0.f, s2 = 0.f;
-      const float as1 = as[0][e], as2 = as[1][e];
-      const float g1 = tta_silu(as1), g2 = tta_silu(as2);
-      const float sg1 = tta_sigmoid_acc(g1), sg2 = tta_sigmoid_acc(g2);
+      sum[0][e] = sum[1][e] = 0.f;
+      sg[0][e] = tta_sigmoid_acc(tta_silu(as[0][e]));
+      sg[1][e] = tta_sigmoid_acc(tta_silu(as[1][e]));
 #pragma unroll
-      for (int c = 0; c < 9; ++c) {
-        const float hv = hs[c][e];
-        const float gg = acc[c][jj][e];
+      for (int i = 0; i < P::TILES; ++i) {
+        const float hv = hs[i][e], gg = acc[i][0][e];
         float gh;
-        if (c == 0) {
+        if (P::deg(i) == 0) {
           gh = gg * tta_silu_grad(hv);
-        } else if (c < 4) {
-          gh = gg * sg1;
-          s1 += gg * hv;
         } else {
-          gh = gg * sg2;
-          s2 += gg * hv;
+          const int l = P::deg(i) - 1;
+          gh = gg * sg[l][e];
+          sum[l][e] += P::used(i, 4 * q + e) ? gg * hv : 0.f;  // (padding rows may hold anything)
         }
-        lrow(buf, c, row)[col] = gh;
+        buf[(16 * i + 4 * q + e) * LDP + col] = gh;
       }
-      gas[row * ldg + col] = s1 * sg1 * (1.f - sg1) * tta_silu_grad(as1);
-      gas[row * ldg + H + col] = s2 * sg2 * (1.f - sg2) * tta_silu_grad(as2);
+    }
+#pragma unroll
+    for (int l = 0; l < 2; ++l) {
+      if (T == 2) {
+        sum[l][0] += sum[l][2];
+        sum[l][1] += sum[l][3];
+      }
+#pragma unroll
+      for (int e = 0; e < (T < 4 ? T : 4); ++e) {
+        if (T <= 4) sum[l][e] += __shfl_xor(sum[l][e], 16);
+        if (T <= 8) sum[l][e] += __shfl_xor(sum[l][e], 32);
+        if (4 * q + e < T)
+          gas[(4 * q + e) * ldg + l * H + col] =
+              sum[l][e] * sg[l][e] * (1.f - sg[l][e]) * tta_silu_grad(as[l][e]);
+      }
     }
   }
-  __syncthreads();
-  // 4. g_n2 = g_h @ w1[l] ([H, C] per degree); coefficient 0 also + g_a_s @ ws ([2H, C]).  The
-  //    x1 values step 5 needs are loaded first, so that they arrive during the products.
+  // the x1 values step 5 needs: they arrive during the products
   float x1v[NS][9][2];
-#pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    const int rr = wave + NW * s;
-    const int64_t n = n0 + rr;
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const int c = lane + 64 * hh;
-#pragma unroll
-      for (int j = 0; j < 9; ++j)
-        x1v[s][j][hh] = (rr < nv && c < C) ? p.x1[(n * 9 + j) * C + c] : 0.f;
-    }
-  }
+  node_vals(p.x1, x1v);
+  __syncthreads();
+  // 4. g_n2 = g_h @ w1[l] ([H, C] per degree); coefficient 0 also + g_a_s @ ws ([2H, C]), the gas
+  //    rows (stride ldg) as the A operand
   zero_acc(acc);
-  coef_mm<9>(buf, LDP, H, p.w1, (int64_t)H * C, C, C, wave, lane, acc);
-  // + g_a_s @ ws on coefficient 0: the gas rows (stride ldg) as the A operand
+  lin.run(buf, LDP, lane, acc);
   {
-    floatx4 acc0[9][MAXJ];
+    floatx4 acc0[1][1];
     zero_acc(acc0);
-    coef_mm<1>(gas, ldg, LH, p.ws, 0, C, C, wave, lane, acc0);
-#pragma unroll
-    for (int jj = 0; jj < MAXJ; ++jj) acc[0][jj] += acc0[0][jj];
+    if (T == 16) scal.start(p.ws, 0, C, LH, C, 0, wave, lane);
+    scal.run(gas, ldg, lane, acc0);
+    acc[0][0] += acc0[0][0];
   }
   __syncthreads();  // every wave is done reading g_h
+  if (cok) {
 #pragma unroll
-  for (int c = 0; c < 9; ++c)
+    for (int i = 0; i < P::TILES; ++i)
 #pragma unroll
-    for (int jj = 0; jj < MAXJ; ++jj) {
-      const int j = wave + NW * jj;
-      if (j >= C / 16) continue;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) lrow(buf, c, 4 * q + e)[j * 16 + r] = acc[c][jj][e];
-    }
+      for (int e = 0; e < 4; ++e) buf[(16 * i + 4 * q + e) * LDP + col] = acc[i][0][e];
+  }
   __syncthreads();
   // 5. g_x1 = norm_2 backward of g_n2 (LDS) with x1 from the registers loaded before step 4,
   //    plus g_x2
@@ -543,9 +597,8 @@ __global__ __launch_bounds__(NTH, 1) void k_spectral_block_bwd(SpecBwdArgs p) {
     const int rr = wave + NW * s;
     if (rr >= nv) continue;
     const int64_t n = n0 + rr;
-    const float* gs = lrow(buf, 0, rr);
     float gx[9][2];
-    rms_bwd_vals([&](int j, int hh) { return gs[j * NT * LDP + lane + 64 * hh]; },
+    rms_bwd_vals([&](int j, int hh) { return lrow<T>(buf, j, rr)[lane + 64 * hh]; },
                  [&](int j, int hh) { return x1v[s][j][hh]; }, p.aw2, p.inv2[n], C, lane, gx);
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) {
@@ -554,6 +607,21 @@ __global__ __launch_bounds__(NTH, 1) void k_spectral_block_bwd(SpecBwdArgs p) {
 #pragma unroll
       for (int j = 0; j < 9; ++j) p.g_x1[(n * 9 + j) * C + c] = gx[j][hh] + gx2[s][j][hh];
     }
+  }
+}
+
+// acc += X (16 rows, LDS stride LDP) @ W (K x ncol, row-major at ldw), one column tile per wave
+__device__ __forceinline__ void scalar_product(const float* X, int K, const float* __restrict__ W,
+                                               int ldw, int ncol, int wave, int lane,
+                                               floatx4 (&acc)[1][1]) {
+  if (K % 64 == 0) {
+    Product<Scalar, 4, 1> m;
+    m.start(W, 0, ldw, K, ncol, 0, wave, lane);
+    m.run(X, LDP, lane, acc);
+  } else {
+    Product<Scalar, 1, 1> m;
+    m.start(W, 0, ldw, K, ncol, 0, wave, lane);
+    m.run(X, LDP, lane, acc);
   }
 }
 
@@ -581,38 +649,32 @@ __global__ __launch_bounds__(NTH, 1) void k_energy_head_fwd(HeadArgs p) {
       buf[rr * LDP + ch] = rr < nv ? p.ne[(n0 + rr) * 9 * C + ch] : 0.f;
   __syncthreads();
   const int r = lane & 15, q = lane >> 4;
-  floatx4 acc[9][MAXJ];
+  floatx4 acc[1][1];
   zero_acc(acc);
-  coef_mm<1>(buf, LDP, C, p.w0t, 0, H, H, wave, lane, acc);
+  scalar_product(buf, C, p.w0t, H, H, wave, lane, acc);
   __syncthreads();
-#pragma unroll
-  for (int jj = 0; jj < MAXJ; ++jj) {
-    const int j = wave + NW * jj;
-    if (j >= H / 16) continue;
-    const int col = j * 16 + r;
+  if (wave < H / 16) {
+    const int col = wave * 16 + r;
     const float bias = p.b0[col];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int row = 4 * q + e;
-      const float a = acc[0][jj][e] + bias;
+      const float a = acc[0][0][e] + bias;
       if (row < nv) p.a1[(n0 + row) * H + col] = a;
       buf[row * LDP + col] = tta_silu(a);
     }
   }
   __syncthreads();
   zero_acc(acc);
-  coef_mm<1>(buf, LDP, H, p.w1t, 0, H, H, wave, lane, acc);
+  scalar_product(buf, H, p.w1t, H, H, wave, lane, acc);
   __syncthreads();
-#pragma unroll
-  for (int jj = 0; jj < MAXJ; ++jj) {
-    const int j = wave + NW * jj;
-    if (j >= H / 16) continue;
-    const int col = j * 16 + r;
+  if (wave < H / 16) {
+    const int col = wave * 16 + r;
     const float bias = p.b1[col];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int row = 4 * q + e;
-      const float a = acc[0][jj][e] + bias;
+      const float a = acc[0][0][e] + bias;
       if (row < nv) p.a2[(n0 + row) * H + col] = a;
       buf[row * LDP + col] = tta_silu(a);
     }
@@ -640,34 +702,28 @@ __global__ __launch_bounds__(NTH, 1) void k_energy_head_bwd(HeadArgs p) {
       buf[rr * LDP + ch] = rr < nv ? p.w2[ch] * tta_silu_grad(p.a2[(n0 + rr) * H + ch]) : 0.f;
   __syncthreads();
   const int r = lane & 15, q = lane >> 4;
-  floatx4 acc[9][MAXJ];
+  floatx4 acc[1][1];
   zero_acc(acc);
-  coef_mm<1>(buf, LDP, H, p.w1, 0, H, H, wave, lane, acc);
+  scalar_product(buf, H, p.w1, H, H, wave, lane, acc);
   __syncthreads();
-#pragma unroll
-  for (int jj = 0; jj < MAXJ; ++jj) {
-    const int j = wave + NW * jj;
-    if (j >= H / 16) continue;
-    const int col = j * 16 + r;
+  if (wave < H / 16) {
+    const int col = wave * 16 + r;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int row = 4 * q + e;
       buf[row * LDP + col] =
-          row < nv ? acc[0][jj][e] * tta_silu_grad(p.a1[(n0 + row) * H + col]) : 0.f;
+          row < nv ? acc[0][0][e] * tta_silu_grad(p.a1[(n0 + row) * H + col]) : 0.f;
     }
   }
   __syncthreads();
   zero_acc(acc);
-  coef_mm<1>(buf, LDP, H, p.w0, 0, C, C, wave, lane, acc);
-#pragma unroll
-  for (int jj = 0; jj < MAXJ; ++jj) {
-    const int j = wave + NW * jj;
-    if (j >= C / 16) continue;
-    const int col = j * 16 + r;
+  scalar_product(buf, H, p.w0, C, C, wave, lane, acc);
+  if (wave < C / 16) {
+    const int col = wave * 16 + r;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int row = 4 * q + e;
-      if (row < nv) p.g_ne[(n0 + row) * 9 * C + col] = acc[0][jj][e];
+      if (row < nv) p.g_ne[(n0 + row) * 9 * C + col] = acc[0][0][e];
     }
   }
   for (int rr = wave; rr < nv; rr += NW)
@@ -681,13 +737,9 @@ bool node_dims_ok(int64_t N, int C, int H) {
 
 }  // namespace
 
-// Nodes per workgroup of the node kernels: NT, or NT / 2 when NT-node workgroups would not
-// cover the compute units (their MFMA tiles keep NT rows, the rows past the workgroup's nodes
-// zero, so a half-full workgroup costs about what a full one does but the per-node phases --
-// loads, norms, stores -- halve and twice as many units work).
-static int spectral_npb(int64_t N) {
-  // compute units per device, queried once; atomics, since host threads calling the library at
-  // the same time may both fill an entry (with the same value)
+static int compute_units() {
+  // queried once per device; atomics, since host threads calling the library at the same time may
+  // both fill an entry (with the same value)
   static std::atomic<int> cus_of[64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
@@ -698,8 +750,41 @@ static int spectral_npb(int64_t N) {
       cus = 256;
     cus_of[dev].store(cus, std::memory_order_relaxed);
   }
-  return (N + NT - 1) / NT < cus ? NT / 2 : NT;
+  return cus;
 }
+
+// Nodes per energy-head workgroup: NT, or NT / 2 when NT-node workgroups would not cover the
+// compute units (the MFMA tile keeps NT rows, those past the workgroup's nodes zero; the per-node
+// phases halve and twice as many units work).
+static int head_nodes(int64_t N) { return (N + NT - 1) / NT < compute_units() ? NT / 2 : NT; }
+
+// Nodes per spectral workgroup: the fewest with at most one workgroup per compute unit.
+static int pick_nodes(int64_t N) {
+  for (int T = 2; T < 16; T *= 2)
+    if ((N + T - 1) / T <= compute_units()) return T;
+  return 16;
+}
+
+template <class Args>
+static void launch_nodes(void (*kernel)(Args), int T, const Args& p, hipStream_t stream) {
+  hipLaunchKernelGGL(kernel, dim3(tta_blocks(p.N, T)), dim3(NTH), 0, stream, p);
+}
+
+// The variant for p.N nodes; two chunks per weight group (Product's D) where the tiles of T nodes
+// leave the registers for it, one at T = 16 and for widths that are no multiple of 32.
+#define LAUNCH_SPECTRAL(kernel, p, stream)                                                        \
+  do {                                                                                            \
+    const int T_ = pick_nodes((p).N);                                                             \
+    const bool d2_ = (p).C % 32 == 0 && (p).H % 32 == 0;                                          \
+    if (T_ == 2)                                                                                  \
+      d2_ ? launch_nodes(kernel<2, 2>, 2, p, stream) : launch_nodes(kernel<2, 1>, 2, p, stream);  \
+    else if (T_ == 4)                                                                             \
+      d2_ ? launch_nodes(kernel<4, 2>, 4, p, stream) : launch_nodes(kernel<4, 1>, 4, p, stream);  \
+    else if (T_ == 8)                                                                             \
+      d2_ ? launch_nodes(kernel<8, 2>, 8, p, stream) : launch_nodes(kernel<8, 1>, 8, p, stream);  \
+    else                                                                                          \
+      launch_nodes(kernel<16, 1>, 16, p, stream);                                                 \
+  } while (0)
 
 extern "C" int tta_spectral_block_fwd(const float* x1, const float* aw2, const float* ab2,
                                       const float* ws_t, const float* bs, const float* w1t,
@@ -717,8 +802,8 @@ extern "C" int tta_spectral_block_fwd(const float* x1, const float* aw2, const f
   TTA_CHECK_ARG(!awn || (abn && yn && invn), "tta_spectral_block_fwd: incomplete next norm");
   if (N == 0) return tta::kOk;
   SpecFwdArgs p{x1, aw2, ab2, ws_t, bs, w1t, b1, w2t, b2, inv2, a_s, h, x2,
-                awn, abn, add0, yn, invn, N, (int)C, (int)H, eps, spectral_npb(N)};
-  hipLaunchKernelGGL(k_spectral_block_fwd, dim3(tta_blocks(N, p.npb)), dim3(NTH), 0, stream, p);
+                awn, abn, add0, yn, invn, N, (int)C, (int)H, eps};
+  LAUNCH_SPECTRAL(k_spectral_block_fwd, p, stream);
   TTA_CHECK_LAUNCH("tta_spectral_block_fwd");
   return tta::kOk;
 }
@@ -737,8 +822,8 @@ extern "C" int tta_spectral_block_bwd(const float* g_n, const float* x2, const f
                 "tta_spectral_block_bwd: null pointer");
   if (N == 0) return tta::kOk;
   SpecBwdArgs p{g_n, x2, awn, invn, res, x1, aw2, inv2, a_s, h, w1, w2, ws, g_x1, N, (int)C,
-                (int)H, spectral_npb(N)};
-  hipLaunchKernelGGL(k_spectral_block_bwd, dim3(tta_blocks(N, p.npb)), dim3(NTH), 0, stream, p);
+                (int)H};
+  LAUNCH_SPECTRAL(k_spectral_block_bwd, p, stream);
   TTA_CHECK_LAUNCH("tta_spectral_block_bwd");
   return tta::kOk;
 }
@@ -753,7 +838,7 @@ extern "C" int tta_energy_head_fwd(const float* ne, const float* w0t, const floa
                 "tta_energy_head_fwd: null pointer");
   if (N == 0) return tta::kOk;
   HeadArgs p{ne, w0t, b0, w1t, b1, w2, b2, nullptr, nullptr, a1, a2, node_e, nullptr, N, (int)C,
-             (int)H, spectral_npb(N)};
+             (int)H, head_nodes(N)};
   hipLaunchKernelGGL(k_energy_head_fwd, dim3(tta_blocks(N, p.npb)), dim3(NTH), 0, stream, p);
   TTA_CHECK_LAUNCH("tta_energy_head_fwd");
   return tta::kOk;
@@ -768,7 +853,7 @@ extern "C" int tta_energy_head_bwd(const float* a1, const float* a2, const float
   if (N == 0) return tta::kOk;
   HeadArgs p{nullptr, nullptr, nullptr, nullptr, nullptr, w2, nullptr, w0, w1,
              const_cast<float*>(a1), const_cast<float*>(a2), nullptr, g_ne, N, (int)C, (int)H,
-             spectral_npb(N)};
+             head_nodes(N)};
   hipLaunchKernelGGL(k_energy_head_bwd, dim3(tta_blocks(N, p.npb)), dim3(NTH), 0, stream, p);
   TTA_CHECK_LAUNCH("tta_energy_head_bwd");
   return tta::kOk;
