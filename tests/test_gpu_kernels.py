@@ -706,6 +706,51 @@ def test_gather_rotate_bw_dst_bit_equal(nat, C):
     assert ((gb - gn_).abs() / (gb.abs() + 1.0)).max() < 1e-5
 
 
+@pytest.mark.parametrize("C", [16, 64, 128])
+def test_node_walks_few_nodes(nat, C):
+    """The walks and segment sums of up to 512 nodes (eight wavefronts per node) against the
+    one-wavefront forms, which take the same edges with isolated nodes appended: degrees around the
+    eight edges of a round (0, 1, 7, 8, 9, 16, 17) and a hub.  The rotation adjoint rows are added
+    in one order, rounded: the same bits.  A segment sum's products may be contracted into the add
+    in one form and not the other: one more rounding per edge, (deg + 2) 2^-23 of the sum of the
+    magnitudes."""
+    deg = [0, 1, 7, 8, 9, 16, 17, 100, 0, 3]
+    g = torch.Generator().manual_seed(C)
+    tgt = torch.repeat_interleave(torch.arange(10), torch.tensor(deg))
+    E = tgt.numel()
+    src = tgt[torch.randperm(E, generator=g)]
+    r = lambda *s: torch.randn(*s, generator=g)
+    x, coef, rad, gout, gc0 = r(10, 9, C), r(E, 35), r(E, 6, 2 * C), r(E, 9, 2 * C), r(E, 35)
+    m, env = r(E, 9, C), torch.rand(E, generator=g)
+    f = lambda t: t.to(DEV).contiguous()
+    perm = torch.argsort(src, stable=True)
+    got = {}
+    for N in (10, 700):
+        xn = torch.zeros(N, 9, C)
+        xn[:10] = x
+        sp, tp = _i32(_csr(src, N)), _i32(_csr(tgt, N))
+        g_rad, half = torch.empty(E, 6, 2 * C, device=DEV), torch.empty(E, 35, device=DEV)
+        ssum, gn, s9, s3 = (torch.full((N, 9, C), float("nan"), device=DEV) for _ in range(4))
+        g_coef = f(gc0.clone())
+        nat.gather_rotate_bw_nodes(f(gout), f(rad), f(xn), sp, _i32(perm), tp, f(coef), g_rad,
+                                   g_coef, half, ssum, f(xn), gn)
+        nat.rotate_env_segsum(f(m), f(coef), f(env), tp, f(xn), s9, n_in=9, env_first=True)
+        nat.rotate_env_segsum(f(m[:, :3]), f(coef), f(env), tp, None, s3, n_in=3,
+                              env_first=False, div=5.0)
+        torch.cuda.synchronize()
+        assert torch.equal(gn[10:], f(xn)[10:]) and not s3[10:].any()
+        got[N] = [t.cpu() for t in (g_rad, g_coef, ssum[:10], gn[:10], s9[:10], s3[:10])]
+    for a, b in zip(got[10][:4], got[700][:4]):
+        assert torch.equal(a, b)
+    W = _dense(coef.double()).abs()
+    zero = torch.zeros(10, 9, C, dtype=torch.float64)
+    for k, mm, sc in ((4, m, env), (5, torch.cat([m[:, :3], torch.zeros(E, 6, C)], 1), env / 5)):
+        mag = zero.index_add(0, tgt, torch.bmm(W.transpose(1, 2), mm.double().abs())
+                             * sc.double()[:, None, None]) + (x.abs().double() if k == 4 else 0.0)
+        n = torch.tensor(deg, dtype=torch.float64)[:, None, None] + 2
+        assert ((got[10][k].double() - got[700][k].double()).abs() <= n * 2.0 ** -23 * mag).all()
+
+
 @pytest.mark.parametrize("C", [16, 128, 256, 1024])
 def test_node_gather_sum_order_and_hubs(nat, C):
     """Every node's sum is bit-equal to a plain fp32 loop in edge order (src edges in the

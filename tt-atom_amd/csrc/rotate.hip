@@ -17,6 +17,8 @@
 // float atomics, deterministic results.
 #include "common.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int NSPH = 9;
@@ -519,6 +521,135 @@ __global__ __launch_bounds__(256) void k_gather_rotate_bw_walk(
   }
 }
 
+// One edge's half of the rotation backward, from its rows gm of g_xf (overwritten by their radial
+// product), its radial rows rd and the node's rows in: the half's g_rad rows gr and the
+// inverse-rotated adjoint gi.
+template <int V>
+__device__ __forceinline__ void walk_edge(const float* c, const typename VecT<V>::T* in,
+                                          typename VecT<V>::T* gm, const typename VecT<V>::T* rd,
+                                          typename VecT<V>::T* gr, typename VecT<V>::T* gi) {
+  typename VecT<V>::T mr[NSPH];
+  rot_fwd(c, in, mr);
+  gr[0] = gm[0] * mr[0];
+  gr[1] = gm[1] * mr[1];
+  gr[2] = gm[2] * mr[2];
+  gr[3] = gm[3] * mr[3] + gm[5] * mr[5];
+  gr[4] = gm[4] * mr[4] + gm[6] * mr[6];
+  gr[5] = gm[7] * mr[7] + gm[8] * mr[8];
+#pragma unroll
+  for (int m = 0; m < NSPH; ++m) gm[m] = gm[m] * rd[rad_block(m)];
+  rot_inv<9>(c, gm, gi);
+}
+
+// The walks for few nodes: a workgroup of kFew wavefronts per node, one edge of a round each.
+// One wavefront per node leaves a small graph to a handful of wavefronts, each a serial chain of
+// one memory round trip per edge; here a round's edges run side by side (the next round's rows
+// in flight), their adjoint rows meet in LDS and every thread adds its elements in edge order, so
+// the node adjoint keeps the bits of the one-wavefront walk (times: few_nodes).
+constexpr int kFew = 8;
+
+// acc[i] (elements t, t + 64 kFew of a node's `len` = 9 C / V vectors) += the round's slots in order
+template <class T>
+__device__ __forceinline__ void add_slots(T (&acc)[2], const T* slot, int count, int len, int t) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int idx = t + 64 * kFew * i;
+    if (idx < len)
+      for (int s = 0; s < count; ++s) acc[i] = acc[i] + slot[s * len + idx];
+  }
+}
+
+template <int V, bool TGT>
+__global__ __launch_bounds__(64 * kFew) void k_gather_rotate_bw_walk_few(
+    const float* __restrict__ g_xf, const float* __restrict__ rad, const float* __restrict__ x,
+    const int* __restrict__ ptr, const int* __restrict__ perm, const float* __restrict__ coef,
+    float* __restrict__ g_rad, float* __restrict__ g_coef, float* __restrict__ coef_half,
+    const float* __restrict__ ssum, const float* __restrict__ res, float* __restrict__ out,
+    int C) {
+  typedef typename VecT<V>::T T;
+  extern __shared__ __align__(16) float lds[];
+  T* slots = reinterpret_cast<T*>(lds);  // [2][kFew][9][C / V]
+  const int t = threadIdx.x, lane = t & 63;
+  const int w = wave_uniform(t >> 6), n = blockIdx.x;
+  const int ki = halving_index<NNZ>(lane);  // the coefficient whose sum this lane ends with
+  const int kl = ki < 0 ? 0 : ki;
+  const int W = 2 * C, cq = C / V, len = NSPH * cq;
+  const bool active = lane < cq;
+  const int qq = active ? lane : 0;       // idle lanes load channel 0 and store nothing
+  const int co = (TGT ? C : 0) + V * qq;  // this lane's first channel within a 2C row
+  const int k0 = wave_uniform(ptr[n]), k1 = wave_uniform(ptr[n + 1]);
+  T in[NSPH], acc[2];
+  acc[0] = acc[1] = zv<V>();
+#pragma unroll
+  for (int j = 0; j < NSPH; ++j) in[j] = ldv<V>(x + (int64_t)n * NSPH * C + j * C + V * qq);
+  // an edge's operands; past the segment's end the last edge's again (loaded, not used)
+  struct Edge {
+    int64_t e;
+    T gm[NSPH], rd[6];
+    float cv, before, half0;
+  };
+  auto load = [&](int k, Edge& d) {
+    k = min(k, k1 - 1);
+    d.e = TGT ? k : wave_uniform(perm[k]);
+    d.cv = coef[d.e * NNZ + (lane < NNZ ? lane : 0)];
+    d.before = TGT ? g_coef[d.e * NNZ + kl] : 0.f;
+    d.half0 = TGT ? coef_half[d.e * NNZ + kl] : 0.f;
+#pragma unroll
+    for (int m = 0; m < NSPH; ++m) d.gm[m] = ldv_nt<V>(g_xf + d.e * NSPH * W + co + m * W);
+#pragma unroll
+    for (int b = 0; b < 6; ++b) d.rd[b] = ldv_nt<V>(rad + d.e * 6 * W + co + b * W);
+  };
+  Edge cur, nxt;
+  if (k0 < k1) load(k0 + w, cur);
+  int buf = 0;
+  for (int kb = k0; kb < k1; kb += kFew) {
+    load(kb + kFew + w, nxt);
+    T* slot = slots + (buf * kFew + w) * len;
+    if (kb + w < k1) {  // wave-uniform
+      float c[NNZ], gc[NNZ];
+#pragma unroll
+      for (int k = 0; k < NNZ; ++k) {
+        c[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cur.cv), k));
+        gc[k] = 0.f;
+      }
+      if (active) {
+        T gr[6], gi[NSPH];
+        walk_edge<V>(c, in, cur.gm, cur.rd, gr, gi);
+        float* grp = g_rad + cur.e * 6 * W + co;
+#pragma unroll
+        for (int b = 0; b < 6; ++b) stv<V>(grp + b * W, gr[b]);
+#pragma unroll
+        for (int j = 0; j < NSPH; ++j) slot[j * cq + lane] = gi[j];
+        coef_partials<9, V>(cur.gm, in, gc);
+      }
+      const float tot = halving_sums<NNZ>(gc, lane);
+      if (ki >= 0) {
+        if (TGT)
+          g_coef[cur.e * NNZ + ki] = cur.before + (cur.half0 + tot);
+        else
+          coef_half[cur.e * NNZ + ki] = tot;
+      }
+    }
+    cur = nxt;
+    __syncthreads();
+    // (the other buffer is free again: its adds came before this barrier)
+    add_slots(acc, slots + buf * kFew * len, min(kFew, k1 - kb), len, t);
+    buf ^= 1;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int idx = t + 64 * kFew * i;
+    if (idx >= len) continue;
+    const int64_t o = (int64_t)n * NSPH * C + V * idx;
+    T v = acc[i];
+    if (TGT) {
+      v = ldv<V>(ssum + o) + v;
+      if (res) v = v + ldv<V>(res + o);
+    }
+    stv<V>(out + o, v);
+  }
+}
+
 // -------------------------------------------------------------------------------------------
 // Inverse rotation + envelope + destination-sorted segmented sum (+ residual):
 //   out[n, j, :] = res[n, j, :] + sum_{e in [ptr[n], ptr[n+1])} contrib_e[j, :]
@@ -621,6 +752,75 @@ __global__ __launch_bounds__(256) void k_rotate_env_segsum(
         stv<V>(out + (int64_t)n * NSPH * C + j * C + V * q, v);
       }
     }
+  }
+}
+
+// The same for few nodes (k_gather_rotate_bw_walk_few's arrangement): kFew wavefronts per node, a
+// round's edges side by side, their contributions added in edge order from LDS.
+template <int V, int NIN, bool ENV_FIRST>
+__global__ __launch_bounds__(64 * kFew) void k_rotate_env_segsum_few(
+    const float* __restrict__ m, const float* __restrict__ coef, const float* __restrict__ env,
+    const int* __restrict__ ptr, const float* __restrict__ res, float* __restrict__ out, int C,
+    float div) {
+  typedef typename VecT<V>::T T;
+  extern __shared__ __align__(16) float lds[];
+  T* slots = reinterpret_cast<T*>(lds);  // [2][kFew][9][C / V]
+  const int t = threadIdx.x, lane = t & 63;
+  const int w = wave_uniform(t >> 6), n = blockIdx.x;
+  const int cq = C / V, len = NSPH * cq;
+  const bool active = lane < cq;
+  const int qq = active ? lane : 0;
+  const int e0 = wave_uniform(ptr[n]), e1 = wave_uniform(ptr[n + 1]);
+  const float rdiv = 1.f / div;
+  T acc[2], row[NIN], nrow[NIN];
+  acc[0] = acc[1] = zv<V>();
+  float ce = 0.f, nce = 0.f;  // lane k < 35: coefficient k; the others: the envelope
+  auto load = [&](int e, T (&r)[NIN], float& c) {
+    e = min(e, e1 - 1);
+    c = *(lane < NNZ ? coef + (int64_t)e * NNZ + lane : env + e);
+#pragma unroll
+    for (int mm = 0; mm < NIN; ++mm) r[mm] = ldv<V>(m + (int64_t)e * NIN * C + mm * C + V * qq);
+  };
+  if (e0 < e1) load(e0 + w, row, ce);
+  int buf = 0;
+  for (int eb = e0; eb < e1; eb += kFew) {
+    load(eb + kFew + w, nrow, nce);
+    if (eb + w < e1) {  // wave-uniform
+      float c[NNZ];
+#pragma unroll
+      for (int k = 0; k < NNZ; ++k)
+        c[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ce), k));
+      const float ev = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ce), NNZ));
+      T in[NSPH], o[NSPH];
+#pragma unroll
+      for (int mm = 0; mm < NSPH; ++mm) in[mm] = mm < NIN ? row[mm < NIN ? mm : 0] : zv<V>();
+      if (ENV_FIRST) {
+#pragma unroll
+        for (int mm = 0; mm < NIN; ++mm) in[mm] = in[mm] * ev;
+      }
+      rot_inv<NIN>(c, in, o);
+      const float sc = ENV_FIRST ? 1.f : ev * rdiv;
+      T* slot = slots + (buf * kFew + w) * len;
+      if (active) {
+#pragma unroll
+        for (int j = 0; j < NSPH; ++j) slot[j * cq + lane] = ENV_FIRST ? o[j] : o[j] * sc;
+      }
+    }
+#pragma unroll
+    for (int mm = 0; mm < NIN; ++mm) row[mm] = nrow[mm];
+    ce = nce;
+    __syncthreads();
+    add_slots(acc, slots + buf * kFew * len, min(kFew, e1 - eb), len, t);
+    buf ^= 1;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int idx = t + 64 * kFew * i;
+    if (idx >= len) continue;
+    const int64_t o = (int64_t)n * NSPH * C + V * idx;
+    T v = acc[i];
+    if (res) v = v + ldv<V>(res + o);
+    stv<V>(out + o, v);
   }
 }
 
@@ -746,6 +946,15 @@ int pick_v(int64_t W) {
   return 1;
 }
 
+// Whether a node-walking launch takes the form for few nodes: up to two workgroups per compute
+// unit (its LDS allows no more at C = 128), whole rows in one lane vector.  One wavefront per node ->
+// few-node form, us (both walks / segment sum of nine coefficients / of three): 24 nodes of 18
+// edges 52.5 -> 21.7 / 13.4 -> 6.0 / 7.3 -> 4.3; 256 of 30 116 -> 48 / 21.8 -> 10.2 / 9.8 -> 5.5;
+// 500 of 30 128 -> 87 / 22.4 -> 15.5 / 12.3 -> 7.2; 864 of 30 148 -> 151 / 25.4 -> 24.9 / 13.6 ->
+// 13.8; 2048 of 30 298 -> 319 / 52 -> 55 / 21 -> 25.
+bool few_nodes(int64_t N, int64_t C, int V) { return N <= 512 && V <= 2 && C / V <= 64; }
+size_t few_lds(int64_t C) { return 2 * kFew * NSPH * C * sizeof(float); }
+
 unsigned wave_blocks(int64_t items) { return (unsigned)((items + WAVES - 1) / WAVES); }
 
 }  // namespace
@@ -857,9 +1066,14 @@ extern "C" int tta_gather_rotate_bw_srcwalk(const float* g_xf, const float* rad,
                 "tta_gather_rotate_bw_srcwalk: null pointer");
   const int V = pick_v(C);
   TTA_V_DISPATCH(V, {
-    hipLaunchKernelGGL((k_gather_rotate_bw_walk<VV, false>), dim3(wave_blocks(N)), dim3(256), 0,
-                       stream, g_xf, rad, x, src_ptr, src_perm, coef, g_rad, nullptr, coef_half,
-                       nullptr, nullptr, ssum, (int)N, (int)C);
+    if (VV <= 2 && few_nodes(N, C, VV))
+      hipLaunchKernelGGL((k_gather_rotate_bw_walk_few<VV <= 2 ? VV : 2, false>), dim3((unsigned)N),
+                         dim3(64 * kFew), few_lds(C), stream, g_xf, rad, x, src_ptr, src_perm, coef, g_rad, nullptr, coef_half,
+                       nullptr, nullptr, ssum, (int)C);
+    else
+      hipLaunchKernelGGL((k_gather_rotate_bw_walk<VV, false>), dim3(wave_blocks(N)), dim3(256), 0,
+                         stream, g_xf, rad, x, src_ptr, src_perm, coef, g_rad, nullptr, coef_half,
+                         nullptr, nullptr, ssum, (int)N, (int)C);
   });
   TTA_CHECK_LAUNCH("tta_gather_rotate_bw_srcwalk");
   return tta::kOk;
@@ -878,9 +1092,14 @@ extern "C" int tta_gather_rotate_bw_tgtwalk(const float* g_xf, const float* rad,
                 "tta_gather_rotate_bw_tgtwalk: null pointer");
   const int V = pick_v(C);
   TTA_V_DISPATCH(V, {
-    hipLaunchKernelGGL((k_gather_rotate_bw_walk<VV, true>), dim3(wave_blocks(N)), dim3(256), 0,
-                       stream, g_xf, rad, x, tgt_ptr, nullptr, coef, g_rad, g_coef,
-                       const_cast<float*>(coef_half), ssum, res, out, (int)N, (int)C);
+    if (VV <= 2 && few_nodes(N, C, VV))
+      hipLaunchKernelGGL((k_gather_rotate_bw_walk_few<VV <= 2 ? VV : 2, true>), dim3((unsigned)N),
+                         dim3(64 * kFew), few_lds(C), stream, g_xf, rad, x, tgt_ptr, nullptr, coef, g_rad, g_coef,
+                       const_cast<float*>(coef_half), ssum, res, out, (int)C);
+    else
+      hipLaunchKernelGGL((k_gather_rotate_bw_walk<VV, true>), dim3(wave_blocks(N)), dim3(256), 0,
+                         stream, g_xf, rad, x, tgt_ptr, nullptr, coef, g_rad, g_coef,
+                         const_cast<float*>(coef_half), ssum, res, out, (int)N, (int)C);
   });
   TTA_CHECK_LAUNCH("tta_gather_rotate_bw_tgtwalk");
   return tta::kOk;
@@ -935,18 +1154,26 @@ extern "C" int tta_rotate_env_segsum(const float* m, const float* coef, const fl
   TTA_CHECK_ARG(coef && env && tgt_ptr && out && (m || E == 0), "tta_rotate_env_segsum: null pointer");
   const int V = pick_v(C);
   TTA_V_DISPATCH(V, {
+    auto launch = [&](auto nin, auto first) {
+      constexpr int NIN = decltype(nin)::value;
+      constexpr bool EF = decltype(first)::value;
+      if (few_nodes(N, C, VV))
+        hipLaunchKernelGGL((k_rotate_env_segsum_few<VV <= 2 ? VV : 2, NIN, EF>),
+                           dim3((unsigned)N), dim3(64 * kFew), few_lds(C), stream, m, coef, env,
+                           tgt_ptr, res, out, (int)C, div);
+      else
+        hipLaunchKernelGGL((k_rotate_env_segsum<VV, NIN, EF>), dim3(wave_blocks(N)), dim3(256), 0,
+                           stream, m, coef, env, tgt_ptr, res, out, (int)N, (int)C, div);
+    };
+    using std::integral_constant;
     if (n_in == 9 && env_first)
-      hipLaunchKernelGGL((k_rotate_env_segsum<VV, 9, true>), dim3(wave_blocks(N)), dim3(256), 0,
-                         stream, m, coef, env, tgt_ptr, res, out, (int)N, (int)C, div);
+      launch(integral_constant<int, 9>{}, std::true_type{});
     else if (n_in == 9)
-      hipLaunchKernelGGL((k_rotate_env_segsum<VV, 9, false>), dim3(wave_blocks(N)), dim3(256), 0,
-                         stream, m, coef, env, tgt_ptr, res, out, (int)N, (int)C, div);
+      launch(integral_constant<int, 9>{}, std::false_type{});
     else if (env_first)
-      hipLaunchKernelGGL((k_rotate_env_segsum<VV, 3, true>), dim3(wave_blocks(N)), dim3(256), 0,
-                         stream, m, coef, env, tgt_ptr, res, out, (int)N, (int)C, div);
+      launch(integral_constant<int, 3>{}, std::true_type{});
     else
-      hipLaunchKernelGGL((k_rotate_env_segsum<VV, 3, false>), dim3(wave_blocks(N)), dim3(256), 0,
-                         stream, m, coef, env, tgt_ptr, res, out, (int)N, (int)C, div);
+      launch(integral_constant<int, 3>{}, std::false_type{});
   });
   TTA_CHECK_LAUNCH("tta_rotate_env_segsum");
   return tta::kOk;
