@@ -256,6 +256,51 @@ def test_small_launch_gemm(nat, mode, M, N, K):
     assert ((outs[0].double() - ref).abs() / mag).max().item() < 4 * 2.0 ** -bits
 
 
+@pytest.mark.parametrize("M,N,K,epi", [(131_073, 260, 1024, 0), (132_000, 640, 512, 4),
+                                       (100_001, 512, 1056, 3), (262_200, 256, 768, 2),
+                                       (66_000, 1000, 1024, 1)])
+def test_wide_gemm(nat, M, N, K, epi):
+    """The 128 x 256 tile (mode 16, at least 3072 k columns per resident workgroup): ragged rows, a last
+    column tile of at most 128 and of more columns, every kind of epilogue, against fp64 on
+    sampled rows (the first and last tile's, and the scaled ones: a row 2^20 up, one 2^-30 down, one
+    that starts in the second half of K, one that grows 2^17 there and so changes its shift within
+    the loop), at the split kernel's fp32-level accuracy, and equal on a second call."""
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    A, B = r(M, K), r(K, N) / math.sqrt(K)
+    A[700] *= 2.0 ** 20
+    A[701] *= 2.0 ** -30
+    A[702, :K // 2] = 0.0
+    A[703, K // 2:] *= 2.0 ** 17
+    bias, C0, aux = r(N), r(M, N), r(M, N)
+    pw = nat.PackedWeight(B, nat.SPLIT_F16X3)
+    outs = []
+    for _ in range(2):
+        C, C2 = C0.clone(), torch.zeros(M, N, device=DEV)
+        nat.linear(A, pw, bias, out=C, epilogue=epi, out2=C2, aux=aux)
+        outs.append((C, C2))
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    rows = torch.cat([torch.arange(128), torch.arange(640, 768), torch.arange(M - 130, M),
+                      torch.randint(M, (200,), generator=torch.Generator().manual_seed(1))]).to(DEV)
+    a, b = A[rows].double(), B.double()
+    pre = a @ b + bias.double()
+    mag = a.abs() @ b.abs() + bias.double().abs()
+    ref = pre
+    if epi == 1:
+        ref = torch.nn.functional.silu(pre)
+    elif epi == 2:
+        ref, mag = pre + C0[rows].double(), mag + C0[rows].double().abs()
+    elif epi == 4:
+        s = torch.sigmoid(aux[rows].double())
+        d = s * (1 + aux[rows].double() * (1 - s))
+        ref, mag = pre * d, mag * (d.abs() + 0.05)
+    assert ((outs[0][0][rows].double() - ref).abs() / mag).max().item() < 2e-6
+    if epi == 3:
+        silu = torch.nn.functional.silu(pre)
+        assert ((outs[0][1][rows].double() - silu).abs() / mag).max().item() < 2e-6
+
+
 def test_gemm_batched_strided(nat):
     g = torch.Generator().manual_seed(5)
     N_, C, H = 50, 32, 24

@@ -299,11 +299,12 @@ __global__ __launch_bounds__(128 * WM, WM == 2 ? 2 : 1) void gemm_bf16x_kernel(G
       rs.check(x0, x1, acc, lh);
       sp(x0, ca);
       int kt = kt0;
-      // Fast loop (K a multiple of 32 and no row of the wave scaled: every product here): no
-      // branch between a k half's MFMAs and the split of the next half, which the scheduler
-      // interleaves.  x0 is split before its slab's shift check and split again in the rare case
-      // that the check rescales; a wave that acquires a nonzero shift finishes in the general loop.
-      if (K % BK == 0 && (!S::F16 || rs.unscaled)) {
+      // Fast loop (K a multiple of 32 and every row's shift 0: nearly every tile): no branch between
+      // a k half's MFMAs and the split of the next half, which the scheduler interleaves, and of the
+      // shift check only its overflow half, on the lane's own values.  x0 is split before its slab's
+      // check and split again in the rare case that the check rescales; a wave that acquires a
+      // nonzero shift finishes in the general loop.
+      if (K % BK == 0 && (!S::F16 || rs.all_zero())) {
         for (; kt < kt1; ++kt) {
           const int stg = (kt - kt0) & 1;
           rdB(stg, 1, nb);
@@ -316,9 +317,10 @@ __global__ __launch_bounds__(128 * WM, WM == 2 ? 2 : 1) void gemm_bf16x_kernel(G
           rdB(stg ^ 1, 0, cb);
           mm(na, nb);
           sp_fast(x0, ca);
-          if (rs.check(x0, x1, acc, lh)) {
+          if (rs.overflows(x0, x1)) {
+            rs.check(x0, x1, acc, lh);
             sp(x0, ca);
-            if (S::F16 && !rs.unscaled) {
+            if (!rs.unscaled) {
               ++kt;
               break;
             }
@@ -821,6 +823,8 @@ int launch_mode(GemmGroup& g, int n, int mode, hipStream_t s, unsigned chunks = 
     }
   }
   if (small_ok(g, n)) return launch_small(g, n, mode, s);
+  if (!(mode == 16 && panel_ok(g, n)) && wide_ok(g, n, mode, persistent_cap()))
+    return launch_wide(g, n, mode, persistent_cap(), s);
   switch (mode) {
     case 1: return launch_bf16x<2, 1>(g, n, s);
     case 3: return launch_bf16x<2, 3>(g, n, s);

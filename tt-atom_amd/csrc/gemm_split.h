@@ -388,6 +388,27 @@ struct RowScale {
     }
     return false;
   }
+  // Whether every row of the wavefront has a shift, 0; while that holds a slab needs a new shift only
+  // where a value reaches 2^15, which each lane can tell of its own values (overflows): no exchange
+  // with the lane that holds the row's other half.
+  __device__ __forceinline__ bool all_zero() const {
+    bool z = true;
+#pragma unroll
+    for (int i = 0; i < TI; ++i) z &= er[i] == 0;
+    return __all(z);
+  }
+  __device__ __forceinline__ bool overflows(const floatx4 (&x0)[TI][2],
+                                            const floatx4 (&x1)[TI][2]) const {
+    if constexpr (!F16) return false;
+    float m = 0.f;
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m = max3_abs(x0[i][c][e], x1[i][c][e], m);
+    return __any(!(m < 32768.f));
+  }
   __device__ __forceinline__ bool all_unscaled() const {
     bool u = true;
 #pragma unroll
@@ -416,5 +437,9 @@ __device__ __forceinline__ int aswz(int row) { return (row >> 1) & 7; }
 // The small-launch kernel (gemm_small.hip): whether the n products of g take it, and its launch.
 bool small_ok(const GemmGroup& g, int n);
 int launch_small(GemmGroup& g, int n, int mode, hipStream_t s);
+
+// The 128 x 256 kernel (gemm_wide.hip); cap: most blocks per product (persistent tiles).
+bool wide_ok(const GemmGroup& g, int n, int mode, int cap);
+int launch_wide(GemmGroup& g, int n, int mode, int cap, hipStream_t s);
 
 }  // namespace tta_gemm
