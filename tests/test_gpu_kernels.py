@@ -1256,3 +1256,36 @@ def test_ln_silu_groups_equal_per_group(nat, n):
         outs.append((nrm.clone(), s.clone(), ga.clone()))
     for x, y in zip(*outs):
         assert not bool(x.isnan().any()) and torch.equal(x, y)
+
+
+@pytest.mark.parametrize("packed", [False, True])
+def test_activation_accuracy(nat, packed):
+    """Sigmoid, SiLU and its derivative as the GEMM epilogues evaluate them, against fp64: a
+    product of zeros plus a bias that holds the arguments (the derivative: bias 1, arguments in
+    aux).  Bound: exp to 1 ulp of the hardware's 2^p and two roundings, 1 + e, the quotient and
+    the product to half an ulp each, 5 ulp = 6e-7 relative in all; the derivative's 1 + x (1 - s)
+    cancels, so its bound is 5 ulp of 1 + |x| in absolute terms times the sigmoid."""
+    x = torch.cat([torch.linspace(-87, 100, 4001), torch.randn(4000, generator=torch.Generator()
+                   .manual_seed(3)), torch.tensor([0.0, 1e-30, -1e-30])])
+    special = torch.tensor([float("inf"), float("-inf"), float("nan"), 3e38, -3e38])
+    args = torch.cat([x, special, torch.zeros(-(len(x) + 5) % 64)]).to(DEV)
+    M, N, K = 3, len(args), 64
+    w = torch.zeros(K, N, device=DEV)
+    w = nat.PackedWeight(w, 16) if packed else w
+    A = torch.zeros(M, K, device=DEV)
+    outs = [nat.linear(A, w, args, epilogue=e)[1].cpu() for e in (nat.EPI_SIGMOID, nat.EPI_SILU)]
+    aux = args.expand(M, N).contiguous()
+    one = torch.ones(N, device=DEV)
+    outs.append(nat.linear(A, w, one, epilogue=nat.EPI_SILU_GRAD, aux=aux)[2].cpu())
+    n, xd = len(x), x.double()
+    s = torch.sigmoid(xd)
+    sig, silu, grad = (o[:n].double() for o in outs)
+    assert ((sig - s).abs() <= 6e-7 * s).all()
+    assert ((silu - xd * s).abs() <= 6e-7 * (xd * s).abs()).all()
+    want = s * (1 + xd * (1 - s))
+    assert ((grad - want).abs() <= 6e-7 * s * (1 + xd.abs())).all()
+    sp = [o[n:n + 5] for o in outs]
+    nan, inf = float("nan"), float("inf")
+    torch.testing.assert_close(sp[0], torch.tensor([1.0, 0.0, nan, 1.0, 0.0]), equal_nan=True)
+    torch.testing.assert_close(sp[1], torch.tensor([inf, nan, nan, 3e38, 0.0]), equal_nan=True)
+    torch.testing.assert_close(sp[2], torch.tensor([nan, nan, nan, 1.0, 0.0]), equal_nan=True)
