@@ -371,6 +371,21 @@ def test_cell_list_dense_rows_and_large_cap():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("cap", [None, 1, 63, 64, 65, 128, 256, 257])
+def test_cell_list_row_sizes(cap):
+    """Separate blobs whose atoms all see each other: rows of 62 to 65, 127 to 129, 255 to 257 and
+    600 kept entries and as many cap candidates, around the 64 keys that are merged at a time and
+    the 256 entries that are placed by rank."""
+    rng = np.random.default_rng(6)
+    blobs = [rng.uniform(-1.5, 1.5, (n + 1, 3)) + [30.0 * q, 4.0 * q, 0.0] for q, n in
+             enumerate((1, 62, 63, 64, 65, 127, 128, 129, 255, 256, 257, 600))]
+    pos = torch.from_numpy(rng.permutation(np.concatenate(blobs)).astype(np.float32))
+    print(f"cell list row sizes: cap={cap}", flush=True)
+    _same(geometry.radius_graph(pos, 6.0, max_neighbors=cap),
+          geometry.radius_graph_device(pos, 6.0, max_neighbors=cap, method="cells"))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("cap", [None, 30])
 def test_cell_list_50k_cluster_equals_row_scan(cap):
     """A 50k-atom cluster: cell list == row scan edge for edge (the host list would need a

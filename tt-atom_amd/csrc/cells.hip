@@ -21,12 +21,16 @@
 //
 // Rows (one wavefront each, scanning the 9 contiguous x-runs of the 27 bins around the row atom):
 //  * thresholds (cap k only): the k-th smallest key (d2, id) of every receiver, kept by a
-//    streaming selection: a sorted buffer of the k smallest keys so far in LDS; every 64
-//    candidates below the buffer's current k-th key are sorted across the wave and merged in.
-//    Needs O(k) LDS whatever the number of candidates.
+//    streaming selection: a sorted buffer of the k smallest keys so far in LDS; candidates below
+//    the buffer's current k-th key are collected, and every 64 of them (and the rest at the end)
+//    are sorted across the wave and merged in.  A sort and merge costs as much as many candidate
+//    steps, and about one candidate in six is inside the cutoff sphere: collecting makes that one
+//    or two sorts per row where a sort at every step of every run made nine.  Needs O(k) LDS
+//    whatever the number of candidates.  (10,007 atoms, cutoff 6, cap 30: 84 -> 33 us.)
 //  * count: kept entries per row;
-//  * write: the row's kept ids gathered in LDS, sorted (bitonic), written at the caller's row
-//    offsets.  A row with more than kRowMax kept entries is not written (err[0] = 1): the caller
+//  * write: the row's kept ids gathered in LDS and written in order at the caller's row
+//    offsets: by rank (the number of smaller ids) up to kRankMax entries, bitonic sort above
+//    (38 -> 26 us there; count 18 -> 14).  A row with more than kRowMax kept entries is not written (err[0] = 1): the caller
 //    writes such a graph with the row-scan write pass, which streams its rows in order.
 #include "nl_math.h"
 
@@ -36,6 +40,8 @@ using namespace tta_nl;
 
 constexpr int kWaves = 4;      // rows per block of the count and write passes
 constexpr int kRowMax = 2048;  // kept entries of one row sorted in LDS by the write pass
+constexpr int kRankMax = 256;  // kept entries placed by rank: n / 64 compares per entry and lane,
+                               // against log2(n)^2 / 2 dependent LDS rounds of the sort
 constexpr int kScanChunk = 2048;  // bins per block of the bin-count scan (256 threads x 8)
 constexpr int kMaxK = 1024;    // largest cap of the threshold pass
 
@@ -91,7 +97,9 @@ __device__ __forceinline__ float3 image_point(const CL& p, int id) {
 }
 
 // Visits every binned point of the 27 bins around row atom pr, 64 per step (wave-uniform loop):
-// f(valid, q) per lane.
+// f(valid, q) per lane.  The nine runs' bounds are read side by side, one run per lane, and the
+// runs are walked as one concatenated list: a run of about 30 points alone fills half a step and
+// starts with a load of its bounds that the next one waits for.
 template <typename F>
 __device__ __forceinline__ void for_candidates(const CL& p, float3 pr, int lane, F&& f) {
   const Grid& g = p.g;
@@ -99,16 +107,28 @@ __device__ __forceinline__ void for_candidates(const CL& p, float3 pr, int lane,
   const int by = clamp_bin(bin_u(pr.y, g.oy, g.inv_h), g.ny);
   const int bz = clamp_bin(bin_u(pr.z, g.oz, g.inv_h), g.nz);
   const int x0 = max(bx - 1, 0), x1 = min(bx + 1, g.nx - 1);
-  for (int z = max(bz - 1, 0); z <= min(bz + 1, g.nz - 1); ++z)
-    for (int y = max(by - 1, 0); y <= min(by + 1, g.ny - 1); ++y) {
-      const int row = (z * g.ny + y) * g.nx;
-      const int s = p.bin_start[row + x0], e = p.bin_start[row + x1 + 1];
-      for (int i0 = s; i0 < e; i0 += 64) {
-        const int i = i0 + lane;
-        const bool ok = i < e;
-        f(ok, ok ? p.pts[i] : make_float4(0.f, 0.f, 0.f, 0.f));
-      }
-    }
+  const int y = by - 1 + lane % 3, z = bz - 1 + lane / 3;
+  int s = 0, len = 0;
+  if (lane < 9 && y >= 0 && y < g.ny && z >= 0 && z < g.nz) {
+    const int row = (z * g.ny + y) * g.nx;
+    s = p.bin_start[row + x0];
+    len = p.bin_start[row + x1 + 1] - s;
+  }
+  int off[9], shift[9], n = 0;  // run r holds list entries off[r] .. at points off[r] + shift[r] ..
+#pragma unroll
+  for (int r = 0; r < 9; ++r) {
+    off[r] = n;
+    shift[r] = __builtin_amdgcn_readlane(s, r) - n;
+    n += __builtin_amdgcn_readlane(len, r);
+  }
+  for (int i0 = 0; i0 < n; i0 += 64) {
+    const int i = i0 + lane;
+    int sh = shift[0];
+#pragma unroll
+    for (int r = 1; r < 9; ++r) sh = i >= off[r] ? shift[r] : sh;
+    const bool ok = i < n;
+    f(ok, ok ? p.pts[i + sh] : make_float4(0.f, 0.f, 0.f, 0.f));
+  }
 }
 
 // Mask of a (row atom, point) pair, evaluated as the row scan evaluates it.
@@ -242,7 +262,7 @@ __global__ __launch_bounds__(256) void k_cl_fill(CL p, int64_t P, const int* __r
 
 // ---------------------------------------------------------------------------- rows
 // Thresholds: k-th smallest cap key of every receiver t (sentinel when it has <= k candidates).
-// Dynamic LDS per wave: two key buffers of k entries and one 64-entry batch, (float, int) each.
+// Dynamic LDS per wave: two key buffers of k entries and 128 collected keys, (float, int) each.
 __global__ __launch_bounds__(256) void k_cl_thresh(CL p, int k, float* __restrict__ thr_d,
                                                    int* __restrict__ thr_a,
                                                    int* __restrict__ thr_c) {
@@ -252,47 +272,26 @@ __global__ __launch_bounds__(256) void k_cl_thresh(CL p, int k, float* __restric
   if (t >= p.N) return;
   float* bd[2];
   int* ba[2];
-  unsigned char* base = smem + (size_t)w * (size_t)(2 * k + 64) * 8;
+  unsigned char* base = smem + (size_t)w * (size_t)(2 * k + 128) * 8;
   bd[0] = (float*)base;
   ba[0] = (int*)(base + 4 * k);
   bd[1] = (float*)(base + 8 * k);
   ba[1] = (int*)(base + 12 * k);
   float* sd = (float*)(base + 16 * k);
-  int* sa = (int*)(base + 16 * k + 256);
+  int* sa = (int*)(base + 16 * k + 512);
   const float3 pt = ld3(p.pos, t);
-  int m = 0, cur = 0, total = 0;
+  int m = 0, cur = 0, total = 0, pend = 0;
   float td = __builtin_inff();  // current k-th key (+inf until the buffer holds k keys)
   int ta = 0x7fffffff;
-  for_candidates(p, pt, lane, [&](bool ok, float4 q) {
-    bool hit = false;
-    float d = __builtin_inff();
-    int a = 0x7fffffff;
-    if (ok) {
-      const int id = __float_as_int(q.w);
-      const float3 pq = make_float3(q.x, q.y, q.z);
-      if (!p.periodic) {
-        const float s = norm2_fma(pq, pt);
-        hit = s > 0.f && (double)s < p.mid2;
-        if (hit) d = cap_d2(pq, pt, make_float3(0.f, 0.f, 0.f));
-      } else {
-        const float d2 = sum_sq(rn_sub(pt.x, q.x), rn_sub(pt.y, q.y), rn_sub(pt.z, q.z));
-        hit = d2 <= p.cut2 && d2 > p.min2;
-        if (hit) {
-          const int j = id / p.n_cells, c = id - j * p.n_cells;
-          d = cap_d2(ld3(p.pos, j), pt, ld3(p.shifts, c));
-        }
-      }
-      if (hit) a = id;
-    }
-    total += __popcll(__ballot(hit));
-    const bool take = hit && klt(d, a, td, ta);
-    if (!__ballot(take)) return;
-    if (!take) {
-      d = __builtin_inff();
-      a = 0x7fffffff;
-    }
+  // merges the first min(pend, 64) collected keys into the buffer and moves the rest down
+  auto merge = [&]() {
+    wave_sync();
+    const int nb = min(pend, 64);
+    float d = lane < nb ? sd[lane] : __builtin_inff();
+    int a = lane < nb ? sa[lane] : 0x7fffffff;
+    const float rd = sd[64 + lane];
+    const int ra = sa[64 + lane];
     wave_sort(d, a, lane);
-    const int nb = __popcll(__ballot(take));
     sd[lane] = d;
     sa[lane] = a;
     wave_sync();
@@ -325,13 +324,49 @@ __global__ __launch_bounds__(256) void k_cl_thresh(CL p, int k, float* __restric
       }
     }
     wave_sync();
+    sd[lane] = rd;
+    sa[lane] = ra;
+    pend -= nb;
     cur ^= 1;
     m = min(k, m + nb);
     if (m == k) {
       td = bd[cur][k - 1];
       ta = ba[cur][k - 1];
     }
+  };
+  for_candidates(p, pt, lane, [&](bool ok, float4 q) {
+    bool hit = false;
+    float d = __builtin_inff();
+    int a = 0x7fffffff;
+    if (ok) {
+      const int id = __float_as_int(q.w);
+      const float3 pq = make_float3(q.x, q.y, q.z);
+      if (!p.periodic) {
+        const float s = norm2_fma(pq, pt);
+        hit = s > 0.f && (double)s < p.mid2;
+        if (hit) d = cap_d2(pq, pt, make_float3(0.f, 0.f, 0.f));
+      } else {
+        const float d2 = sum_sq(rn_sub(pt.x, q.x), rn_sub(pt.y, q.y), rn_sub(pt.z, q.z));
+        hit = d2 <= p.cut2 && d2 > p.min2;
+        if (hit) {
+          const int j = id / p.n_cells, c = id - j * p.n_cells;
+          d = cap_d2(ld3(p.pos, j), pt, ld3(p.shifts, c));
+        }
+      }
+      if (hit) a = id;
+    }
+    total += __popcll(__ballot(hit));
+    const bool take = hit && klt(d, a, td, ta);
+    const uint64_t bal = __ballot(take);
+    if (take) {
+      const int o = pend + __popcll(bal & ((1ull << lane) - 1ull));
+      sd[o] = d;
+      sa[o] = a;
+    }
+    pend += __popcll(bal);
+    if (pend >= 64) merge();
   });
+  if (pend) merge();
   if (lane == 0) {
     if (total <= k) {
       thr_d[t] = __builtin_inff();
@@ -399,6 +434,28 @@ __global__ __launch_bounds__(256) void k_cl_write(CL p, const float* __restrict_
     return;
   }
   if (cnt == 0) return;
+  const int64_t o = offsets[r];
+  auto put = [&](int64_t i, int id) {
+    if (!p.periodic) {
+      e_src[i] = r;
+      e_tgt[i] = id;
+    } else {
+      const int j = id / p.n_cells;
+      e_src[i] = j;
+      e_tgt[i] = r;
+      e_cell[i] = id - j * p.n_cells;
+    }
+  };
+  wave_sync();
+  if (cnt <= kRankMax) {
+    for (int i = lane; i < cnt; i += 64) {
+      const int id = s[i];
+      int rank = 0;
+      for (int q = 0; q < cnt; ++q) rank += s[q] < id;
+      put(o + rank, id);
+    }
+    return;
+  }
   int n = 64;
   while (n < cnt) n <<= 1;
   for (int i = cnt + lane; i < n; i += 64) s[i] = 0x7fffffff;
@@ -415,19 +472,7 @@ __global__ __launch_bounds__(256) void k_cl_write(CL p, const float* __restrict_
       }
       wave_sync();
     }
-  const int64_t o = offsets[r];
-  for (int i = lane; i < cnt; i += 64) {
-    const int id = s[i];
-    if (!p.periodic) {
-      e_src[o + i] = r;
-      e_tgt[o + i] = id;
-    } else {
-      const int j = id / p.n_cells;
-      e_src[o + i] = j;
-      e_tgt[o + i] = r;
-      e_cell[o + i] = id - j * p.n_cells;
-    }
-  }
+  for (int i = lane; i < cnt; i += 64) put(o + i, s[i]);
 }
 
 }  // namespace
@@ -519,7 +564,7 @@ extern "C" int tta_radius_graph_cells_thresholds(const float* pos, int64_t N, co
   const CL p = make_cl(pos, N, shifts, n_cells, periodic, grid, bin_start, points, mid2, cut2,
                        min2);
   const int waves = k <= 256 ? 4 : 1;
-  const size_t lds = (size_t)waves * (size_t)(2 * k + 64) * 8;
+  const size_t lds = (size_t)waves * (size_t)(2 * k + 128) * 8;
   hipLaunchKernelGGL(k_cl_thresh, dim3(tta_blocks(N, waves)), dim3(64 * waves), lds, stream, p,
                      k, thr_d2, thr_src, thr_cell);
   TTA_CHECK_LAUNCH("tta_radius_graph_cells_thresholds");
