@@ -30,8 +30,9 @@
 //  * count: kept entries per row;
 //  * write: the row's kept ids gathered in LDS and written in order at the caller's row
 //    offsets: by rank (the number of smaller ids) up to kRankMax entries, bitonic sort above
-//    (38 -> 26 us there; count 18 -> 14).  A row with more than kRowMax kept entries is not written (err[0] = 1): the caller
-//    writes such a graph with the row-scan write pass, which streams its rows in order.
+//    (38 -> 26 us there; count 18 -> 14).  A row with more than kRowMax kept entries is not
+//    written (err[0] = 1): the caller writes such a graph with the row-scan write pass, which
+//    streams its rows in order.
 #include "nl_math.h"
 
 namespace {
