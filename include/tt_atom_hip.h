@@ -406,6 +406,15 @@ int tta_orb_edge_features_bwd(const float* vec, const float* g_feat, const float
 int tta_rms_residual(const float* h, const float* w, const float* x_old, float* u, float* x_new,
                      float* inv, const float* attn_w, const float* attn_b, float* sig, int64_t R,
                      int64_t C, float eps, tta_stream_t stream);
+/* tta_rms_residual with x_new's row r written at row_map[r] (a permutation of the R rows). */
+int tta_rms_residual_rows(const float* h, const float* w, const float* x_old, float* u,
+                          float* x_new, float* inv, const int* row_map, int64_t R, int64_t C,
+                          float eps, tta_stream_t stream);
+/* out [R, C] = x[row_map] and its attention gates sig [R, 2] = sigmoid(out . (w_r, w_s) + b)
+ * (orb_model.py:225-246); row_map null: the rows as they are, out null: the gates only. */
+int tta_orb_gather_gates(const float* x, const int* row_map, const float* attn_w,
+                         const float* attn_b, float* out, float* sig, int64_t R, int64_t C,
+                         tta_stream_t stream);
 /* g_h = inv w g - inv^3 / C h sum(g w h)  (rmsnorm_bw, orb_forces.py:67-79). */
 int tta_rms_bwd(const float* g, const float* h, const float* w, const float* inv, float* g_h,
                 int64_t R, int64_t C, tta_stream_t stream);
@@ -422,6 +431,13 @@ int tta_orb_edge_bwd(float* g_e, const float* g_node_in, const float* ue, const 
                      const float* cut, const float* h2, const float* inv, const float* wn,
                      const float* attn_w, const int* send, const int* recv, float* g_h2,
                      float* g_cut, int64_t N, int64_t E, int64_t C, tta_stream_t stream);
+/* tta_orb_edge_bwd with g_e's incoming value read from row g_row[e] of g_from (another tensor);
+ * g_e is only written. */
+int tta_orb_edge_bwd_rows(const float* g_from, const int* g_row, float* g_e,
+                          const float* g_node_in, const float* ue, const float* sig,
+                          const float* cut, const float* h2, const float* inv, const float* wn,
+                          const float* attn_w, const int* send, const int* recv, float* g_h2,
+                          float* g_cut, int64_t N, int64_t E, int64_t C, tta_stream_t stream);
 /* out [N, 2H] = [sum_send x | sum_recv x] for x [E, H]: the gather adjoints of orb_forces.py:131-
  * 133 moved in front of the (linear) first-layer weight product. */
 int tta_orb_node_segsum2(const float* x, const int* send_ptr, const int* recv_ptr,

@@ -85,6 +85,47 @@ def test_row_kernels(nat):
     assert (gh.cpu().double() - ref).abs().max() < 5e-6
 
 
+@pytest.mark.parametrize("R,C", [(1, 4), (5, 60), (7, 256), (66, 260), (9, 1024)])
+def test_row_kernels_in_another_order(nat, R, C):
+    """Gates with a row gather, the residual with its rows scattered and the edge adjoint with
+    its incoming rows gathered: the same bits as the plain kernels with torch's indexing around
+    them, the gates against fp64 (a dot product of C terms in fp32: C ulp of its absolute sum,
+    times the sigmoid's slope of 1/4)."""
+    g = torch.Generator().manual_seed(R)
+    t = lambda *sh: torch.randn(*sh, generator=g).to("cuda")
+    rows = torch.randperm(R, generator=g).to("cuda")
+    r32 = rows.int()
+    x, aw, ab = t(R, C), t(2 * C), t(2)
+    e = lambda *sh: torch.full(sh, float("nan"), device="cuda")
+    out, sig, sig2 = e(R, C), e(R, 2), e(R, 2)
+    nat.orb_gather_gates(x, r32, aw, ab, out, sig)
+    assert torch.equal(out, x[rows])
+    nat.orb_gather_gates(x[rows].contiguous(), None, aw, ab, None, sig2)
+    assert torch.equal(sig, sig2)
+    w2 = aw.view(2, C).double()
+    ref = torch.sigmoid(x[rows].double() @ w2.t() + ab.double())
+    bound = 0.25 * C * 2.0 ** -24 * (x[rows].double().abs() @ w2.abs().t() + ab.abs()) + 1e-7
+    assert ((sig.double() - ref).abs() <= bound).all()
+
+    h, w = t(R, C), t(C)
+    u0, xn0, inv0, u1, xn1, inv1 = e(R, C), e(R, C), e(R), e(R, C), e(R, C), e(R)
+    nat.rms_residual(h, w, x, u0, xn0, inv0)
+    nat.rms_residual_rows(h, w, x, u1, xn1, inv1, r32)
+    assert torch.equal(u0, u1) and torch.equal(inv0, inv1) and torch.equal(xn0, xn1[rows])
+
+    N = 3
+    gni, cut = t(N, 3 * C), t(R)
+    send, recv = (torch.randint(N, (R,), generator=g).int().to("cuda") for _ in range(2))
+    res = []
+    for direct in (False, True):
+        g_e = e(R, C) if direct else x[rows].contiguous()
+        g_h2, g_cut = e(R, C), torch.zeros(R, device="cuda")
+        nat.orb_edge_bwd(g_e, gni, u0, sig, cut, h, inv0, w, aw, send, recv, g_h2, g_cut,
+                         *((x, r32) if direct else ()))
+        res.append((g_e, g_h2, g_cut))
+    assert all(torch.equal(a, b) for a, b in zip(*res))
+
+
 def _tiny_batch(K=3, seed=11, cfg=None, n_min=6, n_max=14, side=5.0):
     cfg = dict(S.CFG_ORB_TINY if cfg is None else cfg)
     w = S.random_orb_weights(cfg, seed + S.WEIGHT_SEED_OFFSET)

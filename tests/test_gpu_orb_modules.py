@@ -103,6 +103,30 @@ def test_attention_layer_module(cond):
     _close(g_cut[:, 0], gc_ref, 5e-5, "attn_layer_bw cutoff")
 
 
+def test_attention_layer_module_layouts():
+    """Edge rows and their adjoints as views that the row kernels cannot read in place (a slice
+    off 16-byte alignment, strided rows, more rows than edges): the same bits as contiguous ones."""
+    cfg, w, C, H, N, E, senders, receivers, cut, _, g = _setup(False)
+    layer = orb_model.AttentionInteractionLayer(w, "gnn_stacks.0", DEV, latent_dim=C,
+                                                hidden_dim=H)
+    graph = _graph(N, senders, receivers, cut, None)
+    r = lambda *sh: torch.randn(*sh, generator=g).to(DEV)
+    nodes, gn, edges, ge = r(N, C), r(N, C), r(E, C), r(E, C)
+
+    def off(t):
+        flat = torch.empty(t.numel() + 1, device=DEV)[1:].view_as(t)
+        return flat.copy_(t)
+
+    wide = lambda t: torch.cat([t, t], 1)[:, :C]
+    long = lambda t: torch.cat([t, t])
+    res = []
+    for f in (lambda t: t, off, wide, long):
+        out = layer(nodes, f(edges), graph)
+        res.append(tuple(out) + tuple(orb_forces.attn_layer_bw(layer, graph, gn, f(ge))))
+    for other in res[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(res[0], other))
+
+
 def test_energy_head_and_backbone_bw():
     """EnergyHead (one system and a batch of three) with energy_bw(_batch), and backbone_bw over
     module calls (encoder, both layers, head) against autograd of the oracle's composition."""

@@ -83,10 +83,14 @@ _SIGS = {
     "tta_orb_edge_features": [_P, _P, _P, _P, _F, _I64, _P, _P, _P, _I64, _I64, _P],
     "tta_orb_edge_features_bwd": [_P, _P, _P, _F, _I64, _P, _I64, _P],
     "tta_rms_residual": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _F, _P],
+    "tta_rms_residual_rows": [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _F, _P],
+    "tta_orb_gather_gates": [_P, _P, _P, _P, _P, _P, _I64, _I64, _P],
     "tta_rms_bwd": [_P, _P, _P, _P, _P, _I64, _I64, _P],
     "tta_orb_segsum": [_P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _P],
     "tta_orb_edge_bwd": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64,
                          _P],
+    "tta_orb_edge_bwd_rows": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I64,
+                              _I64, _I64, _P],
     "tta_orb_node_segsum2": [_P, _P, _P, _P, _P, _I64, _I64, _I64, _P],
     "tta_segment_mean": [_P, _P, _P, _I64, _I64, _P],
     "tta_segment_mean_bwd": [_P, _P, _P, _P, _I64, _I64, _P],
@@ -1243,6 +1247,35 @@ def rms_residual(h, w, x_old, u, x_new, inv, attn_w=None, attn_b=None, sig=None,
               _stream())
 
 
+def rms_residual_rows(h, w, x_old, u, x_new, inv, rows, eps=1e-6):
+    """rms_residual with row r of x_new written at row rows[r] (int32, a permutation)."""
+    R, C = h.shape
+    n = R * C
+    _hbm_call("k_rms_residual", 4 * (4 * n + C + 2 * R), "tta_rms_residual_rows",
+              _ptr(h, numel=n, name="h"), _ptr(w, numel=C, name="w"),
+              _ptr(x_old, numel=n, name="x_old"), _ptr(u, numel=n, name="u"),
+              _ptr(x_new, numel=n, name="x_new"), _ptr(inv, numel=R, name="inv"),
+              _i32(rows, R, "rows"), R, C, float(eps), _stream())
+
+
+def rows_direct(t, E, C):
+    """Whether the row kernels can read t's E rows of C themselves (float4 rows in place);
+    other shapes, layouts and alignments go through torch's indexing first."""
+    return tuple(t.shape) == (E, C) and t.is_contiguous() and t.data_ptr() % 16 == 0
+
+
+def orb_gather_gates(x, rows, attn_w, attn_b, out, sig):
+    """sig [R, 2] = the attention gates of x's rows; with ``rows`` (int32) of x[rows], which is
+    also written to ``out``."""
+    R, C = sig.shape[0], x.shape[1]
+    _hbm_call("k_gather_gates", 4 * ((2 if out is not None else 1) * R * C + 3 * R + 2 * C),
+              "tta_orb_gather_gates", _ptr(x, numel=R * C, name="x"),
+              None if rows is None else _i32(rows, R, "rows"),
+              _ptr(attn_w, numel=2 * C, name="attn_w"), _ptr(attn_b, numel=2, name="attn_b"),
+              None if out is None else _ptr(out, numel=R * C, name="out"),
+              _ptr(sig, numel=2 * R, name="sig"), R, C, _stream())
+
+
 def rms_bwd(g, h, w, inv, g_h):
     R, C = h.shape
     _hbm_call("k_rms_bwd", 4 * (3 * R * C + R + C), "tta_rms_bwd",
@@ -1264,13 +1297,18 @@ def orb_segsum(ue, sig, cut, send_ptr, recv_ptr, recv_perm, nodes, node_in):
               compulsory=nbytes - 4 * E * C)
 
 
-def orb_edge_bwd(g_e, g_node_in, ue, sig, cut, h2, inv, wn, attn_w, send, recv, g_h2, g_cut):
+def orb_edge_bwd(g_e, g_node_in, ue, sig, cut, h2, inv, wn, attn_w, send, recv, g_h2, g_cut,
+                 g_from=None, rows=None):
+    """``g_from`` [E, C], ``rows`` (int32): g_e's incoming value is g_from[rows] and g_e is only
+    written."""
     E, C = ue.shape
     N = g_node_in.shape[0]
     n = E * C
     # g_e read and rewritten, two gathered node-row slices per edge, ue, h2, g_h2
     nbytes = 4 * (7 * n + 8 * E + 3 * C)
-    _hbm_call("k_edge_bwd", nbytes, "tta_orb_edge_bwd", _ptr(g_e, numel=n, name="g_e"),
+    lead = () if g_from is None else (_ptr(g_from, numel=n, name="g_from"), _i32(rows, E, "rows"))
+    _hbm_call("k_edge_bwd", nbytes, "tta_orb_edge_bwd" if g_from is None
+              else "tta_orb_edge_bwd_rows", *lead, _ptr(g_e, numel=n, name="g_e"),
               _ptr(g_node_in, numel=N * 3 * C, name="g_node_in"), _ptr(ue, numel=n),
               _ptr(sig, numel=2 * E), _ptr(cut, numel=E), _ptr(h2, numel=n),
               _ptr(inv, numel=E), _ptr(wn, numel=C), _ptr(attn_w, numel=2 * C), _i32(send, E),

@@ -62,7 +62,11 @@ def attn_layer_bw(layer, graph, g_nodes_out, g_edges_out):
     N, E, H = graph.N, graph.E, p.edge.hidden
     dev = t.send.device
     g_n = g_nodes_out.to(device=dev, dtype=torch.float32).clone()
-    g_e = g_edges_out.to(device=dev, dtype=torch.float32)[t.order].contiguous()
+    g_in, g_rows = g_edges_out.to(device=dev, dtype=torch.float32), t.order32
+    if nat.rows_direct(g_in, E, C):
+        g_e = _empty(E, C, like=g_n)
+    else:
+        g_e, g_in, g_rows = g_in[t.order].contiguous(), None, None
     g_cut = torch.zeros(E, device=dev, dtype=torch.float32)
     Hn = p.node.hidden
     g_hn2, g_an1, g_an0 = _empty(N, C, like=g_n), _empty(N, Hn, like=g_n), _empty(N, Hn, like=g_n)
@@ -72,7 +76,7 @@ def attn_layer_bw(layer, graph, g_nodes_out, g_edges_out):
     g_node_in = nat.linear(g_an0, p.node.w[0])                          # [N, 3C]
     g_h2 = _empty(E, C, like=g_n)
     nat.orb_edge_bwd(g_e, g_node_in, c["ue"], c["sig"], t.cut, c["h2"], c["inv"], p.edge.norm,
-                     p.attn_w, t.send, t.recv, g_h2, g_cut)
+                     p.attn_w, t.send, t.recv, g_h2, g_cut, g_in, g_rows)
     g_a1, g_a0 = _empty(E, H, like=g_n), _empty(E, H, like=g_n)
     nat.linear(g_h2, p.edge.w[2], out=g_a1, epilogue=nat.EPI_SILU_GRAD, aux=c["a1"])
     nat.linear(g_a1, p.edge.w[1], out=g_a0, epilogue=nat.EPI_SILU_GRAD, aux=c["a0"])

@@ -152,8 +152,6 @@ class AttentionInteractionLayer:
             raise ValueError(f"{prefix}: MLP hidden width is {self._p.edge.hidden}, expected "
                              f"{hidden_dim}")
         self.has_cond = self._p.cond_w_t is not None
-        # the two attention linears as one [C, 2] product (receive, send)
-        self._attn_w_t = self._p.attn_w.view(2, self.C).t().contiguous()
 
     def __call__(self, nodes, edges, graph):
         """(nodes [N, C], edges [E, C]) -> (nodes + node update, edges + edge update), one
@@ -171,9 +169,15 @@ class AttentionInteractionLayer:
         if self.has_cond and graph.cond_nodes is not None:
             nat.linear(_f32(graph.cond_nodes, dev), p.cond_w_t, p.cond_b, out=n_l,
                        epilogue=nat.EPI_ACCUM)
-        e_s = _f32(edges, dev)[order].contiguous()            # sender order inside
-        sig = f(E, 2)
-        nat.linear(e_s, self._attn_w_t, p.attn_b, out=sig, epilogue=nat.EPI_SIGMOID)
+        # sender order inside; the gates come with the gather, the residual's rows go back to the
+        # caller's order as they are written
+        e, sig = _f32(edges, dev), f(E, 2)
+        if nat.rows_direct(e, E, C):
+            e_s = f(E, C)
+            nat.orb_gather_gates(e, t.order32, p.attn_w, p.attn_b, e_s, sig)
+        else:
+            e_s = e[order].contiguous()
+            nat.orb_gather_gates(e_s, None, p.attn_w, p.attn_b, None, sig)
         P = f(N, 2 * H)
         nat.linear(n_l, p.wsr_t, out=P)
         a0, h0, a1, h1, h2 = f(E, H), f(E, H), f(E, H), f(E, H), f(E, C)
@@ -182,7 +186,7 @@ class AttentionInteractionLayer:
         nat.linear(h0, p.edge.w_t[1], p.edge.b[1], out=a1, epilogue=nat.EPI_PRE_SILU, out2=h1)
         nat.linear(h1, p.edge.w_t[2], p.edge.b[2], out=h2)
         ue, e_new, inv = f(E, C), f(E, C), f(E)
-        nat.rms_residual(h2, p.edge.norm, e_s, ue, e_new, inv)
+        nat.rms_residual_rows(h2, p.edge.norm, e_s, ue, e_new, inv, t.order32)
         node_in = f(N, 3 * C)
         nat.orb_segsum(ue, sig, t.cut, t.send_ptr, t.recv_ptr, t.recv_perm, n_l, node_in)
         Hn = p.node.hidden
@@ -195,9 +199,7 @@ class AttentionInteractionLayer:
         nat.rms_residual(hn2, p.node.norm, n_l, None, n_new, ninv)
         self._cache = dict(sig=sig, a0=a0, a1=a1, h2=h2, ue=ue, inv=inv, an0=an0, an1=an1,
                            hn2=hn2, ninv=ninv, graph=graph)
-        e_out = torch.empty_like(e_new)
-        e_out[order] = e_new
-        return n_new, e_out
+        return n_new, e_new
 
 
 class _HeadModule:
@@ -296,6 +298,7 @@ class OrbGraphContext:
             t.cut = _f32(self.cutoff, self.device).reshape(-1)[t.order].contiguous()
             t.inv_order = torch.empty_like(t.order)
             t.inv_order[t.order] = torch.arange(self.E, device=t.order.device)
+            t.order32 = t.order.to(torch.int32)
             self._topo = t
         return self._topo
 
