@@ -628,6 +628,38 @@ def test_edge_geometry_fwd_equals_two_passes(nat, E, nb, ec, periodic):
         assert torch.equal(x, y), name
 
 
+@pytest.mark.parametrize("E,nb", [(1, 16), (15, 32), (17, 512), (32768, 30), (98304, 16)])
+def test_edge_geometry_block_sizes(nat, E, nb):
+    """The edge geometry of E edges, at most 32,768 backward and 98,304 forward of which run in
+    short blocks: the same bits as the first E edges of a graph of 100,000 (long blocks; their own
+    arithmetic is checked against fp64 here and in the tests around)."""
+    g = torch.Generator(device=DEV).manual_seed(E)
+    big, N, ec = 100_000, 60, 4
+    r = lambda *sh: torch.randn(*sh, generator=g, device=DEV)
+    i = lambda hi: torch.randint(hi, (big,), generator=g, device=DEV)
+    pos, shift = 4 * r(N, 3), r(big, 3)
+    src = i(N)
+    tgt = (src + 1 + i(N - 1)) % N
+    zs, zt, semb, temb = i(10), i(10), r(10, ec), r(10, ec)
+    off = torch.linspace(0, 6.0, nb, device=DEV)
+    jdf = torch.cat([j.reshape(-1) for j in _jd()]).to(DEV)
+    gc, ge, gg = r(big, 35), r(big), r(big, nb)
+    res = []
+    for n in (E, big):
+        o = [torch.full(sh, 7.0, device=DEV) for sh in
+             ((n, 3), (n,), (n, 35), (n, nb + 2 * ec), (n,), (n, 3))]
+        c = lambda t: t[:n].int().contiguous()
+        nat.edge_geometry_fwd(pos, c(src), c(tgt), shift[:n].contiguous(), jdf, 0.3, c(zs), c(zt),
+                              semb, temb, off, -2.0, 6.0, nb, ec, *o[:5])
+        nat.edge_geometry_bwd(o[0], o[1], gc[:n].contiguous(), ge[:n].contiguous(),
+                              gg[:n].contiguous(), nb, off, -2.0, 6.0, nb, jdf, 0.3, o[5])
+        res.append(o)
+    for a, b in zip(*res):
+        assert torch.equal(a, b[:E])
+    x = torch.exp(-2.0 * (res[0][1].double()[:, None] - off.double()) ** 2)
+    assert (res[0][3][:, :nb].double() - x).abs().max() < 1e-5
+
+
 def test_geometry_vjp_matches_autograd(nat):
     jd = _jd()
     ev = _test_vectors(400, 1)

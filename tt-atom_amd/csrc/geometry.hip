@@ -109,15 +109,21 @@ __global__ __launch_bounds__(256) void k_edge_features_v4(
   if (lane == 0) env[e] = tta_geo::envelope(d, cutoff);
 }
 
-// The two forward kernels above in one pass, 64 edges per 256-thread block.  Wave 0 forms the
+// The two forward kernels above in one pass, EPB edges per 256-thread block.  Wave 0 forms the
 // block's edge vectors and distances (one lane per edge, into LDS with the edges' species), then
 // the Wigner coefficients, while waves 1-3 write the block's feature rows with the arithmetic of
-// k_edge_features_v4.  The rows of 64 consecutive edges are one contiguous range, taken as a flat
+// k_edge_features_v4.  The rows of the block's edges are one contiguous range, taken as a flat
 // sequence of float4 columns over the 192 threads, so the stores are contiguous across the waves
 // and every thread has independent columns in flight.  The serial Wigner evaluation overlaps the
 // row stores instead of running as a launch of its own with one wavefront per SIMD.  Coefficient
 // rows and edge vectors leave through LDS with consecutive lanes on consecutive floats.
+// EPB = 16 up to 24 blocks per CU, 64 (one edge per lane of wave 0) above: a block's time is its
+// rows' exponentials, and short blocks spread them, until the waves of the Wigner evaluation with
+// three quarters of their lanes idle cost more (64 -> 16, nb = 512, ec = 128, us: 514 edges 25.6
+// -> 8.5, 7,680 27.8 -> 11.7, 24,000 31.8 -> 17.7, 61,440 37.5 -> 33.8, 100,000 63.7 -> 59.3,
+// 130,000 87.7 -> 94.8, 300,000 198.9 -> 229.3).
 // Requires the v4 conditions of k_edge_features_v4 and (nb + 2 ec) / 4 < 2^12.
+template <int EPB>
 __global__ __launch_bounds__(256) void k_edge_geometry_fwd(
     const float* __restrict__ pos, const int* __restrict__ src, const int* __restrict__ tgt,
     const float* __restrict__ shift, const float* __restrict__ jd, float gamma,
@@ -125,12 +131,12 @@ __global__ __launch_bounds__(256) void k_edge_geometry_fwd(
     const float* __restrict__ temb, const float* __restrict__ off, float coeff, float cutoff,
     int nb, int ec, float* __restrict__ ev_out, float* __restrict__ dist_out,
     float* __restrict__ coef_out, float* __restrict__ x_edge, float* __restrict__ env, int E) {
-  __shared__ float sc[64 * 35];
-  __shared__ float sv[64 * 3];
-  __shared__ float sd[64];
-  __shared__ int sz[2][64];
-  const int64_t eb = (int64_t)blockIdx.x * 64;
-  const int nv = (int)min((int64_t)64, (int64_t)E - eb);
+  __shared__ float sc[EPB * 35];
+  __shared__ float sv[EPB * 3];
+  __shared__ float sd[EPB];
+  __shared__ int sz[2][EPB];
+  const int64_t eb = (int64_t)blockIdx.x * EPB;
+  const int nv = (int)min((int64_t)EPB, (int64_t)E - eb);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   float ev[3] = {0.f, 0.f, 0.f};
   if (w == 0 && lane < nv) {
@@ -200,7 +206,11 @@ __global__ __launch_bounds__(256) void k_edge_geometry_fwd(
 // reads the edge's coefficient adjoints from LDS, where the block's rows (EPB x 35 contiguous
 // floats) arrive by coalesced loads issued before the sums, instead of 35 loads per thread that
 // each touch 64 cache lines.  EPB = 256 for graphs large enough to fill the GPU at one thread per
-// edge, 64 (the sums over all four waves, the VJP on one) for smaller ones.  Giving the VJP to
+// edge, 64 (the sums over all four waves, the VJP on one) for smaller ones, and 16 (one row sum
+// per 16-lane group) where that gives at most eight blocks per CU: the sums of a block run one
+// after the other, and the idle lanes of the VJP only cost once blocks wait for each other (64 ->
+// 16, us: 514 edges 15.1 -> 8.1, 7,680 17.9 -> 10.3, 24,000 23.4 -> 18.6, 32,000 21.7 -> 21.4,
+// 48,000 25.6 -> 30.0).  Giving the VJP to
 // one wave while the other three form the sums measured slower (46 vs 40 us at E = 61,440): the
 // sums, not the VJP, bound the kernel.
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -248,7 +258,7 @@ __global__ __launch_bounds__(256) void k_edge_geometry_bwd(
     const float* __restrict__ g_gauss, int64_t ldg, const float* __restrict__ off, float coeff,
     float cutoff, int nb, const float* __restrict__ jd, float gamma, float* __restrict__ g_ev,
     int E) {
-  static_assert(EPB == 64 || EPB == 256, "64 or 256 edges per block");
+  static_assert(EPB == 16 || EPB == 64 || EPB == 256, "16, 64 or 256 edges per block");
   __shared__ float sgd[EPB];
   __shared__ float sgc[EPB * 35];  // odd row stride: conflict-free per-thread rows
   const int64_t eb = (int64_t)blockIdx.x * EPB;
@@ -358,13 +368,15 @@ __global__ __launch_bounds__(256) void k_virial_partial(const float* __restrict_
   }
 }
 
-__global__ __launch_bounds__(64) void k_virial_final(const float* __restrict__ part, int nb,
-                                                     float* __restrict__ out) {
-  const int i = threadIdx.x;
-  if (i >= 9) return;
+// One wavefront per component.  (One lane per component added the blocks' partials one after the
+// other, 256 loads long: 26.6 us.)
+__global__ __launch_bounds__(9 * 64) void k_virial_final(const float* __restrict__ part, int nb,
+                                                         float* __restrict__ out) {
+  const int i = threadIdx.x >> 6, lane = threadIdx.x & 63;
   float s = 0.f;
-  for (int b = 0; b < nb; ++b) s += part[b * 9 + i];
-  out[i] = s;
+  for (int b = lane; b < nb; b += 64) s += part[b * 9 + i];
+  s = tta_group_sum(s, 64);
+  if (lane == 0) out[i] = s;
 }
 
 }  // namespace
@@ -471,9 +483,15 @@ extern "C" int tta_edge_geometry_fwd(const float* pos, const int* src, const int
     return tta_edge_features(dist, zsrc, ztgt, src_emb, tgt_emb, offsets, coeff, cutoff, nb, ec,
                              x_edge, env, E, stream);
   }
-  hipLaunchKernelGGL(k_edge_geometry_fwd, dim3(tta_blocks(E, 64)), dim3(256), 0, stream, pos, src,
-                     tgt, shift, jd, gamma, zsrc, ztgt, src_emb, tgt_emb, offsets, coeff, cutoff,
-                     (int)nb, (int)ec, ev, dist, coef, x_edge, env, (int)E);
+  auto launch = [&](auto kern, int epb) {
+    hipLaunchKernelGGL(kern, dim3(tta_blocks(E, epb)), dim3(256), 0, stream, pos, src, tgt, shift,
+                       jd, gamma, zsrc, ztgt, src_emb, tgt_emb, offsets, coeff, cutoff, (int)nb,
+                       (int)ec, ev, dist, coef, x_edge, env, (int)E);
+  };
+  if (E <= 16 * 24 * 256)
+    launch(k_edge_geometry_fwd<16>, 16);
+  else
+    launch(k_edge_geometry_fwd<64>, 64);
   TTA_CHECK_LAUNCH("tta_edge_geometry_fwd");
   return tta::kOk;
 }
@@ -488,7 +506,7 @@ extern "C" int tta_edge_geometry_bwd(const float* ev, const float* dist, const f
   TTA_CHECK_ARG(ev && dist && jd && g_ev, "tta_edge_geometry_bwd: null pointer");
   TTA_CHECK_ARG(!g_gauss || (offsets && ldg >= nb), "tta_edge_geometry_bwd: bad gaussian adjoint");
   // 256 edges per block (a full thread per edge in phase 2) once there are enough blocks to fill
-  // the GPU; small graphs take 64 per block for four times the blocks
+  // the GPU; smaller graphs take 64 or 16 per block for as many more blocks
   const bool v4 = g_gauss && nb % 4 == 0 && ldg % 4 == 0 && (uintptr_t)g_gauss % 16 == 0 &&
                   (uintptr_t)offsets % 16 == 0;
   const bool wide = E >= 256 * 512;
@@ -497,7 +515,9 @@ extern "C" int tta_edge_geometry_bwd(const float* ev, const float* dist, const f
                        g_env, g_gauss, ldg, offsets, coeff, cutoff, (int)nb, jd, gamma, g_ev,
                        (int)E);
   };
-  if (wide)
+  if (E <= 16 * 8 * 256)
+    v4 ? launch(k_edge_geometry_bwd<16, true>, 16) : launch(k_edge_geometry_bwd<16, false>, 16);
+  else if (wide)
     v4 ? launch(k_edge_geometry_bwd<256, true>, 256) : launch(k_edge_geometry_bwd<256, false>, 256);
   else
     v4 ? launch(k_edge_geometry_bwd<64, true>, 64) : launch(k_edge_geometry_bwd<64, false>, 64);
@@ -525,7 +545,7 @@ extern "C" int tta_virial(const float* ev, const float* g_ev, int64_t E, float* 
   TTA_CHECK_ARG(work && out && ((ev && g_ev) || E == 0), "tta_virial: null pointer");
   hipLaunchKernelGGL(k_virial_partial, dim3(kVirBlocks), dim3(256), 0, stream, ev, g_ev, (int)E,
                      work);
-  hipLaunchKernelGGL(k_virial_final, dim3(1), dim3(64), 0, stream, work, kVirBlocks, out);
+  hipLaunchKernelGGL(k_virial_final, dim3(1), dim3(9 * 64), 0, stream, work, kVirBlocks, out);
   TTA_CHECK_LAUNCH("tta_virial");
   return tta::kOk;
 }
@@ -543,7 +563,7 @@ extern "C" int tta_virial_noalloc(const float* ev, const float* g_ev, int64_t E,
   if (st != tta::kOk) return st;
   hipLaunchKernelGGL(k_virial_partial, dim3(kVirBlocks), dim3(256), 0, stream, ev, g_ev, (int)E,
                      part);
-  hipLaunchKernelGGL(k_virial_final, dim3(1), dim3(64), 0, stream, part, kVirBlocks, out);
+  hipLaunchKernelGGL(k_virial_final, dim3(1), dim3(9 * 64), 0, stream, part, kVirBlocks, out);
   TTA_CHECK_LAUNCH("tta_virial_noalloc");
   return tta::kOk;
 }

@@ -369,9 +369,10 @@ __global__ __launch_bounds__(256) void k_rmsnorm_sh_fwd(const float* __restrict_
 }
 
 // Register-resident form of the RMSNormSH backward for C <= 64 NPL: each lane loads its NPL
-// channels of all 9 coefficient rows of g and x (and of the 3 degree weights) once and every pass
-// works from registers, so a node costs one memory round trip instead of one per pass (C3: 15 vs
-// 26 us per launch).  The sums run in the same order as the loop form (channel blocks k = 0.. in
+// channels of all 9 coefficient rows of g, x and the residual (and of the 3 degree weights) once
+// and every pass works from registers, so a node costs one memory round trip instead of one per
+// pass (C3: 15 vs 26 us per launch; with the residual read in the last pass, a second round trip,
+// 24 nodes took 13.2 us, now 7.5).  The sums run in the same order as the loop form (channel blocks k = 0.. in
 // turn, coefficients inside).  The forward keeps its loop form, which measured faster (7.2 vs
 // 8.6 us): its re-reads of the row hit in cache.
 template <int NPL>
@@ -387,7 +388,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm_sh_bwd_r(const float* __restric
   if (n >= N) return;
   const float* xn = x + n * 9 * C;
   const float* gn = g + n * 9 * C;
-  float xv[9][NPL], gv[9][NPL], wv[3][NPL];
+  float xv[9][NPL], gv[9][NPL], rv[9][NPL], wv[3][NPL];
 #pragma unroll
   for (int k = 0; k < NPL; ++k) {
     const int c = lane + 64 * k;
@@ -396,6 +397,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm_sh_bwd_r(const float* __restric
     for (int j = 0; j < 9; ++j) {
       xv[j][k] = in ? xn[j * C + c] : 0.f;
       gv[j][k] = in ? gn[j * C + c] : 0.f;
+      rv[j][k] = in && res ? res[n * 9 * C + j * C + c] : 0.f;
     }
 #pragma unroll
     for (int l = 0; l < 3; ++l) wv[l][k] = in ? aw[l * C + c] : 0.f;
@@ -436,7 +438,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm_sh_bwd_r(const float* __restric
       const float v = j == 0 ? xv[0][k] - mu : xv[j][k];
       float gx = gv[j][k] * (inv * wv[deg_of(j)][k]) + v * bdw_of(j) * gms * (2.0f / C);
       if (j == 0) gx -= m0;
-      if (res) gx += res[n * 9 * C + j * C + c];
+      if (res) gx += rv[j][k];
       on[j * C + c] = gx;
     }
   }

@@ -981,7 +981,7 @@ def edge_geometry_bwd(ev, dist, g_coef, g_env, g_gauss, ldg, offsets, coeff, cut
     if g_gauss is not None and (ldg < nb or offsets is None or offsets.numel() < nb):
         raise RuntimeError("edge_geometry_bwd: g_gauss needs ldg >= nb and nb offsets")
     v4 = (g_gauss is not None and nb % 4 == 0 and ldg % 4 == 0 and _al16(g_gauss, offsets))
-    kern = f"k_edge_geometry_bwd<{256 if E >= 256 * 512 else 64},{_tf(v4)}>"
+    kern = f"k_edge_geometry_bwd<{256 if E >= 256 * 512 else 64 if E > 32768 else 16},{_tf(v4)}>"
     # per edge: ev, dist, g_coef, g_env, the Gaussian-adjoint row; out g_ev
     per = 12 + 4 + (140 if g_coef is not None else 0) + (4 if g_env is not None else 0) + \
         (4 * nb if g_gauss is not None else 0) + 12
