@@ -301,6 +301,34 @@ def test_wide_gemm(nat, M, N, K, epi):
         assert ((outs[0][1][rows].double() - silu).abs() / mag).max().item() < 2e-6
 
 
+@pytest.mark.parametrize("M,N,K,epi", [(30_011, 1024, 1024, 3), (30_011, 1000, 416, 4),
+                                       (12_000, 768, 640, 2), (20_000, 512, 384, 0),
+                                       (43_700, 256, 1024, 1)])
+def test_wide_gemm_reduced_precision(nat, M, N, K, epi):
+    """bf16 operands on the 128 x 256 tile (at most five rounds of workgroups for eight of the
+    128 x 128 kernel's): the same bits as column slices too narrow for it, which run on the
+    128 x 128 kernel, with ragged rows and columns, every kind of epilogue and rows of infinities
+    and NaN; every product in the same order there."""
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    A, B, bias, C0, aux = r(M, K), r(K, N) / math.sqrt(K), r(N), r(M, N), r(M, N)
+    A[130, 3], A[131, K - 1] = float("inf"), float("nan")
+    C, C2 = C0.clone(), torch.zeros(M, N, device=DEV)
+    nat.linear(A, nat.PackedWeight(B, nat.SPLIT_BF16), bias, out=C, epilogue=epi, out2=C2, aux=aux)
+    for c in range(0, N, 128):
+        s = slice(c, min(c + 128, N))
+        ref, ref2 = C0[:, s].contiguous(), torch.zeros(M, min(128, N - c), device=DEV)
+        nat.linear(A, nat.PackedWeight(B[:, s].contiguous(), nat.SPLIT_BF16),
+                   bias[s].contiguous(), out=ref, epilogue=epi, out2=ref2,
+                   aux=aux[:, s].contiguous())
+        assert torch.equal(C[:, s].nan_to_num(7.5), ref.nan_to_num(7.5))
+        assert torch.equal(C2[:, s].nan_to_num(7.5), ref2.nan_to_num(7.5))
+    rows = torch.arange(0, 128, device=DEV)
+    want = A[rows].bfloat16().double() @ B.bfloat16().double() + bias.double()
+    if epi == 0:
+        assert (C[rows].double() - want).abs().max() < K * 2.0 ** -23
+
+
 def test_gemm_batched_strided(nat):
     g = torch.Generator().manual_seed(5)
     N_, C, H = 50, 32, 24

@@ -6,9 +6,10 @@
 // eight column blocks instead of four and a step's copies bring 24 KB for as many instructions.
 // Two workgroups still share a compute unit, so that one's epilogue overlaps the other's k loop: a
 // stage holds a 16-wide k step (24 KB) and three stages take 72 KB.  Step s multiplies stage s while
-// it reads and splits the A rows of stage s + 1 and its copies fill stage s + 2 (the one that
-// step s - 1 left, after the barrier that retires it), so a copy has a whole step to land.  A last
-// column tile of 128 columns runs the same loop with four column blocks.
+// it reads and splits the A rows of stage s + 1 and its copies fill the stage that step s - 1 left
+// (after the barrier that retires it), so a copy has a whole step to land.  In mode 1 a stage is
+// 16 KB and a step a third as long: five stages, and a copy has three steps.  A last column tile of
+// 128 columns runs the same loop with four column blocks.
 #include "gemm_split.h"
 
 #include <algorithm>
@@ -35,7 +36,8 @@ __global__ __launch_bounds__(WTH, 2) void gemm_wide_kernel(GemmGroup g) {
   constexpr int A_CH = WM * 4, B_CH = NB * NT * 64, STG = A_CH + B_CH;  // 16-byte chunks
   constexpr int APT = A_CH / WTH, BPT = B_CH / WTH;
   constexpr int LDT = BN + 8;  // epilogue staging: 128 columns at a time
-  constexpr int SMEM = 3 * STG > WM * LDT / 4 ? 3 * STG : WM * LDT / 4;
+  constexpr int NST = MODE == 1 ? 5 : 3, NIF = APT + BPT;  // stages; copies per stage and thread
+  constexpr int SMEM = NST * STG > WM * LDT / 4 ? NST * STG : WM * LDT / 4;
   __shared__ uint4 smem[SMEM];
 
   const GemmArgs& p = g.p[blockIdx.z];
@@ -131,7 +133,8 @@ __global__ __launch_bounds__(WTH, 2) void gemm_wide_kernel(GemmGroup g) {
   // the k loop over the first TJ column blocks.  A pair's fragments are read one pair ahead (the first
   // pair of a step during the last of the step before: its stage landed a barrier earlier); the
   // scheduling barriers keep the reads there
-  auto next = [](int v) { return v == 2 ? 0 : v + 1; };
+  auto next = [](int v) { return v == NST - 1 ? 0 : v + 1; };
+  auto prev = [](int v) { return v == 0 ? NST - 1 : v - 1; };
   auto loop = [&](auto tj) {
     constexpr int TJ = decltype(tj)::value;
     floatx4 x[1][2];
@@ -147,8 +150,8 @@ __global__ __launch_bounds__(WTH, 2) void gemm_wide_kernel(GemmGroup g) {
     float big = 0.f;
     auto step = [&](auto fast) {
       const int s1 = next(stg);
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      issue(min(s + 2, nks - 1), next(s1));
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NST - 3) * NIF) : "memory");
+      issue(min(s + NST - 1, nks - 1), prev(stg));
       rdA(s1, x);
 #pragma unroll
       for (int j = 0; j < TJ; j += 2) {
@@ -203,9 +206,10 @@ __global__ __launch_bounds__(WTH, 2) void gemm_wide_kernel(GemmGroup g) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[0][j][r] = 0.f;
     rs = RowScale<1, NT, S::F16>();
-    issue(min(1, nks - 1), 1);
-    // stage 0 landed (with everything issued before it); stage 1 may still be in flight
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(APT + BPT) : "memory");
+#pragma unroll
+    for (int q = 1; q < NST - 1; ++q) issue(min(q, nks - 1), q);
+    // stage 0 landed (with everything issued before it); the later ones may still be in flight
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NST - 2) * NIF) : "memory");
     const bool whole = cn0 + BN < p.N;  // more than 128 columns in this tile
     if (whole)
       loop(std::integral_constant<int, NT>{});
@@ -271,22 +275,37 @@ __global__ __launch_bounds__(WTH, 2) void gemm_wide_kernel(GemmGroup g) {
 
 namespace tta_gemm {
 
-// Whether a launch takes the wide tile: mode 16, whole 32-wide k slabs, at least one whole column
-// tile per product, and enough work that the uneven last round of the larger tiles costs less than
-// the loop gains: 3072 k columns of tiles per resident workgroup.  Measured, 128 x 128 -> 128 x 256
-// (us): 196,555 x 1024 x 1024 with the SiLU-gradient epilogue (12,288 columns) 1427 -> 1336, with
-// the two-output epilogue 1460 -> 1374; x 1024 x 256 (3072) 557 -> 526; x 256 x 1024 (3072) 332 ->
-// 323; 61,440 rows, conv-1 group (3840) 470 -> 448, its adjoint (7470) 520 -> 500; below the line,
-// conv-2 group (1920) 243 -> 248, 640 x 768 (2160) 197 -> 199, 10,150 x 1024 x 1024 (640) 82 -> 95.
+// Whether a launch takes the wide tile: mode 16 or 1, whole 32-wide k slabs, at least one whole
+// column tile per product and, in mode 16, enough work that the uneven last round of the larger
+// tiles costs less than the loop gains: 3072 k columns of tiles per resident workgroup.  Measured,
+// 128 x 128 -> 128 x 256 (us): 196,555 x 1024 x 1024 with the SiLU-gradient epilogue (12,288
+// columns) 1427 -> 1336, with the two-output epilogue 1460 -> 1374; x 1024 x 256 (3072) 557 -> 526;
+// x 256 x 1024 (3072) 332 -> 323; 61,440 rows, conv-1 group (3840) 470 -> 448, its adjoint (7470)
+// 520 -> 500; below the line, conv-2 group (1920) 243 -> 248, 640 x 768 (2160) 197 -> 199, 10,150 x
+// 1024 x 1024 (640) 82 -> 95.
+//
+// Mode 1 has a third of the products per copied byte, so its gain hangs on whole rounds of
+// resident workgroups rather than on the work in all: it takes the wide tile where that makes
+// five rounds or fewer out of eight of the 128 x 128 kernel's, at an average K of at least 384.
+// Measured, 128 x 128 -> 128 x 256 (us): 30,011 x 1024 x 1024 (4 rounds -> 2) with the two-output
+// epilogue 119 -> 103, with the SiLU-gradient one 131 -> 119; 61,440 rows (8 -> 4), conv-1 group
+// 256 -> 222, its adjoint 341 -> 277; 12,000 x 768 x 640 (2 -> 1) 36 -> 30; below the line, 20,000
+// x 1024 x 512 (3 -> 2) 56 -> 60, 8,000 x 1024 x 1024 (1 -> 1) 36 -> 43, 30,011 x 256 x 1024
+// (1 -> 1) 34 -> 39, and 60,000 x 1024 at K = 256 / 128 (8 -> 4) 110 -> 116 / 96 -> 103.
 bool wide_ok(const GemmGroup& g, int n, int mode, int cap) {
-  if (mode != 16) return false;
-  int64_t cols = 0;
+  if (mode != 16 && mode != 1) return false;
+  int64_t cols = 0, wide = 0, tiles = 0;
   for (int i = 0; i < n; ++i) {
     const GemmArgs& p = g.p[i];
     if (p.K % BK != 0 || p.K < 2 * BK || p.N < WN) return false;
-    cols += (int64_t)tta_blocks(p.N, WN) * tta_blocks(p.M, WM) * p.K;
+    const int64_t rows = tta_blocks(p.M, WM), w = rows * tta_blocks(p.N, WN);
+    wide += w;
+    tiles += rows * tta_blocks(p.N, BN);
+    cols += w * p.K;
   }
-  return cols >= (int64_t)3072 * cap;
+  if (mode == 16) return cols >= (int64_t)3072 * cap;
+  const auto rounds = [&](int64_t c) { return (c + cap - 1) / cap; };
+  return cols >= 384 * wide && 5 * rounds(tiles) >= 8 * rounds(wide);
 }
 
 int launch_wide(GemmGroup& g, int n, int mode, int cap, hipStream_t s) {
@@ -300,8 +319,8 @@ int launch_wide(GemmGroup& g, int n, int mode, int cap, hipStream_t s) {
     }
     grid = std::max(grid, std::min<int64_t>(((ntiles + 7) / 8) * 8, g.cap));
   }
-  hipLaunchKernelGGL(gemm_wide_kernel<16>, dim3((unsigned)grid, 1, (unsigned)n), dim3(WTH), 0, s,
-                     g);
+  const auto kern = mode == 1 ? gemm_wide_kernel<1> : gemm_wide_kernel<16>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid, 1, (unsigned)n), dim3(WTH), 0, s, g);
   TTA_CHECK_LAUNCH("tta_gemm_bf16x");
   return tta::kOk;
 }
