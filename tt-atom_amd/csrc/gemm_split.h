@@ -154,7 +154,7 @@ __device__ __forceinline__ void epilogue_rows(const GemmArgs& p, const float* Ct
     constexpr int RB = 8;
     if (BATCH && full && (LOADS || gather) && rows % (RB * rstep) == 0) {
       // An epilogue that reads memory (the accumulated C, the SiLU argument, the gathered rows;
-      // BATCH: mode 16, whose register budget has room for it)
+      // BATCH: the callers whose register budget has room for it)
       // issues a batch of RB rows' loads -- the gather indices first, then the rows they name --
       // before it uses any, so their latencies overlap instead of adding up row by row.
 #pragma unroll 1

@@ -225,7 +225,10 @@ __global__ __launch_bounds__(WTH, 2) void gemm_wide_kernel(GemmGroup g) {
     float* Ct = reinterpret_cast<float*>(smem);
     const bool mfull = cm0 + WM <= p.M;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {  // 128 columns at a time
+    for (int h = 0; h < 2; ++h) {
+      // 128 columns at a time, the rows' loads batched in mode 1 too (232 registers: 30,011 x 1024 x
+      // 1024 with the SiLU-gradient epilogue 113 -> 102 us, 60,000 rows 293 -> 243; the 128 x 128
+      // kernel in mode 1 loses 3-8 % on its other epilogues with the registers that takes)
       if (h == 1 && !whole) break;
 #pragma unroll
       for (int j = 0; j < NT / 2; ++j)
@@ -237,30 +240,30 @@ __global__ __launch_bounds__(WTH, 2) void gemm_wide_kernel(GemmGroup g) {
       const bool full = mfull && c0 + BN <= p.N;
       switch (p.epi) {
         case EPI_SILU:
-          epilogue_rows<EPI_SILU, S::F16>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full);
+          epilogue_rows<EPI_SILU, true>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full);
           break;
         case EPI_ACCUM:
-          epilogue_rows<EPI_ACCUM, S::F16>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full);
+          epilogue_rows<EPI_ACCUM, true>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full);
           break;
         case EPI_PRE_SILU:
-          epilogue_rows<EPI_PRE_SILU, S::F16>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full);
+          epilogue_rows<EPI_PRE_SILU, true>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full);
           break;
         case EPI_SILU_GRAD:
-          epilogue_rows<EPI_SILU_GRAD, S::F16>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full);
+          epilogue_rows<EPI_SILU_GRAD, true>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full);
           break;
         case EPI_SIGMOID:
-          epilogue_rows<EPI_SIGMOID, S::F16>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full);
+          epilogue_rows<EPI_SIGMOID, true>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full);
           break;
         case EPI_GATE:
-          epilogue_rows<EPI_GATE, S::F16>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full, &g.gate,
+          epilogue_rows<EPI_GATE, true>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full, &g.gate,
                                           g.gc0[blockIdx.z]);
           break;
         case EPI_GATE_BWD:
-          epilogue_rows<EPI_GATE_BWD, S::F16>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full,
+          epilogue_rows<EPI_GATE_BWD, true>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full,
                                               &g.gate, g.gc0[blockIdx.z]);
           break;
         default:
-          epilogue_rows<EPI_STORE, S::F16>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full);
+          epilogue_rows<EPI_STORE, true>(p, Ct, LDT, WM, cm0, c0, t, WTH, vec_ok, full);
       }
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
@@ -288,7 +291,7 @@ namespace tta_gemm {
 // resident workgroups rather than on the work in all: it takes the wide tile where that makes
 // five rounds or fewer out of eight of the 128 x 128 kernel's, at an average K of at least 384.
 // Measured, 128 x 128 -> 128 x 256 (us): 30,011 x 1024 x 1024 (4 rounds -> 2) with the two-output
-// epilogue 119 -> 103, with the SiLU-gradient one 131 -> 119; 61,440 rows (8 -> 4), conv-1 group
+// epilogue 119 -> 103, with the SiLU-gradient one 131 -> 102; 61,440 rows (8 -> 4), conv-1 group
 // 256 -> 222, its adjoint 341 -> 277; 12,000 x 768 x 640 (2 -> 1) 36 -> 30; below the line, 20,000
 // x 1024 x 512 (3 -> 2) 56 -> 60, 8,000 x 1024 x 1024 (1 -> 1) 36 -> 43, 30,011 x 256 x 1024
 // (1 -> 1) 34 -> 39, and 60,000 x 1024 at K = 256 / 128 (8 -> 4) 110 -> 116 / 96 -> 103.
