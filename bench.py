@@ -51,13 +51,14 @@ PEAK_BF16_MFMA = 2500.0
 PEAKS = {"f32": PEAK_FP32_MFMA, "f16x3": PEAK_BF16_MFMA / 3, "f16x3-panel": PEAK_BF16_MFMA / 3,
          "bf16x6": PEAK_BF16_MFMA / 6, "bf16x3": PEAK_BF16_MFMA / 3, "bf16x1": PEAK_BF16_MFMA}
 KERNELS = {"f32": "gemm_f32_kernel (fp32 MFMA 16x16x4)",
-           "f16x3": "gemm_bf16x_kernel<2,16> (split-fp16, 2x2 power-of-two-scaled planes / 3 "
-                    "products, fp32-accurate)",
+           "f16x3": "gemm_wide_kernel<16> / gemm_bf16x_kernel<2,16> / gemm_small_kernel<16,..> by "
+                    "launch size (split-fp16, 2x2 power-of-two-scaled planes / 3 products, "
+                    "fp32-accurate)",
            "f16x3-panel": "gemm_f16x3_panel<KT,2> (the same split-fp16 arithmetic for K <= 128: "
                           "the radial output layer)",
            "bf16x6": "gemm_bf16x_kernel<2,6> (split-bf16, 3x3 planes / 6 products, fp32-accurate)",
            "bf16x3": "gemm_bf16x_kernel<2,3> (split-bf16, 2x2 planes / 3 products)",
-           "bf16x1": "gemm_bf16x_kernel<2,1> (bf16 operands)"}
+           "bf16x1": "gemm_wide_kernel<1> / gemm_bf16x_kernel<2,1> by launch size (bf16 operands)"}
 # rocprofv3 counter summary of the C3 step (per-kernel HBM bytes and MFMA counters), written by
 # ``bench.py --summarize-counters`` from the profiler's CSV output; read to report counter-measured
 # HBM bytes next to the algorithmic ones.
@@ -554,6 +555,12 @@ def _read_pmc(d):
     return rows
 
 
+def _family(variant):
+    """The split-fp16 GEMM family's kernels count together (as the launches timed there do)."""
+    return variant in ("gemm_bf16x_kernel<2,16>", "gemm_wide_kernel<16>") or \
+        variant.startswith("gemm_small_kernel<16,")
+
+
 def summarize_counters(root, out_path, workload="c3"):
     """Per-kernel HBM bytes and MFMA counters of a profiled step (C3 or C5).
 
@@ -573,7 +580,7 @@ def summarize_counters(root, out_path, workload="c3"):
     for c in ("FETCH_SIZE", "WRITE_SIZE"):
         for e in _read_pmc(root / f"step_{c}").values():
             v, b = _kernel_names(e["kernel"])
-            for k in {v, b}:
+            for k in {v, b} | ({"gemm_f16x3"} if _family(v) else set()):
                 d = per.setdefault(k, {"FETCH_SIZE": [], "WRITE_SIZE": [], "variant": k == v})
                 d[c].append(e["c"].get(c, 0.0))
     mf = {}
@@ -581,11 +588,12 @@ def summarize_counters(root, out_path, workload="c3"):
     if mdir.exists():
         for e in _read_pmc(mdir).values():
             v, _ = _kernel_names(e["kernel"])
-            d = mf.setdefault(v, {"util": [], "flops": [], "ns": []})
-            d["util"].append(e["c"].get("MfmaUtil", 0.0))
-            d["flops"].append(sum(e["c"].get(c, 0.0) for c in
-                                  ("MfmaFlopsF16", "MfmaFlopsBF16", "MfmaFlopsF32")))
-            d["ns"].append(e["ns"])
+            for k in {v} | ({"gemm_f16x3"} if _family(v) else set()):
+                d = mf.setdefault(k, {"util": [], "flops": [], "ns": []})
+                d["util"].append(e["c"].get("MfmaUtil", 0.0))
+                d["flops"].append(sum(e["c"].get(c, 0.0) for c in
+                                      ("MfmaFlopsF16", "MfmaFlopsBF16", "MfmaFlopsF32")))
+                d["ns"].append(e["ns"])
     lines = [f"# rocprofv3 counters of the {COUNTER_TITLES[workload]}, MI355X",
              "# Commands (repository root $REPO on the GPU box; one pass per counter group):",
              "#   cd /tmp && export TMPDIR=/tmp"]
@@ -894,7 +902,7 @@ def main():
     achieved = d["flops"] / (d["ms"] * 1e-3) / 1e12 if d["ms"] > 0 else 0.0
     counted = wl in COUNTER_FILES and args.precision == "f32"
     kernel_traffic, kernel_mfma = read_traffic(COUNTER_FILES[wl]) if counted else ({}, {})
-    dom_kernel = {"f16x3": "gemm_bf16x_kernel<2,16>"}.get(dom)
+    dom_kernel = {"f16x3": "gemm_f16x3"}.get(dom)
     traffic = kernel_traffic.get(dom_kernel) if dom_kernel else None
     mfma_counters = kernel_mfma.get(dom_kernel) if dom_kernel else None
     ms_step = dt / args.steps * 1e3
@@ -967,7 +975,7 @@ def main():
                                    "dense MFMA 2500 / number of plane products"),
                      "frac_note": ("the default split (f16x3: 3 fp16 products per fp32 "
                                    "product); the peak assumes the 2.4 GHz clock, which the part "
-                                   "does not hold under this load, and each 128 x 128 tile ends "
+                                   "does not hold under this load, and each output tile ends "
                                    "in an epilogue that writes 64 KB (13-35 % of a tile's time "
                                    "on these shapes); the fp32-accurate bf16x6 mode reads a "
                                    "higher frac (0.43-0.44 of its /6 ceiling) at a lower rate "
