@@ -1349,3 +1349,22 @@ def test_activation_accuracy(nat, packed):
     torch.testing.assert_close(sp[0], torch.tensor([1.0, 0.0, nan, 1.0, 0.0]), equal_nan=True)
     torch.testing.assert_close(sp[1], torch.tensor([inf, nan, nan, 3e38, 0.0]), equal_nan=True)
     torch.testing.assert_close(sp[2], torch.tensor([nan, nan, nan, 1.0, 0.0]), equal_nan=True)
+
+
+@pytest.mark.parametrize("packed", [False, True])
+def test_activation_negative_tail(nat, packed):
+    """Sigmoid and SiLU of large negative arguments, down to where exp(-x) overflows (x = -88.72):
+    the SiLU is a normal number there (5e-37 and above), the sigmoid a denormal one below x = -87.3.
+    expf to 1 ulp, 1 + e and the divide to half an ulp each, the product to another: 5 half ulps,
+    3e-7 of the value, plus half the denormal spacing 2^-149 (times |x| in the SiLU)."""
+    x = torch.linspace(-88.7, -20, 4096)
+    M, K = (4096, 128) if packed else (3, 64)
+    w = torch.zeros(K, len(x), device=DEV)
+    w = nat.PackedWeight(w, nat.SPLIT_F16X3) if packed else w
+    A = torch.zeros(M, K, device=DEV)
+    sig, silu = (nat.linear(A, w, x.to(DEV), epilogue=e)[M - 1].cpu().double()
+                 for e in (nat.EPI_SIGMOID, nat.EPI_SILU))
+    xd = x.double()
+    s, tiny = torch.sigmoid(xd), 2.0 ** -150
+    assert ((sig - s).abs() <= 3e-7 * s + tiny).all()
+    assert ((silu - xd * s).abs() <= 3e-7 * (xd * s).abs() + tiny * xd.abs()).all()

@@ -42,44 +42,14 @@ enum Status : int {
 // ---------------------------------------------------------------------------- device helpers
 __device__ __forceinline__ float tta_sigmoid(float x) { return 1.0f / (1.0f + __expf(-x)); }
 
-// Sigmoid and SiLU for the force path, whose parity tolerance is tight, in a third fewer
-// vector instructions (26 for 38) than 1 / (1 + expf(-x)) with a divide takes: the epilogues of the hidden-layer products
-// evaluate them per output, and their vector instructions were as many as the k loop's.  With
-// e = exp(-|x|) in (0, 1] nothing overflows and sigmoid(x) = (x < 0 ? e : 1) / (1 + e).  e is the
-// hardware's 2^p at p = -|x| log2(e), times 1 + the rounding error of p (two fused steps; NaN at
-// infinite x, where the fminf keeps it harmless), and the quotient n r with the hardware
-// reciprocal r gets one correction step by its own residual.  SiLU puts x into the numerator, one
-// rounding fewer than x sigmoid(x).  Relative 2-norm error against fp64 over x ~ N(0, 1) / N(0, 3)
-// / U(-20, 20), previous form -> this one: sigmoid 3.89e-8 / 3.79e-8 / 3.45e-8 -> 3.79e-8 /
-// 3.78e-8 / 3.45e-8, SiLU 4.48e-8 / 4.57e-8 / 3.35e-8 -> 4.05e-8 / 4.21e-8 / 3.31e-8, its
-// derivative 4.68e-8 / 9.33e-8 / 3.20e-7 -> 4.59e-8 / 9.32e-8 / 3.20e-7.  (U(-80, 0), which no
-// activation here reaches: SiLU 4.75e-8 -> 5.58e-8, the other two lower.  Below x = -87.3 the
-// results are zero; the sigmoid there is denormal.)  Measured (us): 196,555 x 1024 x 1024 with
-// the SiLU-gradient epilogue 1336 -> 1326, with the two-output one 1374 -> 1360; an Orb layer of
-// 30,011 edges 2805 -> 2671, its reduced-precision edge encoder 650 -> 617.
-__device__ __forceinline__ void tta_exp_parts(float x, float& e, float& d, float& r) {
-  const float a = fabsf(x), log2e = 1.44269502f;
-  const float p = -a * log2e;
-  float c = fmaf(-a, log2e, -p);       // rounding error of p,
-  c = fmaf(-a, 1.92596299e-8f, c);     // and of log2e
-  c = fminf(c * 0.693147182f, 1e-4f);
-  e = __builtin_amdgcn_exp2f(p);
-  e = fmaf(e, c, e);
-  d = 1.0f + e;
-  r = __builtin_amdgcn_rcpf(d);
-}
-__device__ __forceinline__ float tta_sigmoid_acc(float x) {
-  float e, d, r;
-  tta_exp_parts(x, e, d, r);
-  const float n = x < 0.f ? e : 1.0f, q = n * r;
-  return fmaf(fmaf(-d, q, n), r, q);
-}
-__device__ __forceinline__ float tta_silu(float x) {
-  float e, d, r;
-  tta_exp_parts(x, e, d, r);
-  const float n = x < 0.f ? x * e : x, q = n * r;
-  return fmaf(fminf(fmaf(-d, q, n), 3e38f), r, q);  // (fminf: the residual of x = inf is NaN)
-}
+// Sigmoid and SiLU with an accurate exp: the parity tolerance of the force path is tight, so the
+// transcendental functions use the full-precision library versions (expf, not __expf) and the
+// divide is correctly rounded.  (exp(-|x|) from the hardware's 2^p with a corrected reciprocal takes
+// 26 vector instructions for these 38 and gains 2-4 % of an Orb layer or encoder step, but over
+// U(-80, 0) its SiLU is further off (relative 2-norm error 5.58e-8 against 4.75e-8), and it flushes
+// SiLU's normal values below x = -87.3 to zero.)
+__device__ __forceinline__ float tta_sigmoid_acc(float x) { return 1.0f / (1.0f + expf(-x)); }
+__device__ __forceinline__ float tta_silu(float x) { return x * tta_sigmoid_acc(x); }
 // d silu / dx = s (1 + x (1 - s))
 __device__ __forceinline__ float tta_silu_grad(float x) {
   float s = tta_sigmoid_acc(x);
