@@ -256,6 +256,37 @@ def test_small_launch_gemm(nat, mode, M, N, K):
     assert ((outs[0].double() - ref).abs() / mag).max().item() < 4 * 2.0 ** -bits
 
 
+@pytest.mark.parametrize("M,N,K,modes", [(72, 1024, 1024, (16, 6, 3, 1)), (4, 64, 128, (16, 1)),
+                                         (1205, 256, 1024, (16, 1)), (2500, 1024, 1024, (16, 6)),
+                                         (4095, 1536, 128, (16, 1)), (576, 1024, 1024, (3, 1))])
+def test_small_products_keep_fp32_operands(nat, M, N, K, modes):
+    """Products of packed weights below 4096 rows that the fp32 kernel runs (few tiles, many, short
+    K; any with reduced-mode weights): the bits of the plain weight, with rows that hold an
+    infinity, a NaN and values 2^40 apart, as one product, in a group and with the row-gather term."""
+    g = torch.Generator().manual_seed(M + N + K)
+    r = lambda *s: torch.randn(*s, generator=g)
+    x, w = r(M, K), (r(K, N) / math.sqrt(K)).to(DEV)
+    x[0, 5], x[1, 7], x[2, K - 1] = float("inf"), float("-inf"), float("nan")
+    x[3, :K // 2] *= 2.0 ** 20
+    x[3, K // 2:] *= 2.0 ** -20
+    x, b, P = x.to(DEV), r(N).to(DEV), r(5, 2 * N).to(DEV)
+    i0, i1 = (torch.randint(5, (M,), generator=g).to(DEV, torch.int32) for _ in range(2))
+    k = min(M - 1, 20)
+
+    def results(wt):
+        one = nat.linear(x, wt, b)
+        two = [torch.empty_like(one) for _ in range(2)]
+        nat.linear_group([(x, wt, b, two[0]), (x[:k], wt, None, two[1][:k])])
+        gat = nat.linear_gather(x, wt, b, torch.empty_like(one), P, i0, i1, N)
+        return [t.nan_to_num(7.5, 8.5, 9.5) for t in (one, two[0], two[1][:k], gat)]
+
+    ref = results(w)
+    assert (ref[0][0] == 8.5).any() and (ref[0][0] == 9.5).any() and not (ref[0][:2] == 7.5).any()
+    for mode in modes:
+        for got, want in zip(results(nat.PackedWeight(w, mode)), ref):
+            assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("M,N,K,epi", [(131_073, 260, 1024, 0), (132_000, 640, 512, 4),
                                        (100_001, 512, 1056, 3), (262_200, 256, 768, 2),
                                        (66_000, 1000, 1024, 1)])

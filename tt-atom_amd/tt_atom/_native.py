@@ -294,14 +294,13 @@ SPLIT_F32, SPLIT_F16X3, SPLIT_3, SPLIT_BF16 = 6, 16, 3, 1
 MODE_KIND = {6: "bf16x6", 16: "f16x3", 3: "bf16x3", 1: "bf16x1"}
 # mode-16 products that tta_gemm_bf16x(_group) runs on its short-K panel kernel (K <= 128, one
 # 32-wide k-slab count for the whole group, plain or SiLU epilogue, no row gathers, at least 128
-# columns, 16-byte aligned rows and operands, ldc < 2^22; launches of fewer than 4096 rows are
-# filed with the rest) are reported as their own family
+# columns, 16-byte aligned rows and operands, ldc < 2^22) are reported as their own family
 PANEL_KIND = "f16x3-panel"
 
 
-def _panel_item(M, N, K, ldc, epilogue, ptrs, gather=False):
+def _panel_item(N, K, ldc, epilogue, ptrs, gather=False):
     al = all(q is None or q % 16 == 0 for q in ptrs)
-    return (M >= 4096 and K <= 128 and epilogue in (EPI_STORE, EPI_SILU) and not gather and N >= 128
+    return (K <= 128 and epilogue in (EPI_STORE, EPI_SILU) and not gather and N >= 128
             and N % 4 == 0 and ldc % 4 == 0 and ldc < (1 << 22) and al)
 
 
@@ -309,32 +308,21 @@ class PackedWeight:
     """A constant GEMM operand w_t [K, N] (fp32, row-major) plus its bf16-plane packing for the
     split kernel (``mode`` 6, 16, 3 or 1; None keeps only the fp32 matrix for the fp32-MFMA
     kernel).  ``shape`` / ``T``-free: it stands wherever a [K, N] weight is passed to linear().
-    The reduced modes (1, 3) apply to products of at least 4096 rows; below that a product is
-    fp32-accurate, so those weights are packed for mode 16 as well."""
+    The reduced modes (1, 3) apply to products of at least 4096 rows; below that linear() and
+    linear_group() run their weights in fp32."""
 
     def __init__(self, w_t, mode=SPLIT_F32):
         if w_t.dim() != 2 or w_t.dtype != torch.float32 or not w_t.is_cuda:
             raise RuntimeError("PackedWeight: w_t must be a 2-D fp32 device tensor")
         self.w_t = w_t
         self.mode = mode
-        self.packed = self._pack(mode)
-        self._packed_few = self._pack(SPLIT_F16X3) if mode in (SPLIT_3, SPLIT_BF16) else None
-
-    def _pack(self, mode):
-        K, N = self.w_t.shape
-        if mode is None or K % 4:
-            return None
-        n = load().tta_pack_b_elems(K, N, mode)
-        packed = torch.empty(n, dtype=torch.int16, device=self.w_t.device)
-        _call("tta_pack_b", _ptr(self.w_t, name="w_t", contiguous=False), K, N,
-              _ld(self.w_t, "w_t"), mode, packed.data_ptr(), n, _stream())
-        return packed
-
-    def planes(self, M):
-        """(packed planes, mode) of a product of M rows."""
-        if self._packed_few is not None and M < 4096:
-            return self._packed_few, SPLIT_F16X3
-        return self.packed, self.mode
+        self.packed = None
+        K, N = w_t.shape
+        if mode is not None and K % 4 == 0:
+            n = load().tta_pack_b_elems(K, N, mode)
+            self.packed = torch.empty(n, dtype=torch.int16, device=w_t.device)
+            _call("tta_pack_b", _ptr(w_t, name="w_t", contiguous=False), K, N, _ld(w_t, "w_t"),
+                  mode, self.packed.data_ptr(), n, _stream())
 
     @property
     def shape(self):
@@ -353,7 +341,7 @@ def _same_rows(out, out2, aux, where):
 def _gemm_bf16x(x, pw, out, bias, epilogue, out2, aux, P=None, idx0=None, idx1=None, off1=0):
     M, K = x.shape
     N = pw.w_t.shape[1]
-    packed, mode = pw.planes(M)
+    mode = pw.mode
     ldx, ldc = _ld(x, "x"), _same_rows(out, out2, aux, "linear")
     _span(x, "x", M, ldx, K)
     for t, nm in ((out, "out"), (out2, "out2"), (aux, "aux")):
@@ -362,11 +350,11 @@ def _gemm_bf16x(x, pw, out, bias, epilogue, out2, aux, P=None, idx0=None, idx1=N
     if probe is not None:
         c_passes = 1 + (epilogue in (EPI_ACCUM, EPI_PRE_SILU, EPI_SILU_GRAD)) + (2 if P is not None else 0)
         panel = mode == 16 and _panel_item(
-            M, N, K, ldc, epilogue,
+            N, K, ldc, epilogue,
             [out.data_ptr(), None if bias is None else bias.data_ptr()], gather=P is not None)
         probe.before(2.0 * M * N * K, 4.0 * (M * K + K * N + c_passes * M * N),
                      PANEL_KIND if panel else MODE_KIND[mode])
-    _call("tta_gemm_bf16x", x.data_ptr(), packed.data_ptr(), out.data_ptr(),
+    _call("tta_gemm_bf16x", x.data_ptr(), pw.packed.data_ptr(), out.data_ptr(),
           None if bias is None else _ptr(bias, numel=N, name="bias"),
           None if out2 is None else out2.data_ptr(), None if aux is None else aux.data_ptr(),
           M, N, K, ldx, ldc, mode,
@@ -377,14 +365,31 @@ def _gemm_bf16x(x, pw, out, bias, epilogue, out2, aux, P=None, idx0=None, idx1=N
         probe.after()
 
 
-def _split_ok(x, pw):
-    """Whether a product runs on the split kernels (packed weight, 16-byte aligned rows); short-K
-    products and the unpacked weights of the heads stay on the fp32 MFMA kernel.  The library
-    chooses the tile by the launch's size (128 x 128, or the small-launch kernel's)."""
+def _split_ok(x, pw, min_rows=4096):
+    """Whether a product runs on the split kernels (packed weight, 16-byte aligned rows): from 4096
+    rows on, and below that where ``_small_split`` says so.  The other products (short K, few
+    rows, the unpacked weights of the heads) keep fp32 operands on the fp32 MFMA kernel."""
     M, K = x.shape
-    return (isinstance(pw, PackedWeight) and pw.packed is not None and M > 0
+    return (isinstance(pw, PackedWeight) and pw.packed is not None and M >= min_rows
             and K >= 128 and K % 4 == 0 and x.data_ptr() % 16 == 0
             and (ld := _ld(x, "x")) % 4 == 0 and ld < (1 << 21))
+
+
+def _tiles(items, rows, cols):
+    return sum(-(-x.shape[0] // rows) * -(-w.shape[1] // cols) for x, w, *_ in items)
+
+
+def _small_split(items):
+    """Whether the products items = [(x, w, ...)] of one launch, all with fewer than 4096 rows, run
+    on the split kernels: K >= 256, weights packed for one fp32-accurate mode (16 or 6), 160 or
+    more of the fp32 kernel's 32 x 64 tiles in all (which it would run unsplit at its matrix rate;
+    its split-K form takes smaller launches) and fewer than 128 tiles of 128 x 128.  The others
+    stay on the fp32 kernel: two fp16 planes hold 22 of an operand's 24 bits and turn an infinite
+    element's output row into NaN."""
+    return (all(isinstance(w, PackedWeight) and w.mode in (SPLIT_F32, SPLIT_F16X3)
+                and w.mode == items[0][1].mode and x.shape[0] < 4096 and x.shape[1] >= 256
+                and _split_ok(x, w, min_rows=1) for x, w, *_ in items)
+            and _tiles(items, 32, 64) >= 160 and _tiles(items, 128, 128) < 128)
 
 
 def linear_group_gate(items, c0, sig, x0, idx8, H, backward=False):
@@ -400,12 +405,12 @@ def linear_group_gate(items, c0, sig, x0, idx8, H, backward=False):
     M = items[0][0].shape[0]
     if not isinstance(items[0][1], PackedWeight):
         raise RuntimeError("linear_group_gate: every product needs a packed weight")
-    mode = items[0][1].planes(M)[1]
+    mode = items[0][1].mode
     probs = (GemmProblem * len(items))()
     flops = nbytes = 0.0
     L = max(_host_idx8(idx8)) + 1
     for i, (x, w, bias, out) in enumerate(items):
-        if not (isinstance(w, PackedWeight) and w.packed is not None and w.planes(M)[1] == mode
+        if not (isinstance(w, PackedWeight) and w.packed is not None and w.mode == mode
                 and x.shape[1] % 4 == 0 and x.data_ptr() % 16 == 0 and _ld(x, "x") % 4 == 0
                 and _ld(x, "x") < (1 << 21)):
             raise RuntimeError("linear_group_gate: every product needs a packed weight of one "
@@ -415,7 +420,7 @@ def linear_group_gate(items, c0, sig, x0, idx8, H, backward=False):
         if Mi != M or K != w.shape[0] or out.shape != (M, N) or N % H:
             raise RuntimeError("linear_group_gate: shape mismatch")
         ldc = _ld(out, "out")
-        probs[i] = GemmProblem(_rows(x, M, _ld(x, "x"), K, "x"), w.planes(M)[0].data_ptr(),
+        probs[i] = GemmProblem(_rows(x, M, _ld(x, "x"), K, "x"), w.packed.data_ptr(),
                                _rows(out, M, ldc, N, "out"),
                                None if bias is None else _ptr(bias, numel=N, name="bias"),
                                None, None, M, N, K, _ld(x, "x"), 0, ldc,
@@ -483,7 +488,7 @@ def linear(x, w_t, bias=None, out=None, epilogue=EPI_STORE, out2=None, aux=None)
     if out is None:
         out = torch.empty(M, N, device=x.device, dtype=torch.float32)
     if isinstance(w_t, PackedWeight):
-        if _split_ok(x, w_t):
+        if _split_ok(x, w_t) or _small_split([(x, w_t)]):
             _gemm_bf16x(x, w_t, out, bias, epilogue, out2, aux)
             return out
         w_t = w_t.w_t
@@ -509,11 +514,13 @@ def linear_group(items):
             raise RuntimeError("linear_group: shape mismatch")
         _same_rows(out, out2, aux, "linear_group")
     split = [isinstance(w, PackedWeight) and _split_ok(x, w) for x, w, *_ in items]
-    modes = {w.planes(x.shape[0])[1] for (x, w, *_), sp in zip(items, split) if sp}
+    modes = {w.mode for (x, w, *_), sp in zip(items, split) if sp}
     if len(items) > MAX_GROUP or (any(split) and not all(split)) or len(modes) > 1:
         for x, w, bias, out, epi, out2, aux in items:
             linear(x, w, bias, out, epi, out2, aux)
         return
+    if not split[0] and _small_split(items):
+        split, modes = [True] * len(items), {items[0][1].mode}
     if not split[0] and any(x.shape[1] >= 256 for x, *_ in items) and _gemm_f32_splitk(
             [(x, w.w_t if isinstance(w, PackedWeight) else w, *rest) for x, w, *rest in items]):
         return
@@ -529,14 +536,14 @@ def linear_group(items):
         ldx, ldc = _ld(x, "x"), _ld(out, "out")
         probs[i] = GemmProblem(
             _rows(x, M, ldx, K, "x"),
-            w.planes(M)[0].data_ptr() if split[0] else _rows(wt, K, _ld(wt, "w_t"), N, "w_t"),
+            w.packed.data_ptr() if split[0] else _rows(wt, K, _ld(wt, "w_t"), N, "w_t"),
             _rows(out, M, ldc, N, "out"),
             None if bias is None else _ptr(bias, numel=N, name="bias"),
             None if out2 is None else _rows(out2, M, ldc, N, "out2"),
             None if aux is None else _rows(aux, M, ldc, N, "aux"),
             M, N, K, ldx, 0 if split[0] else _ld(wt, "w_t"), ldc, epi)
         if probe is not None:
-            panel = panel and _panel_item(M, N, K, ldc, epi, [
+            panel = panel and _panel_item(N, K, ldc, epi, [
                 out.data_ptr(), None if bias is None else bias.data_ptr()])
             c_passes = 1 + (epi in (EPI_ACCUM, EPI_PRE_SILU, EPI_SILU_GRAD))
             flops += 2.0 * M * N * K
