@@ -332,6 +332,78 @@ def test_wide_gemm(nat, M, N, K, epi):
         assert ((outs[0][1][rows].double() - silu).abs() / mag).max().item() < 2e-6
 
 
+def _shift_rows(A):
+    """Plants rows of A (M x K) whose power-of-two shift in mode 16 depends on which columns decide
+    it together: the first slab's max enters [0.5, 2^15) in its second half only, a slab grows past
+    2^15 in its first, its second and both halves, rows start late in either half, and an infinity
+    and a NaN."""
+    K = A.shape[1]
+    A[130:200, :16] *= 0.05
+    A[200:210, :32] *= 0.01
+    for i, k in enumerate((48, 64, 80, K - 16, K - 32)):
+        A[210 + i, k] = 2.0 ** 15 + 3.0
+        A[220 + i, k:] *= 2.0 ** 14
+        A[230 + i, :k] = 0.0
+        A[240 + i, :k] *= 2.0 ** -24
+    A[250, 64:80] *= 2.0 ** 15
+    A[250, 80:96] *= 2.0 ** 17
+    A[251] *= 2.0 ** -30
+    A[252] *= 2.0 ** 20
+    A[253] = 0.0
+    A[260, 70], A[300, K - 1] = float("inf"), float("nan")
+
+
+@pytest.mark.parametrize("M,N,K,epi", [(66_000, 1000, 1024, 4), (131_073, 384, 768, 3),
+                                       (262_200, 256, 768, 0)])
+def test_wide_gemm_bits(nat, M, N, K, epi):
+    """Mode 16 on the 128 x 256 tile: the same bits as 128-column slices, which run on the 128 x 128
+    kernel, with rows of every shift history."""
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    A, B, bias, aux = r(M, K), r(K, N) / math.sqrt(K), r(N), r(M, N)
+    _shift_rows(A)
+    C, C2 = (torch.zeros(M, N, device=DEV) for _ in range(2))
+    nat.linear(A, nat.PackedWeight(B, 16), bias, out=C, epilogue=epi, out2=C2, aux=aux)
+    for c in range(0, N, 128):
+        s = slice(c, min(c + 128, N))
+        ref, ref2 = (torch.zeros(M, min(128, N - c), device=DEV) for _ in range(2))
+        nat.linear(A, nat.PackedWeight(B[:, s].contiguous(), 16), bias[s].contiguous(), out=ref,
+                   epilogue=epi, out2=ref2, aux=aux[:, s].contiguous())
+        assert torch.equal(C[:, s].nan_to_num(7.5), ref.nan_to_num(7.5))
+        assert torch.equal(C2[:, s].nan_to_num(7.5), ref2.nan_to_num(7.5))
+
+
+def test_wide_gemm_gate_bits(nat):
+    """A gated group of products on the 128 x 256 tile: the bits of the ungated products as
+    128-column slices (128 x 128 kernel) followed by tta_gate_fwd."""
+    M, H, L = 61_441, 128, 2
+    idx = (0, 1, 0, 1, 0, 1, 1, 1)
+    g = torch.Generator(device=DEV).manual_seed(8)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    x = r(M, 18 * H)
+    _shift_rows(x[:, :6 * H])
+    _shift_rows(x[:, 6 * H:14 * H])
+    cols = ((0, 6 * H, 3 * H), (6 * H, 14 * H, 4 * H), (14 * H, 18 * H, 2 * H))
+    ws = [r(b - a, n) / math.sqrt(b - a) for a, b, n in cols]
+    gb = r(L * H)                              # gating columns: a product of zeros plus a bias
+    gat = gb.expand(M, L * H).contiguous()
+    sig = nat.linear(torch.zeros(M, 16, device=DEV), torch.zeros(16, L * H, device=DEV), gb,
+                     epilogue=nat.EPI_SIGMOID)
+    y, x0 = torch.empty(M, 9 * H, device=DEV), torch.empty(M, H, device=DEV)
+    off = (0, 3 * H, 7 * H)
+    nat.linear_group_gate([(x[:, a:b], nat.PackedWeight(w, 16), None, y[:, o:o + n])
+                           for (a, b, n), w, o in zip(cols, ws, off)], (0, 3, 7), sig, x0, idx, H)
+    plain = torch.empty(M, 9 * H, device=DEV)
+    for (a, b, n), w, o in zip(cols, ws, off):
+        for c in range(0, n, 128):
+            nat.linear(x[:, a:b], nat.PackedWeight(w[:, c:c + 128].contiguous(), 16),
+                       out=plain[:, o + c:o + c + 128])
+    want = torch.empty(M, 9, H, device=DEV)
+    nat.gate_fwd(plain, gat, want, idx, R=M, H=H, L=L)
+    assert torch.equal(x0.nan_to_num(7.5), plain[:, :H].nan_to_num(7.5))
+    assert torch.equal(y.nan_to_num(7.5), want.view(M, 9 * H).nan_to_num(7.5))
+
+
 @pytest.mark.parametrize("M,N,K,epi", [(30_011, 1024, 1024, 3), (30_011, 1000, 416, 4),
                                        (12_000, 768, 640, 2), (20_000, 512, 384, 0),
                                        (43_700, 256, 1024, 1)])

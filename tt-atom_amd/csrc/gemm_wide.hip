@@ -5,11 +5,14 @@
 // instructions of a wavefront; here a wavefront's tile is 32 x 256, so each split A value feeds
 // eight column blocks instead of four and a step's copies bring 24 KB for as many instructions.
 // Two workgroups still share a compute unit, so that one's epilogue overlaps the other's k loop: a
-// stage holds a 16-wide k step (24 KB) and three stages take 72 KB.  Step s multiplies stage s while
-// it reads and splits the A rows of stage s + 1 and its copies fill the stage that step s - 1 left
-// (after the barrier that retires it), so a copy has a whole step to land.  In mode 1 a stage is
-// 16 KB and a step a third as long: five stages, and a copy has three steps.  A last column tile of
-// 128 columns runs the same loop with four column blocks.
+// stage holds a 16-wide k step (24 KB) and three stages take 72 KB.  Step s multiplies the B of stage
+// s while it reads and splits the A rows of stage s + 1; its copies bring the B of stage s + 2 into
+// the place that step s - 1 left and the A of stage s + 3 into its own (its A rows were read a
+// step ago), after the barrier that retires both, so a copy has a whole step to land.  The A rows
+// run one step further ahead because mode 16 checks a row's shift once per 32-wide slab, on both of
+// its halves, before it splits the first: the same shifts, and so the same bits, as the 128 x 128
+// kernel's.  In mode 1 a stage is 16 KB and a step a third as long: five stages, and a copy has
+// three steps.  A last column tile of 128 columns runs the same loop with four column blocks.
 #include "gemm_split.h"
 
 #include <algorithm>
@@ -78,7 +81,7 @@ __global__ __launch_bounds__(WTH, 2) void gemm_wide_kernel(GemmGroup g) {
       bvo[h] = n32 < NT32 ? (pl * NT32 + n32) * 2048 + (c % 64) * 16 : (int)0x7fffffff;
     }
   };
-  auto issue = [&](int s, int stg) {
+  auto issueA = [&](int s, int stg) {
     uint4* base = smem + stg * STG + 64 * wave;
 #pragma unroll
     for (int h = 0; h < APT; ++h) {
@@ -86,6 +89,9 @@ __global__ __launch_bounds__(WTH, 2) void gemm_wide_kernel(GemmGroup g) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(arsrc, (lds_ptr)(base + WTH * h), 16, vo, s * WK * 4,
                                                0, 0);
     }
+  };
+  auto issueB = [&](int s, int stg) {
+    uint4* base = smem + stg * STG + 64 * wave;
 #pragma unroll
     for (int h = 0; h < BPT; ++h) {
       const int vo = bvo[h];
@@ -103,7 +109,6 @@ __global__ __launch_bounds__(WTH, 2) void gemm_wide_kernel(GemmGroup g) {
     x[0][1] = __builtin_bit_cast(floatx4, As[(2 * lh + 1) ^ wswz(row)]);
   };
   RowScale<1, NT, S::F16> rs;
-  const floatx4 none[1][2] = {{floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}}};
   auto split = [&](const floatx4 (&x)[1][2], int sh, V8 (&a)[NA]) {
     if constexpr (S::F16)
       split8_f16<NA>(x[0][0], x[0][1], sh, a);
@@ -137,68 +142,93 @@ __global__ __launch_bounds__(WTH, 2) void gemm_wide_kernel(GemmGroup g) {
   auto prev = [](int v) { return v == 0 ? NST - 1 : v - 1; };
   auto loop = [&](auto tj) {
     constexpr int TJ = decltype(tj)::value;
-    floatx4 x[1][2];
+    floatx4 x[1][2], y[1][2];
     V8 a[NA], b[2][2][NB];
     rdA(0, x);
+    rdA(1, y);
     rdB(0, 0, b[0]);
-    rs.check(x, none, acc, lh);
+    rs.check(x, y, acc, lh);
     split(x, S::F16 && !rs.unscaled ? rs.er[0] : 0, a);
     int s = 0, stg = 0;
-    // one step's copies, reads and products; the A rows of the next step end up in x and, FAST,
-    // split for shift 0 in na and the largest magnitude of this lane's in big
+    // one step's copies, reads and products.  ODD: the next step opens a 32-wide slab, whose two
+    // halves of A rows end up in x and y; the other steps take y into x.  FAST: the next step's rows
+    // split for shift 0 in na and, ODD, the largest magnitude of this lane's in x and y in big
     V8 na[NA];
     float big = 0.f;
-    auto step = [&](auto fast) {
+    auto take = [&](const floatx4 (&v)[1][2]) {
+      big = max3_abs(v[0][0][0], v[0][0][1], big);
+      big = max3_abs(v[0][0][2], v[0][0][3], big);
+      big = max3_abs(v[0][1][0], v[0][1][1], big);
+      big = max3_abs(v[0][1][2], v[0][1][3], big);
+    };
+    auto step = [&](auto fast, auto odd) {
+      constexpr bool LOOK = S::F16 && decltype(fast)::value && decltype(odd)::value;
       const int s1 = next(stg);
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NST - 3) * NIF) : "memory");
-      issue(min(s + NST - 1, nks - 1), prev(stg));
-      rdA(s1, x);
+      issueB(min(s + NST - 1, nks - 1), prev(stg));
+      issueA(min(s + NST, nks - 1), stg);
+      if constexpr (decltype(odd)::value) {
+        rdA(s1, x);
+      } else {
+        x[0][0] = y[0][0];
+        x[0][1] = y[0][1];
+      }
 #pragma unroll
       for (int j = 0; j < TJ; j += 2) {
         if (j + 2 < TJ)
           rdB(stg, j + 2, b[(j / 2 + 1) & 1]);
         else
           rdB(s1, 0, b[(j / 2 + 1) & 1]);
+        if (decltype(odd)::value && j == TJ - 2) rdA(next(s1), y);
         __builtin_amdgcn_sched_barrier(0);
         mm(a, b[(j / 2) & 1], j);
         if (decltype(fast)::value && j == TJ - 4) {
           split(x, 0, na);
-          if constexpr (S::F16) {
-            big = max3_abs(x[0][0][0], x[0][0][1], 0.f);
-            big = max3_abs(x[0][0][2], x[0][0][3], big);
-            big = max3_abs(x[0][1][0], x[0][1][1], big);
-            big = max3_abs(x[0][1][2], x[0][1][3], big);
+          if constexpr (LOOK) {
+            big = 0.f;
+            take(x);
           }
         }
       }
+      if constexpr (LOOK) take(y);
       stg = s1;
+      ++s;
     };
-    // every row's shift 0: no branch between the multiplications and the next split, and a new
-    // shift is needed only where a value reaches 2^15, which each lane can tell of its own
-    if (!S::F16 || rs.all_zero()) {
-      for (; s < nks; ++s) {
-        step(std::true_type{});
+    using std::false_type;
+    using std::true_type;
+    auto keep = [&]() {
 #pragma unroll
-        for (int q = 0; q < NA; ++q) a[q] = na[q];
+      for (int q = 0; q < NA; ++q) a[q] = na[q];
+    };
+    // (K is a multiple of 32: an even number of steps.)  Every row's shift 0: no branch between the
+    // multiplications and the next split, and a new shift is needed only where a value reaches
+    // 2^15, which each lane can tell of its own
+    if (!S::F16 || rs.all_zero()) {
+      while (s < nks) {
+        step(true_type{}, false_type{});
+        keep();
+        step(true_type{}, true_type{});
+        keep();
         if (S::F16 && __any(!(big < 32768.f))) {
-          rs.check(x, none, acc, lh);
+          rdA(stg, x);
+          rs.check(x, y, acc, lh);
           split(x, rs.er[0], a);
-          if (!rs.unscaled) {
-            ++s;
-            break;
-          }
+          if (!rs.unscaled) break;
         }
       }
     }
-    for (; s < nks; ++s) {
-      step(std::false_type{});
-      rs.check(x, none, acc, lh);
+    while (s < nks) {
+      step(false_type{}, false_type{});
+      split(x, S::F16 && !rs.unscaled ? rs.er[0] : 0, a);
+      step(false_type{}, true_type{});
+      rs.check(x, y, acc, lh);
       split(x, S::F16 && !rs.unscaled ? rs.er[0] : 0, a);
     }
   };
 
   set_tile(tile);
-  issue(0, 0);
+  issueA(0, 0);
+  issueB(0, 0);
   for (;;) {
     const int cm0 = m0, cn0 = n0;
 #pragma unroll
@@ -206,9 +236,14 @@ __global__ __launch_bounds__(WTH, 2) void gemm_wide_kernel(GemmGroup g) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[0][j][r] = 0.f;
     rs = RowScale<1, NT, S::F16>();
+    issueA(min(1, nks - 1), 1);
 #pragma unroll
-    for (int q = 1; q < NST - 1; ++q) issue(min(q, nks - 1), q);
-    // stage 0 landed (with everything issued before it); the later ones may still be in flight
+    for (int q = 1; q < NST - 1; ++q) {
+      issueB(min(q, nks - 1), q);
+      issueA(min(q + 1, nks - 1), q + 1);
+    }
+    // stage 0 and the A rows of stage 1 landed (with everything issued before them); the later
+    // copies may still be in flight
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NST - 2) * NIF) : "memory");
     const bool whole = cn0 + BN < p.N;  // more than 128 columns in this tile
     if (whole)
@@ -270,7 +305,8 @@ __global__ __launch_bounds__(WTH, 2) void gemm_wide_kernel(GemmGroup g) {
     tile += stride;
     if (tile >= t_end) break;
     set_tile(tile);
-    issue(0, 0);
+    issueA(0, 0);
+    issueB(0, 0);
   }
 }
 
