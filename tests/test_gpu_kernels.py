@@ -256,6 +256,37 @@ def test_small_launch_gemm(nat, mode, M, N, K):
     assert ((outs[0].double() - ref).abs() / mag).max().item() < 4 * 2.0 ** -bits
 
 
+@pytest.mark.parametrize("mode", [16, 1])
+@pytest.mark.parametrize("shapes", [((2000, 640, 768), (2000, 512, 1024), (2000, 256, 512)),
+                                    ((200, 256, 512), (300, 256, 512)),
+                                    ((4095, 1024, 256), (300, 128, 512), (256, 64, 256)),
+                                    ((5000, 384, 256), (4095, 64, 160), (1, 64, 32))])
+def test_split_group_is_its_products(nat, mode, shapes):
+    """tta_gemm_bf16x_group gives every product the bits it has alone, whatever it shares the launch
+    with: groups whose small tiles together are more than one round, products on either side of
+    the 256 rows that change the number of wavefronts, and products of the small, the 128 x 128
+    and the 128 x 256 kernel in one group."""
+    g = torch.Generator().manual_seed(mode + len(shapes))
+    xs = [torch.randn(M, K, generator=g).to(DEV) * 0.2 for M, _, K in shapes]
+    ps = [nat.PackedWeight(torch.randn(K, N, generator=g).to(DEV), mode) for _, N, K in shapes]
+    outs = [[torch.full((M, N), 7.5, device=DEV) for M, N, _ in shapes] for _ in range(2)]
+
+    def call(some, out):
+        probs = (nat.GemmProblem * len(some))(*[
+            nat.GemmProblem(xs[i].data_ptr(), ps[i].packed.data_ptr(), out[i].data_ptr(), None, None,
+                            None, *shapes[i], shapes[i][2], 0, shapes[i][1], nat.EPI_STORE)
+            for i in some])
+        nat._call("tta_gemm_bf16x_group", probs, len(some), mode, nat._stream())
+
+    call(range(len(shapes)), outs[0])
+    for i in range(len(shapes)):
+        call([i], outs[1])
+    for (M, N, K), x, p, a, b in zip(shapes, xs, ps, *outs):
+        assert torch.equal(a, b)
+        ref, mag = x.double() @ p.w_t.double(), x.double().abs() @ p.w_t.double().abs()
+        assert ((a.double() - ref).abs() / mag).max() < 4 * 2.0 ** (-22 if mode == 16 else -8)
+
+
 @pytest.mark.parametrize("M,N,K,modes", [(72, 1024, 1024, (16, 6, 3, 1)), (4, 64, 128, (16, 1)),
                                          (1205, 256, 1024, (16, 1)), (2500, 1024, 1024, (16, 6)),
                                          (4095, 1536, 128, (16, 1)), (576, 1024, 1024, (3, 1))])

@@ -822,7 +822,31 @@ int launch_mode(GemmGroup& g, int n, int mode, hipStream_t s, unsigned chunks = 
       default: return launch_bf16x<2, 6>(g, n, s, chunks);
     }
   }
-  if (small_ok(g, n)) return launch_small(g, n, mode, s);
+  // products that run on different kernels go out as one launch per kernel
+  int waves[kMaxGroup];
+  bool same = true;
+  for (int i = 0; i < n; ++i) {
+    waves[i] = small_waves(g.p[i]);
+    same = same && waves[i] == waves[0];
+  }
+  if (!same) {
+    for (int w : {0, 4, 8}) {
+      GemmGroup sub = g;
+      int m = 0;
+      for (int i = 0; i < n; ++i) {
+        if (waves[i] != w) continue;
+        sub.p[m] = g.p[i];
+        sub.NT32[m] = g.NT32[i];
+        sub.vec[m] = g.vec[i];
+        sub.gc0[m] = g.gc0[i];
+        ++m;
+      }
+      const int rc = m > 0 ? launch_mode(sub, m, mode, s) : (int)tta::kOk;
+      if (rc != tta::kOk) return rc;
+    }
+    return tta::kOk;
+  }
+  if (waves[0] > 0) return launch_small(g, n, waves[0], mode, s);
   if (!(mode == 16 && panel_ok(g, n)) && wide_ok(g, n, mode, persistent_cap()))
     return launch_wide(g, n, mode, persistent_cap(), s);
   switch (mode) {

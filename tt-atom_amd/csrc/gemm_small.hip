@@ -7,8 +7,8 @@
 // cutting K over workgroups instead sends every partial product through memory and a second
 // launch.  Here a workgroup owns a small tile (32 or 64 on a side) and its NW wavefronts take
 // consecutive ranges of K slabs (the whole tile over K / NW each), with no barrier in the k loop: a
-// wavefront loads its A rows coalesced into registers, DEPTH slabs ahead, turns them through its own LDS area into MFMA
-// fragments (LDS operations of one wavefront stay in order), and takes the packed B fragments
+// wavefront loads its A rows coalesced into registers, DEPTH slabs ahead, turns them through its
+// own LDS area into MFMA fragments (LDS operations of one wavefront stay in order), and takes the packed B fragments
 // straight to registers.  The partial tiles then meet in LDS, are added in wavefront order (fixed,
 // so results repeat) and go through the shared epilogue.  Tiles are walked column-major inside each
 // XCD's contiguous range, so that an XCD reads its own columns of the weight once.
@@ -201,36 +201,30 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void gemm_small_kernel(Ge
   }
 }
 
-// Which tile a launch takes.  Eight wavefronts share K up to 256 rows, four above (a rule on the
-// rows alone, so that a product's k sums, and its bits, do not depend on what else is in its
-// launch); a compute unit holds one workgroup of eight wavefronts or two of four, and the tile is
-// the smallest one (the shortest chain of k steps) whose workgroups are still one round.  Measured
-// per launch (us; the split-K launch pair or fp32 kernel that ran before, then 32 x 32 / 32 x 64 /
+// Which products run here, and on how many wavefronts, is a rule on the product's own rows and
+// columns (small_waves), so that its k sums, and its bits, do not depend on what else is in its
+// launch: eight wavefronts share K up to 256 rows, four above.  The tile is the launch's (every
+// tile adds an element's products in one order): a compute unit holds one workgroup of eight
+// wavefronts or two of four, and the tile is the smallest one (the shortest chain of k steps)
+// whose workgroups are still one round, or 64 x 64.  Measured per
+// launch (us; the split-K launch pair or fp32 kernel that ran before, then 32 x 32 / 32 x 64 /
 // 64 x 64 tiles, then the tiled kernel): eight wavefronts, 72 x 1024 x 1024: 11.7; 7.3, 8.0, 11.1;
 // 26.6.  Four: 433 x 1024 x 1024: 20.2; 11.0, 10.3, 13.6; 28.1 (eight: 14.4, 9.1, 12.0).
 // 576 x 1024 x 1024: 24.0; 16.3, 12.2, 13.9; 28.2.  1937 x 1024 x 1024: 77.6; 47.3, 29.4, 22.8;
-// 30.2.  2500 x 1024 x 1024 (640 tiles of 64 x 64): 89.8; 56.5, 39.2, 34.2; 31.1.  From 4096 rows
-// on callers split a convolution's columns over launches and expect the same bits: no small tile.
-enum SmallTile { kNoTile, k32x32, k32x64, k64x64 };
+// 30.2.  2500 x 1024 x 1024 (640 tiles of 64 x 64): 89.8; 56.5, 39.2, 34.2; 31.1.  4000 x 1024 x
+// 1024: 64 x 64 tiles 47, tiled 34; 4000 x 4096 x 1024: 175, 117.  From 4096 rows on callers split a
+// convolution's columns over launches and expect the same bits: no small tile.
+enum SmallTile { k32x32, k32x64, k64x64 };
 
-int max_rows(const GemmGroup& g, int n) {
-  int m = 0;
-  for (int i = 0; i < n; ++i) m = std::max(m, g.p[i].M);
-  return m;
-}
-
-SmallTile small_tile(const GemmGroup& g, int n) {
-  const int rows = max_rows(g, n);
-  if (rows >= 4096) return kNoTile;
+SmallTile small_tile(const GemmGroup& g, int n, int waves) {
   auto blocks = [&](int sm, int sn) {
     int64_t b = 0;
     for (int i = 0; i < n; ++i) b += (int64_t)tta_blocks(g.p[i].M, sm) * tta_blocks(g.p[i].N, sn);
     return b;
   };
   if (blocks(32, 32) <= 256) return k32x32;
-  if (blocks(32, 64) <= (rows <= 256 ? 256 : 512)) return k32x64;
-  if (blocks(64, 64) <= 512) return k64x64;
-  return kNoTile;
+  if (blocks(32, 64) <= (waves == 8 ? 256 : 512)) return k32x64;
+  return k64x64;
 }
 
 template <int MODE, int TI, int TJ, int NW, int DEPTH>
@@ -249,7 +243,7 @@ template <int MODE, int NW>
 void launch_waves(const GemmGroup& g, int n, hipStream_t s) {
   // slabs in flight: what 256 registers hold beside the accumulators and fragments
   constexpr int D = Split<MODE>::NB > 2 ? 1 : 2;
-  switch (small_tile(g, n)) {
+  switch (small_tile(g, n, NW)) {
     case k32x32: launch_tile<MODE, 1, 1, NW, 2 * D>(g, n, s); break;
     case k32x64: launch_tile<MODE, 1, 2, NW, D>(g, n, s); break;
     default: launch_tile<MODE, 2, 2, NW, 1>(g, n, s); break;
@@ -257,8 +251,8 @@ void launch_waves(const GemmGroup& g, int n, hipStream_t s) {
 }
 
 template <int MODE>
-void launch_mode_small(const GemmGroup& g, int n, hipStream_t s) {
-  if (max_rows(g, n) <= 256)
+void launch_mode_small(const GemmGroup& g, int n, int waves, hipStream_t s) {
+  if (waves == 8)
     launch_waves<MODE, 8>(g, n, s);
   else
     launch_waves<MODE, 4>(g, n, s);
@@ -268,14 +262,17 @@ void launch_mode_small(const GemmGroup& g, int n, hipStream_t s) {
 
 namespace tta_gemm {
 
-bool small_ok(const GemmGroup& g, int n) { return small_tile(g, n) != kNoTile; }
+int small_waves(const GemmArgs& p) {
+  if (p.M >= 4096 || (int64_t)tta_blocks(p.M, 64) * tta_blocks(p.N, 64) > 512) return 0;
+  return p.M <= 256 ? 8 : 4;
+}
 
-int launch_small(GemmGroup& g, int n, int mode, hipStream_t s) {
+int launch_small(GemmGroup& g, int n, int waves, int mode, hipStream_t s) {
   switch (mode) {
-    case 1: launch_mode_small<1>(g, n, s); break;
-    case 3: launch_mode_small<3>(g, n, s); break;
-    case 16: launch_mode_small<16>(g, n, s); break;
-    default: launch_mode_small<6>(g, n, s); break;
+    case 1: launch_mode_small<1>(g, n, waves, s); break;
+    case 3: launch_mode_small<3>(g, n, waves, s); break;
+    case 16: launch_mode_small<16>(g, n, waves, s); break;
+    default: launch_mode_small<6>(g, n, waves, s); break;
   }
   TTA_CHECK_LAUNCH("tta_gemm_bf16x");
   return tta::kOk;

@@ -434,9 +434,10 @@ struct RowScale {
 // 16 consecutive rows at one logical chunk then cover all 64 banks.
 __device__ __forceinline__ int aswz(int row) { return (row >> 1) & 7; }
 
-// The small-launch kernel (gemm_small.hip): whether the n products of g take it, and its launch.
-bool small_ok(const GemmGroup& g, int n);
-int launch_small(GemmGroup& g, int n, int mode, hipStream_t s);
+// The small-launch kernel (gemm_small.hip): the wavefronts that share a product's K there, 0 for a
+// product that does not run there, and its launch for n products of one such number.
+int small_waves(const GemmArgs& p);
+int launch_small(GemmGroup& g, int n, int waves, int mode, hipStream_t s);
 
 // The 128 x 256 kernel (gemm_wide.hip); cap: most blocks per product (persistent tiles).
 bool wide_ok(const GemmGroup& g, int n, int mode, int cap);
