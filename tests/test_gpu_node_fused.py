@@ -99,6 +99,37 @@ def test_spectral_block_nodes_per_workgroup(nat, N, C, H):
     test_spectral_block_fwd_bwd(nat, N, C, H, True, True)
 
 
+@pytest.mark.parametrize("C,H", [(128, 128), (48, 16)])
+def test_spectral_block_bits_of_a_node(nat, C, H):
+    """A node's results have the same bits however many nodes share the launch (2, 4, 8 or 16 of
+    them in a workgroup)."""
+    g = torch.Generator().manual_seed(C)
+    w = {k: v.float().to(DEV) for k, v in _block_weights(C, H, g).items()}
+    x, gn, res = (torch.randn(2100, 9, C, generator=g).to(DEV) for _ in range(3))
+    W1, W2 = w["ff.so3_linear_1.weight"], w["ff.so3_linear_2.weight"]
+    ws = w["ff.scalar_mlp.0.weight"]
+    t = lambda a: a.transpose(-1, -2).contiguous()
+    ff = (t(ws), w["ff.scalar_mlp.0.bias"], t(W1), w["ff.so3_linear_1.bias"], t(W2),
+          w["ff.so3_linear_2.bias"])
+    norm2, nxt = ((w[f"{n}.affine_weight"], w[f"{n}.affine_bias"]) for n in ("n2", "nn"))
+
+    def block(N):
+        e = lambda *s: torch.full(s, float("nan"), device=DEV)
+        o = [e(N), e(N, 2 * H), e(N, 9, H), e(N, 9, C), e(N, 9, C), e(N), e(N, 9, C)]
+        inv2, a_s, h, x2, yn, invn, gx = o
+        xs, gs, rs = (v[:N].contiguous() for v in (x, gn, res))
+        nat.spectral_block_fwd(xs, norm2, ff, inv2, a_s, h, x2, next_norm=nxt, yn=yn, invn=invn)
+        nat.spectral_block_bwd(gs, x2, nxt[0], invn, rs, xs, norm2[0], inv2, a_s, h,
+                               (W1, W2, ws), gx)
+        return [v[:300] for v in o]
+
+    first = block(300)
+    names = ("inv2", "a_s", "h", "x2", "yn", "invn", "g_x1")
+    differ = [(N, k) for N in (600, 1100, 2100) for k, a, b in zip(names, first, block(N))
+              if not torch.equal(a, b)]
+    assert not differ
+
+
 @pytest.mark.parametrize("N,C,H", [(41, 128, 128), (9, 16, 32)])
 def test_energy_head_fwd_bwd(nat, N, C, H):
     g = torch.Generator().manual_seed(7 * N + C)

@@ -79,6 +79,42 @@ struct Pack {
     return ((tile - first(l)) * 16 + qe) / T < 2 * l + 1;
   }
 };
+// a * b, rounded: never contracted into an addition
+__device__ __forceinline__ float rounded_product(float a, float b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
+
+// A degree's sum over its 2 l + 1 coefficients m of one node and column, p_0 .. p_2l, as
+// ((p_0 + p_4) + p_1) + (p_2 + p_3) for every T, so that a node's bits do not depend on how many
+// nodes share the launch.  v: this lane's rows of the degree's tiles (zero in padding rows), row
+// 4 q + e of tile i in v[i][e]: coefficient 16 / T i + (4 q + e) / T of node (4 q + e) % T.  s[e] is
+// complete in the lane whose row 4 q + e is below T.
+template <int T, int NT_>
+__device__ __forceinline__ void degree_sum(const float (&v)[NT_][4], float (&s)[4]) {
+  constexpr int E = T < 4 ? T : 4;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    if (T == 16) {
+      const float a = NT_ > 3 ? v[0][e] + v[NT_ - 1][e] : v[0][e];
+      const float b = NT_ > 3 ? v[2][e] + v[NT_ > 3 ? 3 : 0][e] : v[2][e];
+      s[e] = (a + v[1][e]) + b;
+    } else if (T == 8) {  // lanes q, q + 2: even and odd coefficients
+      const float a = NT_ > 2 ? v[0][e] + v[NT_ - 1][e] : v[0][e];
+      const float o0 = __shfl_xor(v[0][e], 32), o1 = __shfl_xor(v[1][e], 32);
+      s[e] = (a + o0) + (v[1][e] + o1);
+    } else if (T == 4) {  // lane q: coefficients q and q + 4
+      float a = NT_ > 1 ? v[0][e] + v[NT_ - 1][e] : v[0][e];
+      a += __shfl_xor(a, 16);
+      s[e] = a + __shfl_xor(a, 32);
+    } else {  // T = 2, lane q: coefficients 2 q (rows e) and 2 q + 1 (rows e + 2)
+      float a = v[0][e] + __shfl_xor(v[0][e], 32);
+      a += v[0][e + 2];
+      s[e] = a + __shfl_xor(a, 16);
+    }
+  }
+}
+
 // one row tile with the degree 0 weight (the scalar products)
 struct Scalar {
   static constexpr int TILES = 1;
@@ -216,10 +252,12 @@ __device__ __forceinline__ float rms_fwd_node(XR xr, YR yr, const float* __restr
 // channel mean on coefficient 0.  gv(j, hh) / xv(j, hh) give the adjoint and the input of
 // coefficient j at channel lane + 64 hh (registers or LDS, as the caller holds them); the
 // results for those channels are returned in out[9][2].  The sums run over the lane's channels
-// in order, then across the wavefront.
+// in order, then across the wavefront.  The fused steps are spelled out: which of two products the
+// compiler contracts into their sum differs between the numbers of nodes per workgroup.
 template <class GV, class XV>
 __device__ __forceinline__ void rms_bwd_vals(GV gv, XV xv, const float* __restrict__ aw,
                                              float inv, int C, int lane, float (&out)[9][2]) {
+#pragma clang fp contract(off)
   float s0 = 0.f;
 #pragma unroll
   for (int hh = 0; hh < 2; ++hh)
@@ -233,7 +271,7 @@ __device__ __forceinline__ void rms_bwd_vals(GV gv, XV xv, const float* __restri
 #pragma unroll
     for (int j = 0; j < 9; ++j) {
       const float v = j == 0 ? xv(0, hh) - mu : xv(j, hh);
-      ginv += gv(j, hh) * v * aw[ndeg(j) * C + c];
+      ginv = fmaf(gv(j, hh) * v, aw[ndeg(j) * C + c], ginv);
     }
   }
   ginv = tta_group_sum(ginv, 64);
@@ -244,7 +282,7 @@ __device__ __forceinline__ void rms_bwd_vals(GV gv, XV xv, const float* __restri
     const int c = lane + 64 * hh;
     if (c >= C) continue;
     const float v = xv(0, hh) - mu;
-    s1 += gv(0, hh) * (inv * aw[c]) + v * nbdw(0) * gms * (2.0f / C);
+    s1 += fmaf(gv(0, hh), inv * aw[c], v * nbdw(0) * gms * (2.0f / C));
   }
   const float m0 = tta_group_sum(s1, 64) / C;
 #pragma unroll
@@ -255,7 +293,7 @@ __device__ __forceinline__ void rms_bwd_vals(GV gv, XV xv, const float* __restri
       float gx = 0.f;
       if (c < C) {
         const float v = j == 0 ? xv(0, hh) - mu : xv(j, hh);
-        gx = gv(j, hh) * (inv * aw[ndeg(j) * C + c]) + v * nbdw(j) * gms * (2.0f / C);
+        gx = fmaf(gv(j, hh), inv * aw[ndeg(j) * C + c], v * nbdw(j) * gms * (2.0f / C));
         if (j == 0) gx -= m0;
       }
       out[j][hh] = gx;
@@ -526,15 +564,13 @@ __global__ __launch_bounds__(NTH, 1) void k_spectral_block_bwd(SpecBwdArgs p) {
   Product<Scalar, D, 1> scal;
   if (T < 16) scal.start(p.ws, 0, C, LH, C, 0, wave, lane);
   // 3. gate backward: g_h0 = g_gout0 silu'(h0); g_h_c = g_gout_c sig(gating); the degree sums
-  //    sum_{c in l} g_gout_c h_c (this wave holds every row of its columns: the lane's rows of a
-  //    node, then the lanes 16 and 32 apart that hold the others) give
+  //    sum_{c in l} g_gout_c h_c (this wave holds every row of its columns: degree_sum) give
   //    g_a_s = sum * sig'(gating) * silu'(a_s)
   __syncthreads();  // every wave is done reading g_x2
   if (hok) {
-    float sum[2][4], sg[2][4];
+    float v1[P::T1][4], v2[P::T2][4], sum[2][4], sg[2][4];  // the degrees' terms, their sums
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      sum[0][e] = sum[1][e] = 0.f;
       sg[0][e] = tta_sigmoid_acc(tta_silu(as[0][e]));
       sg[1][e] = tta_sigmoid_acc(tta_silu(as[1][e]));
 #pragma unroll
@@ -546,21 +582,21 @@ __global__ __launch_bounds__(NTH, 1) void k_spectral_block_bwd(SpecBwdArgs p) {
         } else {
           const int l = P::deg(i) - 1;
           gh = gg * sg[l][e];
-          sum[l][e] += P::used(i, 4 * q + e) ? gg * hv : 0.f;  // (padding rows may hold anything)
+          const float pr = P::used(i, 4 * q + e) ? rounded_product(gg, hv) : 0.f;
+          if (l == 0)
+            v1[i - 1][e] = pr;
+          else
+            v2[i - 1 - P::T1][e] = pr;
         }
         buf[(16 * i + 4 * q + e) * LDP + col] = gh;
       }
     }
+    degree_sum<T>(v1, sum[0]);
+    degree_sum<T>(v2, sum[1]);
 #pragma unroll
     for (int l = 0; l < 2; ++l) {
-      if (T == 2) {
-        sum[l][0] += sum[l][2];
-        sum[l][1] += sum[l][3];
-      }
 #pragma unroll
       for (int e = 0; e < (T < 4 ? T : 4); ++e) {
-        if (T <= 4) sum[l][e] += __shfl_xor(sum[l][e], 16);
-        if (T <= 8) sum[l][e] += __shfl_xor(sum[l][e], 32);
         if (4 * q + e < T)
           gas[(4 * q + e) * ldg + l * H + col] =
               sum[l][e] * sg[l][e] * (1.f - sg[l][e]) * tta_silu_grad(as[l][e]);
