@@ -950,9 +950,8 @@ def test_node_walks_few_nodes(nat, C):
     """The walks and segment sums of up to 512 nodes (eight wavefronts per node) against the
     one-wavefront forms, which take the same edges with isolated nodes appended: degrees around the
     eight edges of a round (0, 1, 7, 8, 9, 16, 17) and a hub.  The rotation adjoint rows are added
-    in one order, rounded: the same bits.  A segment sum's products may be contracted into the add
-    in one form and not the other: one more rounding per edge, (deg + 2) 2^-23 of the sum of the
-    magnitudes."""
+    in one order, rounded: the same bits.  The segment sums (whose bits test_segment_sum_bits_of_a_node
+    compares) within (deg + 2) 2^-23 of the sum of the magnitudes."""
     deg = [0, 1, 7, 8, 9, 16, 17, 100, 0, 3]
     g = torch.Generator().manual_seed(C)
     tgt = torch.repeat_interleave(torch.arange(10), torch.tensor(deg))
@@ -988,6 +987,26 @@ def test_node_walks_few_nodes(nat, C):
                              * sc.double()[:, None, None]) + (x.abs().double() if k == 4 else 0.0)
         n = torch.tensor(deg, dtype=torch.float64)[:, None, None] + 2
         assert ((got[10][k].double() - got[700][k].double()).abs() <= n * 2.0 ** -23 * mag).all()
+
+
+@pytest.mark.parametrize("C", [16, 64, 128])
+@pytest.mark.parametrize("n_in,env_first", [(9, True), (3, False), (9, False), (3, True)])
+def test_segment_sum_bits_of_a_node(nat, C, n_in, env_first):
+    """A node's segment sum has the same bits in a graph of up to 512 nodes (eight wavefronts per
+    node) and in a larger one: every contribution enters in one fused step, in edge order."""
+    deg = [0, 1, 7, 8, 9, 16, 17, 100, 0, 3]
+    g = torch.Generator().manual_seed(C + n_in)
+    tgt = torch.repeat_interleave(torch.arange(10), torch.tensor(deg))
+    E = tgt.numel()
+    r = lambda *s: torch.randn(*s, generator=g).to(DEV)
+    m, coef, env, res = r(E, n_in, C), r(E, 35), r(E), r(700, 9, C)
+    out = []
+    for N in (10, 700):
+        o = torch.full((N, 9, C), float("nan"), device=DEV)
+        nat.rotate_env_segsum(m, coef, env, _i32(_csr(tgt, N)), res[:N].contiguous(), o, n_in=n_in,
+                              env_first=env_first, div=5.0)
+        out.append(o[:10])
+    assert torch.equal(*out)
 
 
 @pytest.mark.parametrize("C", [16, 128, 256, 1024])

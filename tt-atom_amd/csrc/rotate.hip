@@ -73,6 +73,12 @@ __device__ __forceinline__ float hsum(typename VecT<V>::T v) {
   }
 }
 
+// x s + a in one rounding
+template <class T>
+__device__ __forceinline__ T fma_vs(T x, float s, T a) {
+  return __builtin_elementwise_fma(x, T(s), a);
+}
+
 // out[m] = sum_j W[m, j] in[j]   (node SH -> edge frame; also the adjoint of the inverse rotation)
 template <class T>
 __device__ __forceinline__ void rot_fwd(const float* c, const T* in, T* out) {
@@ -668,6 +674,29 @@ __global__ __launch_bounds__(64 * kFew) void k_gather_rotate_bw_walk_few(
 // counts stay exact: a conditional load would make it wait for all loads at the join.
 constexpr int kSegPF = 4;
 
+// The contribution of one edge to row j of a segment sum as a product x[j] s[j], so that it is added
+// in one fused step (and a node's bits are those of either kernel below): env / div times the
+// rotated row (edge-degree scaling; one per-edge factor, since a division per element made this
+// variant VALU-bound: it rounds once, so values move by an ulp at most), or, the envelope already
+// in the rows, 1 times the rotated row, a row of one product as that product.
+template <int NIN, bool ENV_FIRST, class T>
+__device__ __forceinline__ void seg_terms(const float* c, T* in, float ev, float rdiv, T* x,
+                                          float* s) {
+  if (ENV_FIRST) {
+#pragma unroll
+    for (int mm = 0; mm < NIN; ++mm) in[mm] = in[mm] * ev;
+  }
+  rot_inv<NIN>(c, in, x);
+#pragma unroll
+  for (int j = 0; j < NSPH; ++j) {
+    s[j] = ENV_FIRST ? 1.f : ev * rdiv;
+    if (ENV_FIRST && (j == 0 || NIN == 3)) {  // coefficient j of rot_inv's first products
+      x[j] = in[j == 0 ? 0 : j < 4 ? 1 : 2];
+      s[j] = c[j];
+    }
+  }
+}
+
 template <int V, int NIN, bool ENV_FIRST>
 __global__ __launch_bounds__(256) void k_rotate_env_segsum(
     const float* __restrict__ m, const float* __restrict__ coef, const float* __restrict__ env,
@@ -725,21 +754,11 @@ __global__ __launch_bounds__(256) void k_rotate_env_segsum(
           // refill this slot with edge e + PF before the arithmetic of edge e
           load_slot(s, e + PF);
           if (e < e1) {  // wave-uniform
-            if (ENV_FIRST) {
-#pragma unroll
-              for (int mm = 0; mm < NIN; ++mm) in[mm] = in[mm] * ev;
-            }
             T o[NSPH];
-            rot_inv<NIN>(c, in, o);
-            // edge-degree scaling: one per-edge factor env / div (a division per element made
-            // this variant VALU-bound; the factor rounds once, so values move by an ulp at most)
-            const float sc = ENV_FIRST ? 1.f : ev * rdiv;
+            float sc[NSPH];
+            seg_terms<NIN, ENV_FIRST>(c, in, ev, rdiv, o, sc);
 #pragma unroll
-            for (int j = 0; j < NSPH; ++j) {
-              T v = o[j];
-              if (!ENV_FIRST) v = v * sc;
-              acc[j] = acc[j] + v;
-            }
+            for (int j = 0; j < NSPH; ++j) acc[j] = fma_vs(o[j], sc[j], acc[j]);
           }
         }
       }
@@ -756,7 +775,8 @@ __global__ __launch_bounds__(256) void k_rotate_env_segsum(
 }
 
 // The same for few nodes (k_gather_rotate_bw_walk_few's arrangement): kFew wavefronts per node, a
-// round's edges side by side, their contributions added in edge order from LDS.
+// round's edges side by side, their contributions (seg_terms) added in edge order from LDS, each in
+// one fused step: the bits of the one-wavefront form.
 template <int V, int NIN, bool ENV_FIRST>
 __global__ __launch_bounds__(64 * kFew) void k_rotate_env_segsum_few(
     const float* __restrict__ m, const float* __restrict__ coef, const float* __restrict__ env,
@@ -768,12 +788,14 @@ __global__ __launch_bounds__(64 * kFew) void k_rotate_env_segsum_few(
   const int t = threadIdx.x, lane = t & 63;
   const int w = wave_uniform(t >> 6), n = blockIdx.x;
   const int cq = C / V, len = NSPH * cq;
+  float* scales = lds + 2 * kFew * NSPH * C;  // [2][kFew][9]
   const bool active = lane < cq;
   const int qq = active ? lane : 0;
   const int e0 = wave_uniform(ptr[n]), e1 = wave_uniform(ptr[n + 1]);
   const float rdiv = 1.f / div;
   T acc[2], row[NIN], nrow[NIN];
   acc[0] = acc[1] = zv<V>();
+  const int j[2] = {t / cq, (t + 64 * kFew) / cq};  // the rows of this thread's two elements
   float ce = 0.f, nce = 0.f;  // lane k < 35: coefficient k; the others: the envelope
   auto load = [&](int e, T (&r)[NIN], float& c) {
     e = min(e, e1 - 1);
@@ -792,25 +814,33 @@ __global__ __launch_bounds__(64 * kFew) void k_rotate_env_segsum_few(
         c[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ce), k));
       const float ev = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ce), NNZ));
       T in[NSPH], o[NSPH];
+      float sc[NSPH];
 #pragma unroll
       for (int mm = 0; mm < NSPH; ++mm) in[mm] = mm < NIN ? row[mm < NIN ? mm : 0] : zv<V>();
-      if (ENV_FIRST) {
-#pragma unroll
-        for (int mm = 0; mm < NIN; ++mm) in[mm] = in[mm] * ev;
-      }
-      rot_inv<NIN>(c, in, o);
-      const float sc = ENV_FIRST ? 1.f : ev * rdiv;
+      seg_terms<NIN, ENV_FIRST>(c, in, ev, rdiv, o, sc);
       T* slot = slots + (buf * kFew + w) * len;
       if (active) {
 #pragma unroll
-        for (int j = 0; j < NSPH; ++j) slot[j * cq + lane] = ENV_FIRST ? o[j] : o[j] * sc;
+        for (int j = 0; j < NSPH; ++j) slot[j * cq + lane] = o[j];
+      }
+      if (lane == 0) {
+#pragma unroll
+        for (int j = 0; j < NSPH; ++j) scales[(buf * kFew + w) * NSPH + j] = sc[j];
       }
     }
 #pragma unroll
     for (int mm = 0; mm < NIN; ++mm) row[mm] = nrow[mm];
     ce = nce;
     __syncthreads();
-    add_slots(acc, slots + buf * kFew * len, min(kFew, e1 - eb), len, t);
+    const T* slot = slots + buf * kFew * len;
+    const int count = min(kFew, e1 - eb);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int idx = t + 64 * kFew * i;
+      const float* sc = scales + buf * kFew * NSPH + j[i];
+      if (idx < len)
+        for (int s = 0; s < count; ++s) acc[i] = fma_vs(slot[s * len + idx], sc[s * NSPH], acc[i]);
+    }
     buf ^= 1;
   }
 #pragma unroll
@@ -953,7 +983,7 @@ int pick_v(int64_t W) {
 // 500 of 30 128 -> 87 / 22.4 -> 15.5 / 12.3 -> 7.2; 864 of 30 148 -> 151 / 25.4 -> 24.9 / 13.6 ->
 // 13.8; 2048 of 30 298 -> 319 / 52 -> 55 / 21 -> 25.
 bool few_nodes(int64_t N, int64_t C, int V) { return N <= 512 && V <= 2 && C / V <= 64; }
-size_t few_lds(int64_t C) { return 2 * kFew * NSPH * C * sizeof(float); }
+size_t few_lds(int64_t C) { return 2 * kFew * NSPH * (C + 1) * sizeof(float); }
 
 unsigned wave_blocks(int64_t items) { return (unsigned)((items + WAVES - 1) / WAVES); }
 
