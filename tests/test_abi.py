@@ -33,6 +33,12 @@ def test_argument_errors_are_reported_without_a_device():
     assert b"negative" in lib.tta_last_error()
     assert lib.tta_gather_rotate(None, None, None, None, None, None, 1, 1, 6, None) != 0
     assert b"unsupported channel count" in lib.tta_last_error()
+    # an edge adjoint that gathers its rows from the buffer it writes
+    one = [16] * 14
+    assert lib.tta_orb_edge_bwd_rows(16, *one, 1, 1, 4, None) != 0
+    assert b"different buffers" in lib.tta_last_error()
+    assert lib.tta_orb_edge_bwd_rows(32, None, *one[1:], 1, 1, 4, None) != 0
+    assert b"null pointer" in lib.tta_last_error()
 
 
 def test_walk_width_rule_matches_the_library():

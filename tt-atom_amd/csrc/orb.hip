@@ -734,8 +734,10 @@ static int edge_bwd(const char* who, float* g_e, const float* g_node_in, const f
   TTA_CHECK_ARG(N >= 0 && E >= 0 && row_width_ok(C), "%s: bad sizes", who);
   if (E == 0) return tta::kOk;
   TTA_CHECK_ARG(g_e && g_node_in && ue && sig && cut && h2 && inv && wn && attn_w && send &&
-                    recv && g_h2 && g_cut && (!g_from || (g_row && g_from != g_e)),
+                    recv && g_h2 && g_cut && (!g_from || g_row),
                 "%s: null pointer", who);
+  TTA_CHECK_ARG(g_from != g_e, "%s: g_from and g_e must be different buffers (rows are read in "
+                "another order than they are written)", who);
   hipLaunchKernelGGL(k_edge_bwd, dim3(tta_blocks(E, 4)), dim3(256), 0, stream, g_e, g_node_in, ue,
                      sig, cut, h2, inv, wn, attn_w, send, recv, g_h2, g_cut, E, (int)C, g_from,
                      g_row);
