@@ -1,6 +1,8 @@
 """Per-kernel parity on the MI355X: every HIP kernel of the edgewise path against a torch-CPU
 (fp64) restatement of the same operation, or against the oracle.  Run with ``-m gpu``."""
+import ctypes
 import math
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -149,10 +151,10 @@ def test_gemm_splitk_group_bits(nat):
 @pytest.mark.parametrize("epi", [0, 1, 2, 3, 4])
 def test_split_gemm_small_splitk(nat, epi):
     """Small-M products of packed (mode 16) weights that would run unsplit on the fp32 kernel at
-    its matrix rate take the split kernel's split-K form: 576 x 1024 x 1024 (8 chunks of 128)
-    against fp64 at the split kernel's fp32-level accuracy, every epilogue, with rows scaled far
-    outside the unscaled window and a row whose values only start in the second chunk, and
-    bit-identical on a second call."""
+    its matrix rate take the small-launch split kernel (the launches that the library's split-K
+    rule cuts): 576 x 1024 x 1024 against fp64 at the split kernel's fp32-level accuracy, every
+    epilogue, with rows scaled far outside the unscaled window and a row whose values only start
+    in the second wavefront's share of K, and bit-identical on a second call."""
     g = torch.Generator().manual_seed(40 + epi)
     M, N, K = 576, 1024, 1024
     A = torch.randn(M, K, generator=g)
@@ -197,7 +199,7 @@ def test_split_gemm_small_splitk(nat, epi):
 
 def test_split_gemm_small_splitk_group(nat):
     """An SO(2)-shaped group at 576 edges (the three m-block products, K = 768 / 1024 / 512)
-    through linear_group on the split kernel's split-K form, each product against fp64."""
+    through linear_group on the small-launch split kernel, each product against fp64."""
     g = torch.Generator().manual_seed(77)
     M = 576
     shapes = [(768, 640), (1024, 512), (512, 256)]
@@ -214,6 +216,105 @@ def test_split_gemm_small_splitk_group(nat):
         ref = x.double() @ w.double()
         mag = x.double().abs() @ w.double().abs()
         assert ((o.cpu().double() - ref).abs() / mag).max().item() < 2e-6
+
+
+@pytest.mark.parametrize("mode", [1, 3, 6, 16])
+@pytest.mark.parametrize("epi", [0, 1, 2, 3, 4, 5])
+def test_splitk_entry(nat, mode, epi):
+    """tta_gemm_bf16x_group_splitk itself: two products whose K is cut into chunks (ragged rows,
+    columns and k slabs) and one that stays whole, every epilogue, in mode 16 with scaled rows and
+    a row that starts in a later chunk, against fp64 with the bounds of the plane formats, twice with
+    the same bits; a workspace that is too small is refused."""
+    g = torch.Generator().manual_seed(10 * mode + epi)
+    shapes = [(576, 1024, 1024), (101, 260, 388), (70, 64, 128)]
+    r = lambda *s: torch.randn(*s, generator=g)
+    xs, bs = [r(M, K) for M, _, K in shapes], [r(N) for _, N, _ in shapes]
+    if mode == 16:
+        xs[0][3] *= 2.0 ** 20
+        xs[0][4] *= 2.0 ** -30
+        xs[0][5, :300] = 0.0
+        xs[1][6, 200:] *= 2.0 ** 17
+    ws = [r(K, N) / math.sqrt(K) for _, N, K in shapes]
+    pws = [nat.PackedWeight(w.to(DEV), mode) for w in ws]
+    xd, bd = [x.to(DEV) for x in xs], [b.to(DEV) for b in bs]
+    c0, aux = [r(M, N) for M, N, _ in shapes], [r(M, N) for M, N, _ in shapes]
+    auxd = [a.to(DEV) for a in aux]
+    runs = []
+    for _ in range(2):
+        out, out2 = [c.to(DEV) for c in c0], [torch.zeros_like(c, device=DEV) for c in c0]
+        probs = (nat.GemmProblem * 3)(*[
+            nat.GemmProblem(xd[i].data_ptr(), pws[i].packed.data_ptr(), out[i].data_ptr(),
+                            bd[i].data_ptr(), out2[i].data_ptr(), auxd[i].data_ptr(), M, N, K, K, 0,
+                            N, epi) for i, (M, N, K) in enumerate(shapes)])
+        need = nat.load().tta_gemm_bf16x_splitk_work(probs, 3)
+        assert need > sum(M * N for M, N, _ in shapes)
+        work = torch.full((need,), float("nan"), device=DEV)
+        with pytest.raises(RuntimeError, match="work holds"):
+            nat._call("tta_gemm_bf16x_group_splitk", probs, 3, mode, work.data_ptr(), need - 1,
+                      nat._stream())
+        nat._call("tta_gemm_bf16x_group_splitk", probs, 3, mode, work.data_ptr(), need,
+                  nat._stream())
+        runs.append([t.cpu() for t in out + out2])
+    for a, b in zip(*runs):
+        assert torch.equal(a, b)
+    bound = 4 * 2.0 ** -{1: 8, 3: 16, 6: 22, 16: 22}[mode]
+    for i in range(3):
+        pre = xs[i].double() @ ws[i].double() + bs[i].double()
+        mag = xs[i].double().abs() @ ws[i].double().abs() + bs[i].double().abs()
+        s = torch.sigmoid(aux[i].double())
+        d = s * (1 + aux[i].double() * (1 - s))
+        silu = torch.nn.functional.silu
+        ref, m = {0: (pre, mag), 1: (silu(pre), mag), 2: (pre + c0[i].double(), mag + c0[i].abs()),
+                  3: (pre, mag), 4: (pre * d, mag * (d.abs() + 0.05)),
+                  5: (torch.sigmoid(pre), mag + 0.25)}[epi]
+        # SiLU's slope is at most 1.1; the sigmoid itself (3 half ulps of 1: 2e-7 absolute) is below
+        # a quarter of the smallest bound
+        assert ((runs[0][i].double() - ref).abs() / m).max() < 1.1 * bound
+        if epi == 3:
+            assert ((runs[0][3 + i].double() - silu(pre)).abs() / mag).max() < 1.1 * bound
+
+
+@pytest.mark.parametrize("backward", [False, True])
+def test_splitk_gate_entries(nat, backward):
+    """tta_gemm_bf16x_group_gate(_bwd) with a workspace (K cut into chunks, the gate applied in the
+    reduction) against fp64, and against the same call without one."""
+    M, H, idx = 700, 48, (0, 1, 0, 1, 0, 1, 1, 1)
+    g = torch.Generator().manual_seed(3 + backward)
+    shapes, c0 = [(M, 3 * H, 768), (M, 4 * H, 1024), (M, 2 * H, 512)], (0, 3, 7)
+    r = lambda *s: torch.randn(*s, generator=g)
+    xs, ws = [r(M, K) for _, _, K in shapes], [r(K, N) / math.sqrt(K) for _, N, K in shapes]
+    pws, xd = [nat.PackedWeight(w.to(DEV), 16) for w in ws], [x.to(DEV) for x in xs]
+    sig, x0 = torch.rand(M, 2 * H, generator=g), r(M, H)
+    got = []
+    for split in (True, False):
+        y, x0d = torch.full((M, 9 * H), float("nan"), device=DEV), x0.to(DEV)
+        sd = sig.to(DEV)
+        outs = [y[:, c * H:c * H + N] for c, (_, N, _) in zip(c0, shapes)]
+        probs = (nat.GemmProblem * 3)(*[
+            nat.GemmProblem(xd[i].data_ptr(), pws[i].packed.data_ptr(), outs[i].data_ptr(), None,
+                            None, None, M, N, K, K, 0, 9 * H,
+                            nat.EPI_GATE_BWD if backward else nat.EPI_GATE)
+            for i, (_, N, K) in enumerate(shapes)])
+        need = nat.load().tta_gemm_bf16x_splitk_work(probs, 3)
+        assert need > M * 9 * H
+        work = torch.full((need,), float("nan"), device=DEV)
+        nat._call("tta_gemm_bf16x_group_gate_bwd" if backward else "tta_gemm_bf16x_group_gate",
+                  probs, 3, 16, (ctypes.c_int64 * 3)(*c0), sd.data_ptr(), 2 * H, x0d.data_ptr(), H, H,
+                  (ctypes.c_int * 8)(*idx), work.data_ptr() if split else None,
+                  need if split else 0, nat._stream())
+        got.append((y.cpu().double().view(M, 9, H), x0d.cpu().double()))
+    pre = torch.cat([x.double() @ w.double() for x, w in zip(xs, ws)], 1).view(M, 9, H)
+    mag = torch.cat([x.double().abs() @ w.double().abs() for x, w in zip(xs, ws)], 1).view(M, 9, H)
+    s = torch.cat([torch.ones(M, 1, H), sig.view(M, 2, H)[:, list(idx)]], 1).double()
+    ref = pre * s
+    if backward:
+        s0 = torch.sigmoid(x0.double())
+        ref[:, 0] = pre[:, 0] * s0 * (1 + x0.double() * (1 - s0))
+    else:
+        ref[:, 0] = torch.nn.functional.silu(pre[:, 0])
+    for y, x0o in got:
+        assert ((y - ref).abs() / mag).max() < 2e-6
+        assert ((x0o - (x0.double() if backward else pre[:, 0])).abs() / mag[:, 0]).max() < 2e-6
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 36, 128), (31, 130, 132), (33, 64, 1024), (256, 1000, 160),
@@ -1137,8 +1238,8 @@ def test_gemm_gate_epilogue(nat, mode, M):
     gate table, H = 48 so that 128-column tiles straddle coefficients) after the gating columns'
     sigmoid epilogue: at M = 5000 (direct launches, ragged last row tile) the gated rows and
     coefficient 0's pre-activation equal the ungated launch followed by tta_gate_fwd bit for bit,
-    the sigmoids match; at M = 700 (split-K, the gate applied in the reduction) all of them match
-    fp64 at fp32-GEMM accuracy."""
+    the sigmoids match; at M = 700 (small-launch kernel) all of them match fp64 at fp32-GEMM
+    accuracy."""
     H, cin, L = 48, 32, 2
     x, wm0, w1, w2, bm0 = _conv1_case(M, H, cin, 60 + mode + M)
     idx = (0, 1, 0, 1, 0, 1, 1, 1)
@@ -1192,7 +1293,7 @@ def test_gemm_gate_bwd_epilogue(nat, M):
     strided views of one [gating | coefficients] adjoint row: at M = 5000 the coefficient
     adjoints equal the plain products followed by tta_gate_bwd bit for bit (the sigmoids come
     from the GEMM's sigmoid epilogue on the same gating pre-activations) and the gating adjoint
-    matches it to fp32 rounding; at M = 700 (split-K) both match fp64."""
+    matches it to fp32 rounding; at M = 700 (small-launch kernel) both match fp64."""
     H, C, L = 48, 64, 2                                # K = 192, 256, 128: all on the split kernel
     idx = (0, 1, 0, 1, 0, 1, 1, 1)
     g = torch.Generator().manual_seed(90 + M)
@@ -1471,25 +1572,36 @@ def test_ln_silu_groups_equal_per_group(nat, n):
         assert not bool(x.isnan().any()) and torch.equal(x, y)
 
 
-@pytest.mark.parametrize("packed", [False, True])
-def test_activation_accuracy(nat, packed):
-    """Sigmoid, SiLU and its derivative as the GEMM epilogues evaluate them, against fp64: a
-    product of zeros plus a bias that holds the arguments (the derivative: bias 1, arguments in
-    aux).  Bound: exp to 1 ulp of the hardware's 2^p and two roundings, 1 + e, the quotient and
-    the product to half an ulp each, 5 ulp = 6e-7 relative in all; the derivative's 1 + x (1 - s)
-    cancels, so its bound is 5 ulp of 1 + |x| in absolute terms times the sigmoid."""
+@pytest.mark.parametrize("kinds,M,K", [(("f32",), 3, 64), (("f16x3",), 40, 256),
+                                       (("f16x3",), 4099, 256), (("f16x3", "f16x3-panel"), 4099, 128),
+                                       (("bf16x1",), 8192, 384)])
+def test_activation_accuracy(nat, kinds, M, K):
+    """Sigmoid, SiLU and its derivative as the GEMM epilogues evaluate them (fp32 kernel, small,
+    128 x 128, panel and 128 x 256 split kernels), against fp64: a product of zeros plus a bias that
+    holds the arguments (the derivative: bias 1, arguments in aux).  Bound: expf to 1 ulp, 1 + e,
+    the quotient and the product to half an ulp each, 5 half ulps = 3e-7 relative; twice that
+    here.  The derivative's 1 + x (1 - s) cancels, so its bound is in terms of 1 + |x| times the
+    sigmoid."""
     x = torch.cat([torch.linspace(-87, 100, 4001), torch.randn(4000, generator=torch.Generator()
                    .manual_seed(3)), torch.tensor([0.0, 1e-30, -1e-30])])
     special = torch.tensor([float("inf"), float("-inf"), float("nan"), 3e38, -3e38])
     args = torch.cat([x, special, torch.zeros(-(len(x) + 5) % 64)]).to(DEV)
-    M, N, K = 3, len(args), 64
+    N = len(args)
     w = torch.zeros(K, N, device=DEV)
-    w = nat.PackedWeight(w, 16) if packed else w
+    w = w if kinds[0] == "f32" else nat.PackedWeight(w, 1 if kinds[0] == "bf16x1" else 16)
     A = torch.zeros(M, K, device=DEV)
-    outs = [nat.linear(A, w, args, epilogue=e)[1].cpu() for e in (nat.EPI_SIGMOID, nat.EPI_SILU)]
-    aux = args.expand(M, N).contiguous()
-    one = torch.ones(N, device=DEV)
-    outs.append(nat.linear(A, w, one, epilogue=nat.EPI_SILU_GRAD, aux=aux)[2].cpu())
+    ran = []
+    nat.set_gemm_probe(SimpleNamespace(before=lambda flops, nbytes, kind, **_: ran.append(kind),
+                                       after=lambda: None))
+    try:
+        outs = [nat.linear(A, w, args, epilogue=e)[M - 2].cpu()
+                for e in (nat.EPI_SIGMOID, nat.EPI_SILU)]
+        aux = args.expand(M, N).contiguous()
+        one = torch.ones(N, device=DEV)
+        outs.append(nat.linear(A, w, one, epilogue=nat.EPI_SILU_GRAD, aux=aux)[M - 1].cpu())
+    finally:
+        nat.set_gemm_probe(None)
+    assert set(ran) == set(kinds)
     n, xd = len(x), x.double()
     s = torch.sigmoid(xd)
     sig, silu, grad = (o[:n].double() for o in outs)
