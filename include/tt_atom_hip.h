@@ -80,8 +80,9 @@ int tta_gemm_bf16x(const float* A, const void* Bp, float* C, const float* bias, 
  * blocks.  Same checks and results as one call per product;
  * empty products are skipped. */
 int tta_gemm_bf16x_group(const tta_gemm_problem* probs, int64_t n, int mode, tta_stream_t stream);
-/* tta_gemm_bf16x_group for launches too small to fill the GPU (the same call sites on small
- * systems, where the fp32 kernel would otherwise run them at its matrix rate): when the products
+/* tta_gemm_bf16x_group with K cut over workgroups, for launches too small to fill the GPU and
+ * callers with a workspace (tta_gemm_bf16x_group itself shares K over the wavefronts of a
+ * workgroup below 4096 rows, without one, and is what the package calls): when the products
  * have fewer than 128 tiles of 128 x 128 in all, those with K >= 256 have their K cut into
  * chunks of whole 32-wide slabs (at least 128); each chunk's partial product goes to work and a
  * second launch sums the chunks in order and applies bias and epilogue.  No row-gather term.

@@ -450,8 +450,8 @@ __global__ __launch_bounds__(256) void k_pack_b(const float* __restrict__ B, int
 // row's scale over the whole of K (E = 0 while the row max is in [2^-1, 2^15), else the max lands
 // below 2^kTop, as in the tiled kernel) and keeps the two fp16 planes in registers for the whole
 // run.  The packed B tiles, their column exponents and the bias reach LDS by direct copies
-// (buffer_load ... lds, no register round trip; F and the bias through registers).  Each output tile is computed transposed,
-// D^T = B^T A^T: the packed B fragment is the MFMA's first operand and the A planes its second, so
+// (buffer_load ... lds, no register round trip; F and the bias through registers).  Each output
+// tile is computed transposed, D^T = B^T A^T: the packed B fragment is the MFMA's first operand and the A planes its second, so
 // accumulator elements 4g .. 4g + 3 of lane l are four consecutive columns of row l % 32; the
 // epilogue stages them through LDS (16 rows at a time) and stores 128-byte row segments.
 // Requires ldc < 2^22 (32-bit store offsets within a wave's 32 rows).

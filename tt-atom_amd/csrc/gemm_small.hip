@@ -1,6 +1,7 @@
-// Split-plane GEMM for launches too small to fill the GPU with 128 x 128 tiles (the linears of
-// small systems and mid-size node batches): the products, arithmetic and epilogues of
-// gemm_bf16.hip, K split over the wavefronts of one workgroup.
+// Split-plane GEMM for products too small to fill the GPU with 128 x 128 tiles (the wider linears
+// of small systems and mid-size node batches; their narrow ones keep fp32 operands, gemm.hip): the
+// products, arithmetic and epilogues of gemm_bf16.hip, K split over the wavefronts of one
+// workgroup.
 //
 // A launch of few tiles is bound by the serial chain of a tile's k steps, not by the matrix cores:
 // the tiled kernel's workgroup waits out a copy round trip and a barrier per 32-wide slab, and
@@ -8,9 +9,9 @@
 // launch.  Here a workgroup owns a small tile (32 or 64 on a side) and its NW wavefronts take
 // consecutive ranges of K slabs (the whole tile over K / NW each), with no barrier in the k loop: a
 // wavefront loads its A rows coalesced into registers, DEPTH slabs ahead, turns them through its
-// own LDS area into MFMA fragments (LDS operations of one wavefront stay in order), and takes the packed B fragments
-// straight to registers.  The partial tiles then meet in LDS, are added in wavefront order (fixed,
-// so results repeat) and go through the shared epilogue.  Tiles are walked column-major inside each
+// own LDS area into MFMA fragments (LDS operations of one wavefront stay in order), and takes the
+// packed B fragments straight to registers.  The partial tiles then meet in LDS, are added in
+// wavefront order (fixed, so results repeat) and go through the shared epilogue.  Tiles are walked column-major inside each
 // XCD's contiguous range, so that an XCD reads its own columns of the weight once.
 #include "gemm_split.h"
 

@@ -1,5 +1,5 @@
-// Shared pieces of the split-plane GEMM kernels (gemm_bf16.hip, gemm_small.hip): the plane formats
-// and their products, the splits of an fp32 operand, and the epilogue of a tile staged in LDS.  The
+// Shared pieces of the split-plane GEMM kernels (gemm_bf16.hip, gemm_small.hip, gemm_wide.hip): the
+// plane formats and their products, the splits of an fp32 operand, and the epilogue of a tile staged in LDS.  The
 // modes, the packed layout of B and the scaling of mode 16 are described in gemm_bf16.hip.
 #pragma once
 

@@ -262,8 +262,9 @@ __global__ __launch_bounds__(WTH, 2) void gemm_wide_kernel(GemmGroup g) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       // 128 columns at a time, the rows' loads batched in mode 1 too (232 registers: 30,011 x 1024 x
-      // 1024 with the SiLU-gradient epilogue 113 -> 102 us, 60,000 rows 293 -> 243; the 128 x 128
-      // kernel in mode 1 loses 3-8 % on its other epilogues with the registers that takes)
+      // 1024 with the SiLU-gradient epilogue 113 -> 102 us, 60,000 rows 293 -> 243, when it was made;
+      // the 128 x 128 kernel in mode 1 loses 3-8 % on its other epilogues with the registers that
+      // takes)
       if (h == 1 && !whole) break;
 #pragma unroll
       for (int j = 0; j < NT / 2; ++j)
@@ -315,22 +316,26 @@ __global__ __launch_bounds__(WTH, 2) void gemm_wide_kernel(GemmGroup g) {
 namespace tta_gemm {
 
 // Whether a launch takes the wide tile: mode 16 or 1, whole 32-wide k slabs, at least one whole
-// column tile per product and, in mode 16, enough work that the uneven last round of the larger
-// tiles costs less than the loop gains: 3072 k columns of tiles per resident workgroup.  Measured,
-// 128 x 128 -> 128 x 256 (us): 196,555 x 1024 x 1024 with the SiLU-gradient epilogue (12,288
-// columns) 1427 -> 1336, with the two-output epilogue 1460 -> 1374; x 1024 x 256 (3072) 557 -> 526;
-// x 256 x 1024 (3072) 332 -> 323; 61,440 rows, conv-1 group (3840) 470 -> 448, its adjoint (7470)
-// 520 -> 500; below the line, conv-2 group (1920) 243 -> 248, 640 x 768 (2160) 197 -> 199, 10,150 x
-// 1024 x 1024 (640) 82 -> 95.
+// column tile per product.  Mode 16 also needs 3072 k columns of tiles per resident workgroup: from
+// there on the uneven last round of the larger tiles costs at most 1 %, below it decides by how
+// that round happens to fill.  Measured, 128 x 128 -> 128 x 256 (us; M x N x K, k columns): 196,555
+// x 1024 x 1024 (12,288) with the two-output epilogue 1460 -> 1350, with the SiLU-gradient one 1432
+// -> 1337; 61,440 rows, conv-1 group (4560) 461 -> 438, its adjoint (4200) 484 -> 470; 90,000 x 640
+// x 768 (3168) 285 -> 286; 50,000 x 1024 x 1024 (3128) 362 -> 341; 196,555 x 1024 x 256 (3072) 559 ->
+// 546, x 256 x 1024 (3072) 339 -> 320.  Below the line, 45,000 x 1024 x 1024 (2816) 314 -> 316,
+// 180,000 x 256 x 1024 (2814) 315 -> 307, 80,000 x 640 x 768 (2812) 246 -> 262, 40,000 x 1024 x 1024
+// (2504) 297 -> 267, conv-2 group of 80,000 rows (2500) 288 -> 299 and of 61,440 (1920) 219 -> 231,
+// 61,440 x 640 x 768 (2160) 198 -> 195, 10,150 x 1024 x 1024 (640) 86 -> 97.
 //
 // Mode 1 has a third of the products per copied byte, so its gain hangs on whole rounds of
 // resident workgroups rather than on the work in all: it takes the wide tile where that makes
 // five rounds or fewer out of eight of the 128 x 128 kernel's, at an average K of at least 384.
 // Measured, 128 x 128 -> 128 x 256 (us): 30,011 x 1024 x 1024 (4 rounds -> 2) with the two-output
-// epilogue 119 -> 103, with the SiLU-gradient one 131 -> 102; 61,440 rows (8 -> 4), conv-1 group
-// 256 -> 222, its adjoint 341 -> 277; 12,000 x 768 x 640 (2 -> 1) 36 -> 30; below the line, 20,000
-// x 1024 x 512 (3 -> 2) 56 -> 60, 8,000 x 1024 x 1024 (1 -> 1) 36 -> 43, 30,011 x 256 x 1024
-// (1 -> 1) 34 -> 39, and 60,000 x 1024 at K = 256 / 128 (8 -> 4) 110 -> 116 / 96 -> 103.
+// epilogue 135 -> 112, with the SiLU-gradient one 170 -> 135; 61,440 rows (8 -> 4), conv-1 group
+// 303 -> 260, its adjoint 346 -> 285; 12,000 x 768 x 640 (2 -> 1) 38 -> 31.  Below the line the gain
+// is 0 to 7 %: 20,000 x 1024 x 512 (3 -> 2) 46 -> 44, 8,000 x 1024 x 1024 (1 -> 1) 29 -> 28, 30,011 x
+// 256 x 1024 (1 -> 1) 28.5 -> 28.5, 60,000 x 1024 at K = 256 / 128 (8 -> 4) 81 -> 77 / 63 -> 60.
+// (Drawn when those were losses of 5 to 20 %, before the epilogue's loads went out in batches.)
 bool wide_ok(const GemmGroup& g, int n, int mode, int cap) {
   if (mode != 16 && mode != 1) return false;
   int64_t cols = 0, wide = 0, tiles = 0;

@@ -189,9 +189,9 @@ __global__ __launch_bounds__(256) void k_segment_sum_table(const float* __restri
   *(reinterpret_cast<vec*>(out) + gid) = acc;
 }
 
-// Edges per workgroup of the tiled forms: as many as 256 float4 columns (tiled rotation) or about
-// 36 KB of rows take, so that four workgroups share a compute unit; 0: one edge's rows pass
-// 64 KB, the general form.
+// Edges per workgroup of the tiled forms: what 38 KB of LDS hold, at most 64, so that four
+// workgroups share a compute unit; one edge whose rows take more gets a workgroup of its own (two
+// per compute unit) up to 64 KB; 0: past that, the general form.
 int tile_edges(int64_t floats_per_edge) {
   const int64_t bytes = 4 * floats_per_edge;
   if (bytes > 65536) return 0;

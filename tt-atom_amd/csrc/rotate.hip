@@ -1098,8 +1098,8 @@ extern "C" int tta_gather_rotate_bw_srcwalk(const float* g_xf, const float* rad,
   TTA_V_DISPATCH(V, {
     if (VV <= 2 && few_nodes(N, C, VV))
       hipLaunchKernelGGL((k_gather_rotate_bw_walk_few<VV <= 2 ? VV : 2, false>), dim3((unsigned)N),
-                         dim3(64 * kFew), few_lds(C), stream, g_xf, rad, x, src_ptr, src_perm, coef, g_rad, nullptr, coef_half,
-                       nullptr, nullptr, ssum, (int)C);
+                         dim3(64 * kFew), few_lds(C), stream, g_xf, rad, x, src_ptr, src_perm, coef,
+                         g_rad, nullptr, coef_half, nullptr, nullptr, ssum, (int)C);
     else
       hipLaunchKernelGGL((k_gather_rotate_bw_walk<VV, false>), dim3(wave_blocks(N)), dim3(256), 0,
                          stream, g_xf, rad, x, src_ptr, src_perm, coef, g_rad, nullptr, coef_half,
@@ -1124,8 +1124,8 @@ extern "C" int tta_gather_rotate_bw_tgtwalk(const float* g_xf, const float* rad,
   TTA_V_DISPATCH(V, {
     if (VV <= 2 && few_nodes(N, C, VV))
       hipLaunchKernelGGL((k_gather_rotate_bw_walk_few<VV <= 2 ? VV : 2, true>), dim3((unsigned)N),
-                         dim3(64 * kFew), few_lds(C), stream, g_xf, rad, x, tgt_ptr, nullptr, coef, g_rad, g_coef,
-                       const_cast<float*>(coef_half), ssum, res, out, (int)C);
+                         dim3(64 * kFew), few_lds(C), stream, g_xf, rad, x, tgt_ptr, nullptr, coef,
+                         g_rad, g_coef, const_cast<float*>(coef_half), ssum, res, out, (int)C);
     else
       hipLaunchKernelGGL((k_gather_rotate_bw_walk<VV, true>), dim3(wave_blocks(N)), dim3(256), 0,
                          stream, g_xf, rad, x, tgt_ptr, nullptr, coef, g_rad, g_coef,
