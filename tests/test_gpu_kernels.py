@@ -357,6 +357,35 @@ def test_small_launch_gemm(nat, mode, M, N, K):
     assert ((outs[0].double() - ref).abs() / mag).max().item() < 4 * 2.0 ** -bits
 
 
+@pytest.mark.parametrize("M,N,K", [(72, 1024, 1024), (576, 1024, 1024), (514, 640, 768),
+                                   (1237, 1024, 1024), (300, 512, 256), (300, 256, 2048)])
+@pytest.mark.parametrize("mode", [16, 6])
+def test_small_launch_error(nat, mode, M, N, K):
+    """The small-launch kernel is no further from fp64 (2-norm) than the split-K form, whose launches
+    it takes (K in chunks of 128 to 160 columns, added in order), and than the fp32 kernel."""
+    g = torch.Generator(device=DEV).manual_seed(K + M)
+    x = torch.randn(M, K, generator=g, device=DEV)
+    w = torch.randn(K, N, generator=g, device=DEV) / math.sqrt(K)
+    pw = nat.PackedWeight(w, mode)
+    ref = x.double() @ w.double()
+    err = {}
+    for kind in ("small", "splitk", "f32"):
+        o = torch.empty(M, N, device=DEV)
+        probs = (nat.GemmProblem * 1)(nat.GemmProblem(
+            x.data_ptr(), pw.packed.data_ptr(), o.data_ptr(), None, None, None, M, N, K, K, 0, N, 0))
+        if kind == "small":
+            nat._call("tta_gemm_bf16x_group", probs, 1, mode, nat._stream())
+        elif kind == "splitk":
+            need = nat.load().tta_gemm_bf16x_splitk_work(probs, 1)
+            work = torch.empty(need, device=DEV)
+            nat._call("tta_gemm_bf16x_group_splitk", probs, 1, mode, work.data_ptr(), need,
+                      nat._stream())
+        else:
+            nat.linear(x, w, out=o)
+        err[kind] = float((o.double() - ref).norm() / ref.norm())
+    assert err["small"] <= err["splitk"] and err["small"] <= err["f32"], err
+
+
 @pytest.mark.parametrize("mode", [16, 1])
 @pytest.mark.parametrize("shapes", [((2000, 640, 768), (2000, 512, 1024), (2000, 256, 512)),
                                     ((200, 256, 512), (300, 256, 512)),

@@ -82,23 +82,41 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void gemm_small_kernel(Ge
               brsrc, bvo, ((kt * NB + q) * NT32 + n0 / 32 + j) * 2048 + ks * 1024, 0);
   };
   uint4* As = smem + wave * (SM * SLDT / 4);
-  auto mm = [&](const floatx4 (&x)[TI][2], const u32x4 (&b)[TJ][2][NB], int ks, bool scaled) {
-    V8 av[TI][NA];
+  // The products of one slab.  All but the leading ones (a0 b0) are summed by themselves and enter
+  // the accumulator together, once per slab: every rounding of the accumulator costs half an ulp of
+  // the whole sum, and a wavefront's share of K is up to twice the split-K form's chunk.  Relative
+  // 2-norm error in mode 16, one chain -> this (split-K form, fp32 kernel): 576 x 1024 x 1024 1.96e-7 ->
+  // 1.47e-7 (1.57e-7, 5.7e-7), 514 x 640 x 768 1.75e-7 -> 1.36e-7 (1.54e-7, 5.0e-7), 300 x 1024 x 256
+  // 1.23e-7 -> 1.10e-7 (1.48e-7, 2.9e-7); 12.7 -> 13.2 us at 576 x 1024 x 1024
+  auto mm = [&](const floatx4 (&x)[2][TI][2], const u32x4 (&b)[TJ][2][NB], bool scaled) {
+    V8 av[2][TI][NA];
 #pragma unroll
-    for (int i = 0; i < TI; ++i) {
-      if constexpr (S::F16)
-        split8_f16<NA>(x[i][0], x[i][1], scaled ? rs.er[i] : 0, av[i]);
-      else
-        split8<NA>(x[i][0], x[i][1], av[i]);
-    }
+    for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-    for (int q = 0; q < S::NP; ++q)
+      for (int i = 0; i < TI; ++i) {
+        if constexpr (S::F16)
+          split8_f16<NA>(x[ks][i][0], x[ks][i][1], scaled ? rs.er[i] : 0, av[ks][i]);
+        else
+          split8<NA>(x[ks][i][0], x[ks][i][1], av[ks][i]);
+      }
+    auto prod = [&](int i, int j, int ks, int q, const floatx16& c) {
+      return mfma32(av[ks][i][S::pa[q]], __builtin_bit_cast(V8, b[j][ks][S::pb[q]]), c);
+    };
 #pragma unroll
-      for (int i = 0; i < TI; ++i)
+    for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int j = 0; j < TJ; ++j)
-          acc[i][j] = mfma32(av[i][S::pa[q]], __builtin_bit_cast(V8, b[j][ks][S::pb[q]]),
-                             acc[i][j]);
+      for (int j = 0; j < TJ; ++j) {
+        floatx16 lo;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) lo[r] = 0.f;
+#pragma unroll
+        for (int q = 0; q + 1 < S::NP; ++q)
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks) lo = prod(i, j, ks, q, lo);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) acc[i][j] = prod(i, j, ks, S::NP - 1, acc[i][j]);
+        if constexpr (S::NP > 1) acc[i][j] += lo;
+      }
   };
   // (the LDS area passes values between lanes of the wavefront, whose LDS operations run in program
   // order: the wave barriers only keep the compiler from moving them across each other)
@@ -120,13 +138,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void gemm_small_kernel(Ge
         x[ks][i][1] = __builtin_bit_cast(floatx4, As[row * 8 + ((c0 + 1) ^ aswz(row))]);
       }
     rs.check(x[0], x[1], acc, lh);
-    if (!S::F16 || rs.unscaled) {
-      mm(x[0], b, 0, false);
-      mm(x[1], b, 1, false);
-    } else {
-      mm(x[0], b, 0, true);
-      mm(x[1], b, 1, true);
-    }
+    if (!S::F16 || rs.unscaled)
+      mm(x, b, false);
+    else
+      mm(x, b, true);
   };
 #pragma unroll
   for (int d = 0; d < DEPTH; ++d)
@@ -204,7 +219,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void gemm_small_kernel(Ge
 
 // Which products run here, and on how many wavefronts, is a rule on the product's own rows and
 // columns (small_waves), so that its k sums, and its bits, do not depend on what else is in its
-// launch: eight wavefronts share K up to 256 rows, four above.  The tile is the launch's (every
+// launch: eight wavefronts share K up to 256 rows and past 1024 columns (shares of 256
+// columns at most, up to K = 2048), four otherwise.  The tile is the launch's (every
 // tile adds an element's products in one order): a compute unit holds one workgroup of eight
 // wavefronts or two of four, and the tile is the smallest one (the shortest chain of k steps)
 // whose workgroups are still one round, or 64 x 64.  Measured per
@@ -265,7 +281,7 @@ namespace tta_gemm {
 
 int small_waves(const GemmArgs& p) {
   if (p.M >= 4096 || (int64_t)tta_blocks(p.M, 64) * tta_blocks(p.N, 64) > 512) return 0;
-  return p.M <= 256 ? 8 : 4;
+  return p.M <= 256 || p.K > 1024 ? 8 : 4;
 }
 
 int launch_small(GemmGroup& g, int n, int waves, int mode, hipStream_t s) {
