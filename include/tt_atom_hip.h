@@ -59,8 +59,8 @@ int tta_gemm_f32(const float* A, const float* B, float* C, const float* bias, fl
  * accuracy over fp32's whole range, at half the matrix work of mode 6; mode 6: 3 x 3 bf16 planes,
  * products a0b0 + a0b1 + a1b0 + a0b2 + a2b0 + a1b1 -- fp32 GEMM accuracy; mode 3: 2 x 2 bf16
  * planes, 3 products (~2^-16 relative); mode 1: bf16 operands.  A needs K, lda multiples of 4,
- * lda < 2^21 and 16-byte alignment.  The order of a product's k sums is a rule on its own M and N,
- * from 4096 rows on on neither: there a column's result does not depend on the other columns (the
+ * lda < 2^21 and 16-byte alignment.  The order of a product's k sums is a rule on its own M, N and K,
+ * from 4096 rows on on none of them: there a column's result does not depend on the other columns (the
  * short-K kernel of mode 16, K <= 128, aside, which takes a row's power of two over the whole row).
  * Replaces the same ttnn.linear / ttnn.matmul call sites as tta_gemm_f32 (the reference runs
  * them in bf16 / bf8 with fp32 accumulation: compute_kernel_config, device.py). */

@@ -217,20 +217,20 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void gemm_small_kernel(Ge
   }
 }
 
-// Which products run here, and on how many wavefronts, is a rule on the product's own rows and
-// columns (small_waves), so that its k sums, and its bits, do not depend on what else is in its
-// launch: eight wavefronts share K up to 256 rows and past 1024 columns (shares of 256
-// columns at most, up to K = 2048), four otherwise.  The tile is the launch's (every
-// tile adds an element's products in one order): a compute unit holds one workgroup of eight
-// wavefronts or two of four, and the tile is the smallest one (the shortest chain of k steps)
-// whose workgroups are still one round, or 64 x 64.  Measured per
-// launch (us; the split-K launch pair or fp32 kernel that ran before, then 32 x 32 / 32 x 64 /
-// 64 x 64 tiles, then the tiled kernel): eight wavefronts, 72 x 1024 x 1024: 11.7; 7.3, 8.0, 11.1;
-// 26.6.  Four: 433 x 1024 x 1024: 20.2; 11.0, 10.3, 13.6; 28.1 (eight: 14.4, 9.1, 12.0).
-// 576 x 1024 x 1024: 24.0; 16.3, 12.2, 13.9; 28.2.  1937 x 1024 x 1024: 77.6; 47.3, 29.4, 22.8;
-// 30.2.  2500 x 1024 x 1024 (640 tiles of 64 x 64): 89.8; 56.5, 39.2, 34.2; 31.1.  4000 x 1024 x
-// 1024: 64 x 64 tiles 47, tiled 34; 4000 x 4096 x 1024: 175, 117.  From 4096 rows on callers split a
-// convolution's columns over launches and expect the same bits: no small tile.
+// Which products run here, and on how many wavefronts, is a rule on the product's own rows, columns
+// and K (small_waves), so that its k sums, and its bits, do not depend on what else is in its
+// launch: eight wavefronts share K up to 256 rows and past 1024 columns of K (shares of 256 at most
+// up to K = 2048), four otherwise.  The tile is the launch's (every tile adds an element's products
+// in one order): a compute unit holds one workgroup of eight wavefronts or two of four, and the
+// tile is the smallest one (the shortest chain of k steps) whose workgroups are still one round, or
+// 64 x 64.  Measured per launch with one chain of additions per accumulator, 3 to 4 % faster than now
+// (us; the split-K launch pair or fp32 kernel that ran before, then 32 x 32 / 32 x 64 / 64 x 64
+// tiles, then the tiled kernel): eight wavefronts, 72 x 1024 x 1024: 11.7; 7.3, 8.0, 11.1; 26.6.
+// Four: 433 x 1024 x 1024: 20.2; 11.0, 10.3, 13.6; 28.1 (eight: 14.4, 9.1, 12.0).  576 x 1024 x
+// 1024: 24.0; 16.3, 12.2, 13.9; 28.2.  1937 x 1024 x 1024: 77.6; 47.3, 29.4, 22.8; 30.2.  2500 x
+// 1024 x 1024 (640 tiles of 64 x 64): 89.8; 56.5, 39.2, 34.2; 31.1.  4000 x 1024 x 1024: 64 x 64
+// tiles 47, tiled 34; 4000 x 4096 x 1024: 175, 117.  From 4096 rows on callers split a convolution's
+// columns over launches and expect the same bits: no small tile.
 enum SmallTile { k32x32, k32x64, k64x64 };
 
 SmallTile small_tile(const GemmGroup& g, int n, int waves) {

@@ -318,7 +318,11 @@ namespace tta_gemm {
 // Whether a launch takes the wide tile: mode 16 or 1, whole 32-wide k slabs, at least one whole
 // column tile per product.  Mode 16 also needs 3072 k columns of tiles per resident workgroup: from
 // there on the uneven last round of the larger tiles costs at most 1 %, below it decides by how
-// that round happens to fill.  Measured, 128 x 128 -> 128 x 256 (us; M x N x K, k columns): 196,555
+// that round happens to fill.  And where a product's last column tile is at most half full, an
+// average K of at least 512 (the half tile's prologue and epilogue are not halved): conv-2 group
+// (384 x 384, 512 x 512, 256 x 256) of 110,000 / 150,000 / 204,800 rows 476 -> 484 / 549 -> 561 / 745
+// -> 748 us, its 384 columns alone 238 -> 261 at 204,800 rows; 640 columns at K = 768 683 -> 650.
+// Measured, 128 x 128 -> 128 x 256 (us; M x N x K, k columns): 196,555
 // x 1024 x 1024 (12,288) with the two-output epilogue 1460 -> 1350, with the SiLU-gradient one 1432
 // -> 1337; 61,440 rows, conv-1 group (4560) 461 -> 438, its adjoint (4200) 484 -> 470; 90,000 x 640
 // x 768 (3168) 285 -> 286; 50,000 x 1024 x 1024 (3128) 362 -> 341; 196,555 x 1024 x 256 (3072) 559 ->
@@ -339,6 +343,7 @@ namespace tta_gemm {
 bool wide_ok(const GemmGroup& g, int n, int mode, int cap) {
   if (mode != 16 && mode != 1) return false;
   int64_t cols = 0, wide = 0, tiles = 0;
+  bool half = false;
   for (int i = 0; i < n; ++i) {
     const GemmArgs& p = g.p[i];
     if (p.K % BK != 0 || p.K < 2 * BK || p.N < WN) return false;
@@ -346,8 +351,9 @@ bool wide_ok(const GemmGroup& g, int n, int mode, int cap) {
     wide += w;
     tiles += rows * tta_blocks(p.N, BN);
     cols += w * p.K;
+    half = half || (p.N % WN > 0 && p.N % WN <= BN);
   }
-  if (mode == 16) return cols >= (int64_t)3072 * cap;
+  if (mode == 16) return cols >= (int64_t)3072 * cap && (!half || cols >= 512 * wide);
   const auto rounds = [&](int64_t c) { return (c + cap - 1) / cap; };
   return cols >= 384 * wide && 5 * rounds(tiles) >= 8 * rounds(wide);
 }
